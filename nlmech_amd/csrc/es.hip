@@ -821,24 +821,6 @@ size_t es_lds_bytes(const FdState& s) {
   return size_t(s.halo_max + 1) * es_record_bytes(s.precision);
 }
 
-// Raises a kernel's dynamic-LDS limit to what the launch needs.  The grant
-// is kept per kernel (keyed by its address: every template instance has its
-// own attribute) and per device.
-void allow_lds(const void* kernel, size_t bytes) {
-  static std::mutex mu;
-  static std::map<std::pair<int, const void*>, size_t> granted;
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  std::lock_guard<std::mutex> lock(mu);
-  size_t& g = granted[{dev, kernel}];
-  if (bytes > g) {
-    (void)hipFuncSetAttribute(kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              int(bytes));
-    g = bytes;
-  }
-}
-
 template <int DIM, int MODE>
 void launch_dil(nlm_ctx* c, const EsArgs<DIM>& e) {
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
@@ -925,6 +907,24 @@ void launch_any(nlm_ctx* c, int kind, bool base_f, double tf, double tn,
 }
 
 }  // namespace
+
+// Raises a kernel's dynamic-LDS limit to what the launch needs.  The grant
+// is kept per kernel (keyed by its address: every template instance has its
+// own attribute) and per device.
+void allow_lds(const void* kernel, size_t bytes) {
+  static std::mutex mu;
+  static std::map<std::pair<int, const void*>, size_t> granted;
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> lock(mu);
+  size_t& g = granted[{dev, kernel}];
+  if (bytes > g) {
+    (void)hipFuncSetAttribute(kernel,
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              int(bytes));
+    g = bytes;
+  }
+}
 
 // Device arrays and the weighted volume; called by nlm_fd_setup after the
 // node arrays and slices are in place.

@@ -32,6 +32,7 @@
 #include "bond_rnp.h"
 #include "device_common.h"
 #include "fd_common.h"
+#include "fd_staged.h"
 #include "layout.h"
 #include "nlm_internal.h"
 
@@ -106,17 +107,6 @@ __device__ __forceinline__ void bond_mode(const RnpDev& m, const double* xi,
     bond_fp32<DIM, INF>(m, xi, ui, xj, uj, voli, volj, brk, fs, F);
 }
 
-// One halo node staged in LDS by the tiled step kernel (2D): reference
-// position, displacement, volume and flags in one 48-byte record, so a
-// neighbor costs one address computation and three LDS reads.
-struct alignas(16) HaloRec {
-  double2 x;
-  double2 u;
-  double vol;
-  uint32_t flags;
-  float cv;  // FP32-force mode: vol * c4 (* J when constant), in FP32
-};
-
 // The FP32-force mode's record (40 bytes: a 10-dword stride puts record
 // starts on 32 of the 64 LDS banks where an 8-dword stride reaches 8): the
 // displacement in FP64 and the position relative to the block's origin in
@@ -146,9 +136,9 @@ struct alignas(8) HaloRec32 {
 };
 static_assert(sizeof(HaloRec32) == 40, "FP32-force record");
 
-template <int MODE>
-using HaloRecOf =
-    typename std::conditional<MODE == kModeFp32, HaloRec32, HaloRec>::type;
+// LDS budget of the staged kernels: halos whose records of this size exceed
+// 64 KiB take the direct gathers.
+constexpr int64_t kHaloRecBudget = 48;
 
 template <int DIM, int MODE, int KIND, bool BASE_F, int INF, int U,
           bool NOFAIL, bool TILED>
@@ -168,10 +158,11 @@ __device__ __forceinline__ void fd_step_body(
   int64_t nblk = (a.nslices * 64 + bn - 1) / bn;
   int64_t lb = xcd_block(nblk);
   if (lb >= nblk) return;
-  static_assert(!TILED || DIM == 2, "the LDS-staged kernel is 2D");
-  constexpr bool REL = TILED && MODE == kModeFp32;  // block-relative FP32
-  typedef HaloRecOf<MODE> Rec;
-  extern __shared__ HaloRec smem_halo[];
+  static_assert(!TILED || (DIM == 2 && MODE == kModeFp32),
+                "the LDS-staged form is 2D, FP32-force (others: k_fd_st)");
+  constexpr bool REL = TILED;  // block-relative FP32 records
+  typedef HaloRec32 Rec;
+  extern __shared__ double smem_halo[];
   Rec* const halo_lds = reinterpret_cast<Rec*>(smem_halo);
   double2 org = make_double2(0., 0.);
   int64_t hb = 0;
@@ -205,13 +196,8 @@ __device__ __forceinline__ void fd_step_body(
         r.xr = make_float2(float((xg.x - org.x) * a.m.sigma),
                            float((xg.y - org.y) * a.m.sigma));
         r.u = make_double2(ug.x * a.m.tau, ug.y * a.m.tau);
-      } else {
-        r.cv = float(vg) * a.m.c4f_infl;
-        r.x = xg;
-        r.u = ug;
-        r.vol = vg;
       }
-      halo_lds[REL ? t + 1 : t] = r;
+      halo_lds[t + 1] = r;
     }
     __syncthreads();
   }
@@ -320,18 +306,6 @@ __device__ __forceinline__ void fd_step_body(
         duj[q][1] = float(r->u.y - uis[1]);
         cvj[q] = r->cv;
         if (NOFAIL) flj[q] = r->flags;
-      } else if constexpr (TILED) {
-        typedef const __attribute__((address_space(3))) HaloRec LdsRec;
-        LdsRec* r = (LdsRec*)j;
-        xj[q][0] = r->x.x;
-        xj[q][1] = r->x.y;
-        xj[q][2] = 0.;
-        uj[q][0] = r->u.x;
-        uj[q][1] = r->u.y;
-        uj[q][2] = 0.;
-        vj[q] = r->vol;
-        cvj[q] = r->cv;
-        if (NOFAIL) flj[q] = r->flags;
       } else {
         load3<DIM>(ld32(a.x, j), xj[q]);
         load3<DIM>(ld32(a.u, j), uj[q]);
@@ -438,19 +412,6 @@ __device__ __forceinline__ void fd_step_body(
               load3<DIM>(ld32(a.x, g), xs);
               load3<DIM>(ld32(a.u, g), us);
               vs = ld32(a.vol, g);
-            } else if constexpr (TILED) {
-              // the neighbor's record is re-read from LDS (volatile, so the
-              // common path need not keep its FP64 values alive)
-              typedef volatile const __attribute__((address_space(3))) HaloRec
-                  LdsRecV;
-              LdsRecV* r = (LdsRecV*)jc[q];
-              xs[0] = r->x.x;
-              xs[1] = r->x.y;
-              xs[2] = 0.;
-              us[0] = r->u.x;
-              us[1] = r->u.y;
-              us[2] = 0.;
-              vs = r->vol;
             } else {
               // re-read from global memory (volatile, so the common path
               // need not keep the FP64 values alive)
@@ -958,15 +919,14 @@ template <int DIM, int MODE, int KIND, bool BASE_F, int INF, int U,
 void launch_t(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
   const unsigned long long* bits_ro = a.bits;
-  if constexpr (DIM == 2) {
+  if constexpr (DIM == 2 && MODE == kModeFp32) {
     if (c->fd.tiled && c->fd.use_tiled) {
-      // one workgroup per tile of the layout's halos
+      // one workgroup per tile of the layout's halos; the records follow a
+      // zero-weight record 0
       const int bn = c->fd.tile;
       const unsigned gt = grid_xcd(c->fd.sell.nslices * 64, bn);
-      // (the FP32-force records follow a zero-weight record 0)
-      size_t lds = size_t(a.halo_cap + (MODE == kModeFp32 ? 1 : 0)) *
-                   sizeof(HaloRecOf<MODE>);
-      if constexpr (MODE == kModeFp32 && U == 2) {
+      const size_t lds = size_t(a.halo_cap + 1) * sizeof(HaloRec32);
+      if constexpr (U == 2) {
         hipLaunchKernelGGL((k_fd_w6<DIM, MODE, KIND, BASE_F, INF, U, NOFAIL>),
                            dim3(gt), dim3(bn), lds, c->stream, a, bits_ro,
                            a.vexw, tf, tn);
@@ -1019,6 +979,16 @@ void launch_inf(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
 template <int DIM, int KIND, bool BASE_F>
 void launch_mode(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
                  int U) {
+  if constexpr (DIM == 2) {
+    // the FP64 modes' staged kernel
+    if (c->fd.tiled && c->fd.use_tiled && c->fd.precision != kModeFp32) {
+      FdArgs<2> b = a;
+      b.kind = KIND == KIND_CD ? KIND_CD : BASE_F ? KIND_FORCE_ADD : KIND_FORCE;
+      b.halo_bytes = (c->fd.halo_max + 1) *
+                     int64_t(st_rec_bytes(2, c->fd.has_nofail));
+      return st_launch2(c, b, tf, tn, U);
+    }
+  }
   switch (c->fd.precision) {
     case kModeExact:
       launch_inf<DIM, kModeExact, KIND, BASE_F>(c, a, tf, tn, U);
@@ -1224,21 +1194,16 @@ using namespace nlm;
 
 namespace {
 
-// LDS byte offsets of the staged step kernel's slot entries (halo-local
-// record index times the record size).  In the FP32-force mode the records
-// start at index 1: record 0 is a zero-weight record far from every node,
-// addressed by the padded slots (past a row's length) and by the fetches
-// past a slice, so the common path needs no per-slot row-length test.
+// LDS byte offsets of the staged step kernels' slot entries (record index
+// times the record size).  The records start at index 1: record 0 is a
+// zero-weight record far from every node, addressed by the padded slots
+// (past a row's length) and by the fetches past a slice, so the common path
+// needs no per-slot row-length test.
 std::vector<uint16_t> staged_entries(const std::vector<uint16_t>& colL,
-                                     int precision, const int64_t* sl_ptr,
+                                     size_t rec, const int64_t* sl_ptr,
                                      int64_t nslices, const uint16_t* rowlen,
                                      int64_t n) {
   std::vector<uint16_t> out(colL.size(), 0);
-  if (precision != NLM_PREC_FP32_FORCE) {
-    for (size_t e = 0; e < colL.size(); e++)
-      out[e] = uint16_t(uint32_t(colL[e]) * uint32_t(sizeof(HaloRec)));
-    return out;
-  }
   for (int64_t sl = 0; sl < nslices; sl++) {
     const int64_t e0 = sl_ptr[sl];
     const int64_t width = (sl_ptr[sl + 1] - e0) / 64;
@@ -1246,11 +1211,17 @@ std::vector<uint16_t> staged_entries(const std::vector<uint16_t>& colL,
       for (int lane = 0; lane < 64; lane++) {
         const int64_t e = e0 + 64 * k + lane, a = sl * 64 + lane;
         if (a < n && k < int64_t(rowlen[a]))
-          out[size_t(e)] = uint16_t((uint32_t(colL[size_t(e)]) + 1u) *
-                                    uint32_t(sizeof(HaloRec32)));
+          out[size_t(e)] =
+              uint16_t((uint32_t(colL[size_t(e)]) + 1u) * uint32_t(rec));
       }
   }
   return out;
+}
+
+// Bytes of a halo record of the 2D staged kernels.
+size_t halo_rec_bytes(int precision, bool nofail) {
+  return precision == NLM_PREC_FP32_FORCE ? sizeof(HaloRec32)
+                                          : st_rec_bytes(2, nofail);
 }
 
 }  // namespace
@@ -1369,28 +1340,35 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   if ((rc = up(s.halo, L.halo.data(), sizeof(int32_t) * L.halo.size()))) return rc;
   s.halo_max = L.halo_max;
   s.tile = 256;
-  // LDS budget of the staged kernel: one 48-byte record per halo node
+  // the staged kernels: 2D, when a block's halo fits the LDS budget
+  bool has_nofail = false;
+  if (p->interior)
+    for (int64_t i = 0; i < n; i++) has_nofail = has_nofail || !p->interior[i];
   s.tiled = !es_mat && dim == 2 && L.halo_max > 0 &&
-            (L.halo_max + 1) * int64_t(sizeof(HaloRec)) <= 64 * 1024;
+            (L.halo_max + 1) * kHaloRecBudget <= 64 * 1024;
+  // the FP64 modes' arithmetic (bond_fast64.h) takes beta > 0 and lengths
+  // far inside the exponent range
+  if (s.tiled && p->precision != NLM_PREC_FP32_FORCE)
+    s.tiled = p->mat.beta > 0. && std::isfinite(p->mat.beta) &&
+              p->mat.horizon > kStagedLenMin &&
+              p->mat.horizon < kStagedLenMax && p->mat.h > kStagedLenMin;
   if (s.tiled) {
-    // the staged kernel addresses its dynamic LDS from 0, which holds while
-    // it has no static LDS (one instance checked: all share the source)
+    // the staged kernels address their dynamic LDS from 0, which holds while
+    // they have no static LDS (one instance checked: all share the source)
     hipFuncAttributes fa;
     if (hipFuncGetAttributes(
             &fa, reinterpret_cast<const void*>(
                      &k_fd_w6<2, kModeFp32, KIND_CD, false, 0, 2, false>)) !=
             hipSuccess ||
-        fa.sharedSizeBytes != 0)
+        fa.sharedSizeBytes != 0 || !st_lds_base_zero())
       s.tiled = false;
   }
-  // the bond-based staged kernel reads halo-local entries as LDS byte
-  // offsets of its records (below 64 KiB by the budget above; the FP32-force
-  // mode's records are the 40-byte block-relative ones after a zero-weight
-  // record 0)
+  // the bond-based staged kernels read halo-local entries as LDS byte
+  // offsets of their records (below 64 KiB by the budget above)
   if (s.tiled) {
-    const std::vector<uint16_t> colL_off =
-        staged_entries(L.colL, p->precision, L.sl_ptr.data(), L.nslices,
-                       L.rowlen.data(), n);
+    const std::vector<uint16_t> colL_off = staged_entries(
+        L.colL, halo_rec_bytes(p->precision, has_nofail), L.sl_ptr.data(),
+        L.nslices, L.rowlen.data(), n);
     if ((rc = up(s.colL, colL_off.data(), sizeof(uint16_t) * nent))) return rc;
   } else if ((rc = up(s.colL, L.colL.data(), sizeof(uint16_t) * nent))) {
     return rc;
@@ -1548,6 +1526,11 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
                                         double(m.break_guard_f))
                                 : std::numeric_limits<float>::infinity();
   m.up_rcp_h_f = float(m.check_up * m.rcp_h);
+  m.up_rcp_h = m.check_up * m.rcp_h;
+  m.c4_infl = m.inf_type == 0 ? m.c4 * m.inf_a : m.c4;
+  m.x_break_lo = m.irreversible
+                     ? m.beta * (m.break_lo * m.krbar_sq)
+                     : std::numeric_limits<double>::infinity();
   m.vex_tol_f = float(3e-5 * m.low_band);
   {
     const double b2 = m.beta * 1.4426950408889634;  // beta log2 e
@@ -2327,14 +2310,15 @@ int retile(nlm_ctx* c, int bn) {
   int64_t hmax = 0;
   build_halos(n, ns, slp.data(), colS.data(), bn / 64, hp, halo, colL, hmax);
   if (!es) {
-    if ((hmax + 1) * int64_t(sizeof(HaloRec)) > 64 * 1024)
+    if ((hmax + 1) * kHaloRecBudget > 64 * 1024)
       return fail(c, NLM_ERR_INVALID,
                   "tile of " + std::to_string(bn) +
                       " nodes: its largest halo exceeds the LDS budget");
     std::vector<uint16_t> rl(static_cast<size_t>(n));
     NLM_HIP(c, hipMemcpy(rl.data(), s.sell.rowlen.p, sizeof(uint16_t) * n,
                          hipMemcpyDeviceToHost));
-    colL = staged_entries(colL, s.precision, slp.data(), ns, rl.data(), n);
+    colL = staged_entries(colL, halo_rec_bytes(s.precision, s.has_nofail),
+                          slp.data(), ns, rl.data(), n);
   } else {
     int lds_max = 0;
     NLM_HIP(c, hipDeviceGetAttribute(&lds_max,

@@ -43,6 +43,9 @@ struct FdArgs {
   int has_nofail;
   const double* __restrict__ node_rate;  // node-list BC rates (or null)
   const double* __restrict__ tdev;       // step times from device memory
+  int kind;            // KIND_* of the launch (k_fd_st)
+  int tile;            // nodes of a workgroup's tile
+  int64_t halo_bytes;  // LDS bytes of the halo records (k_fd_st)
 };
 
 // Displacement and velocity of a prescribed dof at time t: ULoading::apply
@@ -101,7 +104,7 @@ __device__ __forceinline__ void fext_node(const BcTable* bc, uint32_t fl,
 // KIND_CD: fused force at t_force + central-difference update + BCs at t_next.
 constexpr int KIND_FORCE = 0;
 constexpr int KIND_CD = 1;
-constexpr int KIND_VERLET = 2;
+constexpr int KIND_FORCE_ADD = 2;  // f += internal force
 
 // Fourth dword of a raw buffer resource on gfx9 targets (32-bit untyped
 // accesses, range-checked against the record count).
@@ -187,12 +190,18 @@ inline FdArgs<DIM> make_args(nlm_ctx* c) {
   a.has_nofail = s.has_nofail ? 1 : 0;
   a.node_rate = s.node_rate.as<double>();
   a.tdev = nullptr;
+  a.kind = KIND_CD;
+  a.tile = s.tile;
+  a.halo_bytes = 0;
   return a;
 }
 
 inline int64_t force_blocks(const FdState& s) {
   return (s.sell.nslices * 64 + 255) / 256;
 }
+
+// Raises a kernel's dynamic-LDS limit to what the launch needs (es.hip).
+void allow_lds(const void* kernel, size_t bytes);
 
 // Force of the configured material at the current u (fd.hip).
 void fd_launch_force(nlm_ctx* c, bool base_f, double t);

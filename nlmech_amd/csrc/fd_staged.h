@@ -1,0 +1,320 @@
+// fd_staged.h -- the LDS-staged bond-based step kernel of the FP64 modes
+// (k_fd_st).
+//
+// A workgroup owns a tile of the layout's internal order (128, 256 or 512
+// nodes): it stages the tile's halo -- every node its rows reference -- in
+// LDS once (one record a node) and reads neighbors through 16-bit LDS byte
+// offsets.  Record 0 is a zero-volume record far from every node; padded
+// slots and fetches past a slice address it and come out as exact zeros, so
+// the common path carries no row-length mask.  The kernel is bound by FP64
+// instructions; bond_fast64.h says what a bond costs.  Per step, before and
+// after that arithmetic (and the records without the row-length mask):
+// 400 x 397 nodes, horizon 4 h, exact mode 57 -> 28 us; 619 x 451 nodes,
+// FP64 mode, four slots a chunk 48 -> 31 us.
+//
+// Launch kinds (a.kind, wavefront-uniform): force, force added to f, the
+// fused central-difference step.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "bond_fast64.h"
+#include "bond_rnp.h"
+#include "device_common.h"
+#include "fd_common.h"
+#include "nlm_internal.h"
+
+namespace nlm {
+
+// Halo record of the FP64 modes: position, displacement and the volume (FP64
+// mode: times c4, and J when constant).  10- and 14-dword strides spread
+// record starts over 32 of the 64 LDS banks.
+template <int DIM, bool NOFAIL>
+struct alignas(8) StRec64 {
+  double x[DIM];
+  double u[DIM];
+  double c;
+};
+template <int DIM>
+struct alignas(8) StRec64<DIM, true> {
+  double x[DIM];
+  double u[DIM];
+  double c;
+  uint32_t flags, pad;
+};
+
+template <int DIM, int MODE, bool NOFAIL>
+using StRec = StRec64<DIM, NOFAIL>;
+
+// The end of a launch for node i with force density f = base + sum.
+template <int DIM>
+__device__ __forceinline__ void st_tail(const FdArgs<DIM>& a, int64_t i,
+                                        uint32_t fl, const double* xi,
+                                        const double* ui, double* acc,
+                                        double t_force, double t_next) {
+  double f[3] = {0., 0., 0.};
+  if (a.kind == KIND_FORCE_ADD) {
+    load3<DIM>(a.f_in[i], f);
+  } else if (a.has_fbc) {
+    fext_node<DIM>(a.bc, fl, xi, t_force, f);
+  }
+  for (int d = 0; d < DIM; d++) f[d] += acc[d];
+  if (a.kind == KIND_FORCE || a.kind == KIND_FORCE_ADD) {
+    a.f_out[i] = make_v<DIM>(f);
+    return;
+  }
+  double vi[3];
+  load3<DIM>(a.v[i], vi);
+  double un[3] = {0., 0., 0.}, vn[3] = {0., 0., 0.};
+  for (int d = 0; d < DIM; d++) {
+    const uint32_t id = (fl >> (kFlagUbcShift + 4 * d)) & 0xfu;
+    if (id == 0) {
+      const double uo = ui[d];
+      // u += fact*f + dt*v; v = (u - u_old)/dt  (fDModel.cpp:386-394)
+      un[d] = uo + (a.fact * f[d] + a.dt * vi[d]);
+      vn[d] = (un[d] - uo) / a.dt;
+    } else {
+      double du, dv;
+      ubc_dof(a, id, i, d, xi, t_next, du, dv);
+      un[d] = du;
+      vn[d] = dv;
+    }
+  }
+  a.u_out[i] = make_v<DIM>(un);
+  a.v_out[i] = make_v<DIM>(vn);
+}
+
+// Exact evaluation of a deferred bond from the neighbor's global arrays.
+template <int DIM, int MODE, int INF>
+__device__ __forceinline__ void st_deferred(const FdArgs<DIM>& a, uint32_t g,
+                                            const double* xi,
+                                            const double* ui, double voli,
+                                            bool brk, bool& fs, double* F) {
+  double xs[3], us[3];
+  load3<DIM>(ld32(a.x, g), xs);
+  load3<DIM>(ld32(a.u, g), us);
+  const double vs = ld32(a.vol, g);
+  if constexpr (MODE == kModeExact)
+    bond_exact<DIM, false>(a.m, xi, ui, xs, us, voli, vs, brk, fs, F, nullptr);
+  else
+    bond_fp64<DIM, INF>(a.m, xi, ui, xs, us, voli, vs, brk, fs, F);
+}
+
+template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT>
+__global__ __launch_bounds__(512) void k_fd_st(
+    FdArgs<DIM> a, const unsigned long long* __restrict__ bits_ro,
+    const unsigned long long* __restrict__ vex_ro, double t_force,
+    double t_next) {
+  if (a.tdev) {  // graph-captured steps read the step's times
+    t_force = a.tdev[0];
+    t_next = a.tdev[1];
+  }
+  constexpr bool EXACT = MODE == kModeExact;
+  typedef StRec<DIM, MODE, NOFAIL> Rec;
+  const int bn = int(blockDim.x);
+  const int nsl = bn >> 6;  // slices of the tile
+  const int64_t nblk = (a.nslices * 64 + bn - 1) / bn;
+  const int64_t lb = xcd_block(nblk);
+  if (lb >= nblk) return;
+  extern __shared__ double st_smem[];
+  Rec* const halo_lds = reinterpret_cast<Rec*>(st_smem);
+  const int64_t hb = a.halo_ptr[lb];
+  const int hn = int(a.halo_ptr[lb + 1] - hb);
+  for (int t = int(threadIdx.x) - 1; t < hn; t += int(blockDim.x)) {
+    Rec r;
+    if (t < 0) {  // record 0
+      for (int d = 0; d < DIM; d++) r.u[d] = 0.;
+      r.c = 0;
+      for (int d = 0; d < DIM; d++) r.x[d] = 1e15;
+      if constexpr (NOFAIL) r.flags = 0u;
+      halo_lds[0] = r;
+      continue;
+    }
+    const uint32_t g = uint32_t(a.halo[hb + t]);
+    double xg[3], ug[3];
+    load3<DIM>(ld32(a.x, g), xg);
+    load3<DIM>(ld32(a.u, g), ug);
+    const double vg = ld32(a.vol, g);
+    for (int d = 0; d < DIM; d++) {
+      r.x[d] = xg[d];
+      r.u[d] = ug[d];
+    }
+    r.c = EXACT ? vg : vg * a.m.c4_infl;
+    if constexpr (NOFAIL) r.flags = ld32(a.flags, g);
+    halo_lds[t + 1] = r;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t s = lb * nsl + wave;
+  if (s >= a.nslices) return;  // whole wavefront
+  const int64_t i = s * 64 + lane;
+  const bool valid = i < a.n;
+  const int64_t cb = a.sl_ptr[s];
+  const int width = int((a.sl_ptr[s + 1] - cb) >> 6);
+  const int64_t bb = cb >> 6;
+  const int len = valid ? int(a.rowlen[i]) : 0;
+  double xi[3] = {0., 0., 0.}, ui[3] = {0., 0., 0.};
+  double voli = 1.;
+  uint32_t fl = 0;
+  if (valid) {
+    load3<DIM>(a.x[i], xi);
+    load3<DIM>(a.u[i], ui);
+    voli = a.vol[i];
+    fl = a.flags[i];
+  }
+  const bool int_i = !(fl & kFlagNonInterior);
+  const unsigned long long* __restrict__ bits_in = bits_ro + bb;
+  const unsigned long long* __restrict__ vex_in = vex_ro + bb;
+  // slot entries through a buffer resource over the slice (fetches past it
+  // return 0: record 0)
+  const __amdgpu_buffer_rsrc_t col_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.colL + cb), 0, width * 64 * int(sizeof(uint16_t)),
+      kBufferRsrcWord3);
+  auto slot_entry = [&](int k) -> uint32_t {
+    return uint32_t(__builtin_amdgcn_raw_buffer_load_b16(
+        col_rsrc, lane * int(sizeof(uint16_t)), k * 64 * int(sizeof(uint16_t)),
+        0));
+  };
+  const unsigned long long int_m =
+      NOFAIL ? __builtin_amdgcn_ballot_w64(int_i) : ~0ull;
+  // one chunk of U slots from slot k0: the bonds' forces (exact mode: F[q])
+  // or the slot pairs' sums (fast modes: F[m])
+  constexpr int NF = EXACT ? U : U / 2;
+  uint32_t jn[U];
+  auto chunk = [&](int k0, double (&F)[NF][DIM]) {
+    uint32_t jc[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      jc[q] = jn[q];
+      jn[q] = slot_entry(k0 + U + q);
+    }
+    unsigned long long w[U], vx[U], brk[U], band[U], ex[U];
+    unsigned long long ex_any = 0ull;
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      w[q] = bits_in[k0 + q];
+      vx[q] = vex_in[k0 + q];
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      // the slot entry is the record's LDS address (the kernel has no
+      // static LDS, checked by the host)
+      typedef const __attribute__((address_space(3))) Rec LdsRec;
+      LdsRec* r = (LdsRec*)jc[q];
+      SlotMasks km;
+      km.act = ~0ull;
+      km.w = w[q];
+      km.vex = vx[q];
+      if constexpr (NOFAIL)
+        km.brk = int_m & __builtin_amdgcn_ballot_w64(
+                             (r->flags & kFlagNonInterior) == 0u);
+      else
+        km.brk = ~0ull;
+      brk[q] = km.brk;
+      double dx[DIM], du[DIM];
+      for (int d = 0; d < DIM; d++) {
+        dx[d] = r->x[d] - xi[d];
+        du[d] = r->u[d] - ui[d];
+      }
+      if constexpr (EXACT)
+        bond_exact_fast<DIM, INF, NOFAIL, SHORT>(a.m, dx, du, r->c, km,
+                                                 band[q], ex[q], F[q]);
+      else if (q % 2 == 1)
+        bond_fp64_staged<DIM, INF, NOFAIL, SHORT, true>(
+            a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
+      else
+        bond_fp64_staged<DIM, INF, NOFAIL, SHORT, false>(
+            a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
+      ex_any |= ex[q];
+    }
+    if (ex_any != 0ull) {  // rare: whole wavefronts skip it
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (ex[q] == 0ull) continue;
+        bool fsn = false;
+        if (__builtin_amdgcn_inverse_ballot_w64(ex[q]) && k0 + q < len) {
+          const uint32_t g = uint32_t(
+              a.halo[hb + jc[q] / uint32_t(sizeof(Rec)) - 1]);
+          const bool fs0 = __builtin_amdgcn_inverse_ballot_w64(w[q]);
+          bool fs = fs0;
+          double Fd[3];
+          st_deferred<DIM, MODE, INF>(
+              a, g, xi, ui, voli,
+              __builtin_amdgcn_inverse_ballot_w64(brk[q]), fs, Fd);
+          fsn = fs && !fs0;
+          for (int d = 0; d < DIM; d++) {
+            if constexpr (EXACT) F[q][d] = Fd[d];
+            else F[q / 2][d] += Fd[d];
+          }
+        }
+        // new broken bits: every lane stores the same word
+        const unsigned long long nb =
+            band[q] & __builtin_amdgcn_ballot_w64(fsn);
+        if (nb != 0ull && k0 + q < width) a.bits[bb + k0 + q] = w[q] | nb;
+      }
+    }
+  };
+  double acc[3] = {0., 0., 0.};
+#pragma unroll
+  for (int q = 0; q < U; ++q) jn[q] = slot_entry(q);
+  for (int k0 = 0; k0 < width; k0 += U) {
+    double F[NF][DIM];
+    chunk(k0, F);
+#pragma unroll
+    for (int m = 0; m < NF; ++m)
+      for (int d = 0; d < DIM; d++) acc[d] += F[m][d];
+  }
+  if (!valid) return;
+  st_tail<DIM>(a, i, fl, xi, ui, acc, t_force, t_next);
+}
+
+inline size_t st_rec_bytes(int dim, bool nofail) {
+  return size_t(2 * dim + 1) * 8 + (nofail ? 8 : 0);
+}
+
+// Launch of the staged kernel for the configured tile (fd_st2.hip).
+void st_launch2(nlm_ctx* c, const FdArgs<2>& a, double tf, double tn, int U);
+// Whether the kernels' static LDS size is 0, as their addressing needs.
+bool st_lds_base_zero();
+
+// Instances of one dimension and mode.
+template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT>
+void st_go(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
+  static_assert(sizeof(StRec<DIM, MODE, NOFAIL>) % 8 == 0, "record");
+  const unsigned g = grid_xcd(c->fd.sell.nslices * 64, a.tile);
+  const size_t lds = size_t(a.halo_bytes);
+  allow_lds(reinterpret_cast<const void*>(
+                &k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT>),
+            lds);
+  hipLaunchKernelGGL((k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT>),
+                     dim3(g), dim3(unsigned(a.tile)), lds,
+                     c->stream, a, a.bits, a.vexw, tf, tn);
+}
+
+template <int DIM, int MODE, int U, bool SHORT, bool NOFAIL>
+void st_inf(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
+  const int inf = c->fd.rnp.inf_type;
+  if (inf == 0)
+    st_go<DIM, MODE, 0, U, NOFAIL, SHORT>(c, a, tf, tn);
+  else if (inf == 1)
+    st_go<DIM, MODE, 1, U, NOFAIL, SHORT>(c, a, tf, tn);
+  else
+    st_go<DIM, MODE, 2, U, NOFAIL, SHORT>(c, a, tf, tn);
+}
+
+template <int DIM, int MODE, int U>
+void st_opt(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
+  // the exponent's range form is chosen where the break test bounds it
+  // (exp_short); models with no-fail regions keep the general form
+  if (a.has_nofail)
+    st_inf<DIM, MODE, U, false, true>(c, a, tf, tn);
+  else if (a.m.x_break_lo <= kExpShortMax)
+    st_inf<DIM, MODE, U, true, false>(c, a, tf, tn);
+  else
+    st_inf<DIM, MODE, U, false, false>(c, a, tf, tn);
+}
+
+}  // namespace nlm

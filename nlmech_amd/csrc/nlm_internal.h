@@ -109,6 +109,10 @@ struct RnpDev {
   float break_lo_s;        // break_lo_f times beta log2 e
   float low_dd_f;          // (sigma low_band)^2
   float vex_dd_tol_f;      // half-width of the edge band on (sigma r)^2
+  // FP64 staged kernel: c4 (times J when constant), check_up / h, and the
+  // lower bound of the break test's guard band on beta r S^2 (+inf when bonds
+  // never break)
+  double c4_infl, up_rcp_h, x_break_lo;
 };
 
 // ElasticState constants as used by the kernels.
