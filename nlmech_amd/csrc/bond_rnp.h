@@ -449,6 +449,11 @@ __device__ __forceinline__ void bond_fp32_scaled(
     num = __builtin_fmaf(dx2, dv2, num);
   }
   float rinv = __builtin_amdgcn_rsqf(dd);
+  // 3D: one Newton step (the force takes 1/|dx| to the third power, and on a
+  // lattice the estimate's rounding is the same for every bond of a length)
+  if (DIM == 3)
+    rinv = __builtin_fmaf(0.5f * rinv,
+                          __builtin_fmaf(-(dd * rinv), rinv, 1.f), rinv);
   float q = num * rinv;           // tau S r
   float Ss = q * rinv;            // tau S / sigma
   float b = q * Ss;               // beta log2(e) r S^2

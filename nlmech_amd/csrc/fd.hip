@@ -979,15 +979,16 @@ void launch_inf(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
 template <int DIM, int KIND, bool BASE_F>
 void launch_mode(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
                  int U) {
-  if constexpr (DIM == 2) {
-    // the FP64 modes' staged kernel
-    if (c->fd.tiled && c->fd.use_tiled && c->fd.precision != kModeFp32) {
-      FdArgs<2> b = a;
-      b.kind = KIND == KIND_CD ? KIND_CD : BASE_F ? KIND_FORCE_ADD : KIND_FORCE;
-      b.halo_bytes = (c->fd.halo_max + 1) *
-                     int64_t(st_rec_bytes(2, c->fd.has_nofail));
-      return st_launch2(c, b, tf, tn, U);
-    }
+  // the staged kernel of the FP64 modes and of 3D models
+  if (c->fd.tiled && c->fd.use_tiled &&
+      (DIM == 3 || c->fd.precision != kModeFp32 || c->fd.parts > 1)) {
+    FdArgs<DIM> b = a;
+    b.kind = KIND == KIND_CD ? KIND_CD : BASE_F ? KIND_FORCE_ADD : KIND_FORCE;
+    b.halo_bytes =
+        (c->fd.halo_max + 1) *
+        int64_t(st_rec_bytes(DIM, c->fd.precision, c->fd.has_nofail));
+    if constexpr (DIM == 2) return st_launch2(c, b, tf, tn, U);
+    else return st_launch3(c, b, tf, tn, U);
   }
   switch (c->fd.precision) {
     case kModeExact:
@@ -1218,10 +1219,61 @@ std::vector<uint16_t> staged_entries(const std::vector<uint16_t>& colL,
   return out;
 }
 
-// Bytes of a halo record of the 2D staged kernels.
-size_t halo_rec_bytes(int precision, bool nofail) {
-  return precision == NLM_PREC_FP32_FORCE ? sizeof(HaloRec32)
-                                          : st_rec_bytes(2, nofail);
+// Bytes of a halo record of the bond-based staged kernels.
+size_t halo_rec_bytes(int dim, int precision, bool nofail) {
+  return dim == 2 && precision == NLM_PREC_FP32_FORCE
+             ? sizeof(HaloRec32)
+             : st_rec_bytes(dim, precision, nofail);
+}
+
+// Tile (nodes of a workgroup) and parts (wavefronts that share a slice's
+// rows) of the bond-based staged kernels, by the number of slices: few
+// slices take small tiles and split rows, so that every CU has wavefronts;
+// many slices take the tile with the fewest halo nodes a node.  Microseconds
+// per step at the lines (tile x parts):
+//   2D FP64 / exact, 100 x 100 nodes (157 slices): 64 x 8 6.9 / 7.4, 64 x 4
+//     7.3 / 7.8, 256 x 1 9.5 / 10.4; 200 x 190 (594): 64 x 4 11.8 / 14.0,
+//     256 x 1 13.1 / 15.4; 333 x 217 (1130), FP64: 64 x 4 13.0, 256 x 1 11.5;
+//   2D FP32-force, 157: 64 x 8 5.4, 256 x 1 7.8; 594: 64 x 4 7.2, 256 x 1
+//     10.4; 400 x 397 (2482): 128 x 2 13.5, 256 x 1 14.5; 619 x 451 (4362):
+//     128 x 2 23.1, 256 x 1 20.4;
+//   3D FP64 / exact, 20 x 18 x 22 (124): 64 x 8 11.6 / 14.0, 256 x 1 24 / 32;
+//     41 x 37 x 45 (1067): 64 x 8 33 / 42, 128 x 1 49 / 67; 72 x 64 x 56
+//     (4032): 64 x 4 83 / 107, 256 x 1 65 / 91, 128 x 1 97 / 138, 128 x 4
+//     83 / 107;
+//   3D FP32-force, 124: 64 x 8 8.4, 256 x 1 20.5; 1067: 128 x 2 20.0, 64 x 8
+//     22.6, 256 x 1 24.8; 4032: 256 x 2 43.7, 128 x 2 44.9, 256 x 1 51.5.
+// Direct gathers before (3D): 1067, FP64 61; 4032, FP32-force 95.
+struct StageRule {
+  int tile, parts;
+};
+StageRule stage_rule(int dim, int precision, int64_t nslices) {
+  const bool f32 = precision == NLM_PREC_FP32_FORCE;
+  if (nslices <= 256) return {64, 8};
+  if (nslices <= 800) return {64, 4};
+  if (dim == 2) {
+    if (f32 && nslices <= 3000) return {128, 2};
+    return {256, 1};
+  }
+  if (f32) return {nslices <= 2500 ? 128 : 256, 2};
+  if (nslices <= 2500) return {64, 8};
+  return {256, 1};
+}
+
+// Parts at a tile other than the rule's own (a tile set by hand, or one that
+// fits the LDS): at most 512 threads a workgroup; in the FP64 modes tiles of
+// 256 nodes and more keep whole rows (their rounds over four slices cost
+// more than the split gains: 157 slices, FP64 10.1 against 9.5 us).
+int stage_parts(int dim, int precision, int64_t nslices, int tile) {
+  const StageRule r = stage_rule(dim, precision, nslices);
+  if (tile == r.tile) return r.parts;
+  if (precision != NLM_PREC_FP32_FORCE) {
+    if (tile >= 256) return 1;
+    // (3D: 256-node tiles that do not fit fall to 128 x 4)
+    return std::max(r.parts == 1 && dim == 3 ? 4 : 1,
+                    std::min(r.parts, 512 / tile));
+  }
+  return std::max(1, std::min(r.parts, 512 / tile));
 }
 
 }  // namespace
@@ -1309,7 +1361,24 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   }
   // internal order, slices and halos (layout.cpp)
   HostLayout L;
-  build_layout(dim, n, p->x, mesh_h, h_row, h_col, L);
+  const bool bond3 = !es_mat && dim == 3;
+  bool has_nofail = false;
+  if (p->interior)
+    for (int64_t i = 0; i < n; i++) has_nofail = has_nofail || !p->interior[i];
+  const size_t rec = halo_rec_bytes(dim, p->precision, has_nofail);
+  StageRule rule{256, 1};
+  if (!es_mat) rule = stage_rule(dim, p->precision, (n + 63) / 64);
+  int tile = rule.tile;
+  build_layout(dim, n, p->x, mesh_h, h_row, h_col, tile / 64, L);
+  bool fits = (L.halo_max + 1) * int64_t(bond3 ? rec : kHaloRecBudget) <=
+              64 * 1024;
+  while (bond3 && !fits && tile > 64) {
+    tile /= 2;
+    L.nblocks = (L.nslices * 64 + tile - 1) / tile;
+    build_halos(n, L.nslices, L.sl_ptr.data(), L.colS.data(), tile / 64,
+                L.halo_ptr, L.halo, L.colL, L.halo_max);
+    fits = (L.halo_max + 1) * int64_t(rec) <= 64 * 1024;
+  }
   s.perm_host = L.perm;
   s.inv_host = L.inv;
   s.sell.nslices = L.nslices;
@@ -1339,16 +1408,13 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     return rc;
   if ((rc = up(s.halo, L.halo.data(), sizeof(int32_t) * L.halo.size()))) return rc;
   s.halo_max = L.halo_max;
-  s.tile = 256;
-  // the staged kernels: 2D, when a block's halo fits the LDS budget
-  bool has_nofail = false;
-  if (p->interior)
-    for (int64_t i = 0; i < n; i++) has_nofail = has_nofail || !p->interior[i];
-  s.tiled = !es_mat && dim == 2 && L.halo_max > 0 &&
-            (L.halo_max + 1) * kHaloRecBudget <= 64 * 1024;
-  // the FP64 modes' arithmetic (bond_fast64.h) takes beta > 0 and lengths
-  // far inside the exponent range
-  if (s.tiled && p->precision != NLM_PREC_FP32_FORCE)
+  s.tile = tile;
+  s.parts = es_mat ? 1 : stage_parts(dim, p->precision, L.nslices, tile);
+  // the staged bond-based kernels
+  s.tiled = !es_mat && L.halo_max > 0 && fits;
+  // k_fd_st's arithmetic takes beta > 0 and lengths far inside the exponent
+  // range
+  if (s.tiled && (dim == 3 || p->precision != NLM_PREC_FP32_FORCE))
     s.tiled = p->mat.beta > 0. && std::isfinite(p->mat.beta) &&
               p->mat.horizon > kStagedLenMin &&
               p->mat.horizon < kStagedLenMax && p->mat.h > kStagedLenMin;
@@ -1367,8 +1433,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   // offsets of their records (below 64 KiB by the budget above)
   if (s.tiled) {
     const std::vector<uint16_t> colL_off = staged_entries(
-        L.colL, halo_rec_bytes(p->precision, has_nofail), L.sl_ptr.data(),
-        L.nslices, L.rowlen.data(), n);
+        L.colL, rec, L.sl_ptr.data(), L.nslices, L.rowlen.data(), n);
     if ((rc = up(s.colL, colL_off.data(), sizeof(uint16_t) * nent))) return rc;
   } else if ((rc = up(s.colL, L.colL.data(), sizeof(uint16_t) * nent))) {
     return rc;
@@ -1382,12 +1447,12 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     for (int d = 0; d < dim; d++) hx[a * stride + d] = p->x[3 * i + d];
     hv[a] = p->vol[i];
   }
-  // Per 256-node block: the centre of its nodes' bounding box, the origin of
+  // Per tile: the centre of its nodes' bounding box, the origin of
   // the FP32 block-relative positions (double2 per block in 2D, double4 in
   // 3D).
   std::vector<double> borg(size_t(L.nblocks) * stride, 0.);
   for (int64_t b = 0; b < L.nblocks; b++) {
-    const int64_t a0 = 256 * b, a1 = std::min<int64_t>(n, a0 + 256);
+    const int64_t a0 = tile * b, a1 = std::min<int64_t>(n, a0 + tile);
     if (a0 >= n) break;
     double lo[3], hi[3];
     for (int d = 0; d < dim; d++) lo[d] = hi[d] = hx[a0 * stride + d];
@@ -1408,7 +1473,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
         org_range = std::max(
             org_range, std::fabs(hx[a * stride + d] - borg[stride * b + d]));
     };
-    for (int64_t a = 256 * b; a < std::min<int64_t>(n, 256 * b + 256); a++)
+    for (int64_t a = tile * b; a < std::min<int64_t>(n, tile * (b + 1)); a++)
       span(a);
     for (int64_t t = L.halo_ptr[b]; t < L.halo_ptr[b + 1]; t++)
       span(L.halo[size_t(t)]);
@@ -1535,12 +1600,28 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   {
     const double b2 = m.beta * 1.4426950408889634;  // beta log2 e
     if (b2 > 0.) {  // (beta > 0 for RNP bonds)
-      m.tau = std::ldexp(1.0, int(std::lround(0.5 * std::log2(b2))));
+      // 3D: 1/sigma is the quantum of the fixed-point positions, the
+      // smallest with every offset from a tile's origin (at most org_range)
+      // below 2^30 that keeps tau a power of two (between one and four times
+      // org_range / 2^30)
+      const double e = dim == 3
+                           ? std::floor(0.5 * std::log2(b2 * 0x1p+30 /
+                                                        std::max(org_range,
+                                                                 m.h)))
+                           : std::round(0.5 * std::log2(b2));
+      m.tau = std::ldexp(1.0, int(e));
       m.sigma = m.tau * m.tau / b2;
+      // 3D: sigma moved by up to 2^-25 so that 1/(sigma h), the constant of
+      // the volume correction, is an FP32 number (rounded, it is an error of
+      // every bond at the horizon's edge that does not average out: forces of
+      // the 72 x 64 x 56 block 4.4e-7 off instead of 2.6e-7); the exponent
+      // beta r S^2 takes that relative error instead
+      if (dim == 3) m.sigma = 1.0 / (double(float(1.0 / (m.sigma * m.h))) * m.h);
     } else {
       m.tau = m.sigma = 1.0;
     }
     const double bl = m.tau * m.tau / m.sigma;  // beta log2 e
+    m.c4_infl_s = m.c4_infl * m.sigma / m.tau;
     m.c4f_infl_s = float(double(m.c4f_infl) * m.sigma / m.tau);
     m.rcp_h_s = float(1.0 / (m.sigma * m.h));
     m.rcp_sigma_f = float(1.0 / m.sigma);
@@ -2317,7 +2398,8 @@ int retile(nlm_ctx* c, int bn) {
     std::vector<uint16_t> rl(static_cast<size_t>(n));
     NLM_HIP(c, hipMemcpy(rl.data(), s.sell.rowlen.p, sizeof(uint16_t) * n,
                          hipMemcpyDeviceToHost));
-    colL = staged_entries(colL, halo_rec_bytes(s.precision, s.has_nofail),
+    colL = staged_entries(colL,
+                          halo_rec_bytes(s.dim, s.precision, s.has_nofail),
                           slp.data(), ns, rl.data(), n);
   } else {
     int lds_max = 0;
@@ -2378,6 +2460,7 @@ int retile(nlm_ctx* c, int bn) {
     return rc;
   s.halo_max = hmax;
   s.tile = bn;
+  if (!es) s.parts = stage_parts(s.dim, s.precision, ns, bn);
   if (es) es_set_quantum(s.es, org_range);
   return NLM_OK;
 }

@@ -45,6 +45,7 @@ struct FdArgs {
   const double* __restrict__ tdev;       // step times from device memory
   int kind;            // KIND_* of the launch (k_fd_st)
   int tile;            // nodes of a workgroup's tile
+  int parts;           // wavefronts that share a slice's rows (k_fd_st)
   int64_t halo_bytes;  // LDS bytes of the halo records (k_fd_st)
 };
 
@@ -104,6 +105,7 @@ __device__ __forceinline__ void fext_node(const BcTable* bc, uint32_t fl,
 // KIND_CD: fused force at t_force + central-difference update + BCs at t_next.
 constexpr int KIND_FORCE = 0;
 constexpr int KIND_CD = 1;
+constexpr int kStSplitU = 2;       // slots a chunk of split rows (k_fd_st)
 constexpr int KIND_FORCE_ADD = 2;  // f += internal force
 
 // Fourth dword of a raw buffer resource on gfx9 targets (32-bit untyped
@@ -192,6 +194,7 @@ inline FdArgs<DIM> make_args(nlm_ctx* c) {
   a.tdev = nullptr;
   a.kind = KIND_CD;
   a.tile = s.tile;
+  a.parts = s.parts;
   a.halo_bytes = 0;
   return a;
 }

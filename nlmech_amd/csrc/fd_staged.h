@@ -1,5 +1,5 @@
 // fd_staged.h -- the LDS-staged bond-based step kernel of the FP64 modes
-// (k_fd_st).
+// and of every mode in 3D (k_fd_st).
 //
 // A workgroup owns a tile of the layout's internal order (128, 256 or 512
 // nodes): it stages the tile's halo -- every node its rows reference -- in
@@ -11,6 +11,15 @@
 // after that arithmetic (and the records without the row-length mask):
 // 400 x 397 nodes, horizon 4 h, exact mode 57 -> 28 us; 619 x 451 nodes,
 // FP64 mode, four slots a chunk 48 -> 31 us.
+//
+// Split rows.  One wavefront per 64-node slice leaves a small model a few
+// wavefronts per CU that walk their rows serially (100 x 100 nodes: 157
+// slices on 1024 SIMDs), and the 3D halos leave a CU two tiles.  With SPLIT,
+// `parts` wavefronts share a slice: part p takes the slot chunks p, p +
+// parts, ...  In the FP64 modes the summands pass through LDS in rounds of
+// parts x U slots and are added in list order, so their bits depend
+// on neither the split nor the tile; the FP32-force mode adds the parts' FP64
+// sums at the end in the order of the parts.
 //
 // Launch kinds (a.kind, wavefront-uniform): force, force added to f, the
 // fused central-difference step.
@@ -45,15 +54,45 @@ struct alignas(8) StRec64<DIM, true> {
   uint32_t flags, pad;
 };
 
+// FP32-force mode, 2D: the scaled displacement in FP64, the scaled
+// block-relative position in FP32 (bond_fp32_scaled), the force constant.
+template <int DIM, bool NOFAIL>
+struct alignas(8) StRec32 {
+  double u[2];
+  float xq[2];
+  float c;
+  uint32_t flags;
+  uint32_t pad[2];
+};
+// 3D: the position as a fixed-point offset from the tile's origin in units of
+// the quantum 1/sigma, so a bond's position difference is an exact integer
+// difference rounded once to FP32.
+template <bool NOFAIL>
+struct alignas(8) StRec32<3, NOFAIL> {
+  double u[3];
+  int32_t xq[3];
+  float c;
+};
+template <>
+struct alignas(8) StRec32<3, true> {
+  double u[3];
+  int32_t xq[3];
+  float c;
+  uint32_t flags, pad;
+};
+
 template <int DIM, int MODE, bool NOFAIL>
-using StRec = StRec64<DIM, NOFAIL>;
+using StRec = typename std::conditional<MODE == kModeFp32,
+                                        StRec32<DIM, NOFAIL>,
+                                        StRec64<DIM, NOFAIL>>::type;
 
 // The end of a launch for node i with force density f = base + sum.
 template <int DIM>
 __device__ __forceinline__ void st_tail(const FdArgs<DIM>& a, int64_t i,
                                         uint32_t fl, const double* xi,
-                                        const double* ui, double* acc,
-                                        double t_force, double t_next) {
+                                        const double* ui, const double* vi,
+                                        double* acc, double t_force,
+                                        double t_next) {
   double f[3] = {0., 0., 0.};
   if (a.kind == KIND_FORCE_ADD) {
     load3<DIM>(a.f_in[i], f);
@@ -65,8 +104,6 @@ __device__ __forceinline__ void st_tail(const FdArgs<DIM>& a, int64_t i,
     a.f_out[i] = make_v<DIM>(f);
     return;
   }
-  double vi[3];
-  load3<DIM>(a.v[i], vi);
   double un[3] = {0., 0., 0.}, vn[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) {
     const uint32_t id = (fl >> (kFlagUbcShift + 4 * d)) & 0xfu;
@@ -98,11 +135,29 @@ __device__ __forceinline__ void st_deferred(const FdArgs<DIM>& a, uint32_t g,
   const double vs = ld32(a.vol, g);
   if constexpr (MODE == kModeExact)
     bond_exact<DIM, false>(a.m, xi, ui, xs, us, voli, vs, brk, fs, F, nullptr);
-  else
+  else if constexpr (MODE == kModeFp64)
     bond_fp64<DIM, INF>(a.m, xi, ui, xs, us, voli, vs, brk, fs, F);
+  else
+    bond_fp32<DIM, INF>(a.m, xi, ui, xs, us, voli, vs, brk, fs, F);
 }
 
-template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT>
+// A coordinate as the FP32-force records hold it: its offset from the tile's
+// origin times sigma, in fixed point (3D) or FP32 (2D).
+__device__ __forceinline__ void st_pos(double x, double o, double sigma,
+                                       int32_t& q) {
+  q = __double2int_rn((x - o) * sigma);
+}
+__device__ __forceinline__ void st_pos(double x, double o, double sigma,
+                                       float& q) {
+  q = float((x - o) * sigma);
+}
+__device__ __forceinline__ float st_diff(int32_t a, int32_t b) {
+  return float(int32_t(uint32_t(a) - uint32_t(b)));
+}
+__device__ __forceinline__ float st_diff(float a, float b) { return a - b; }
+
+template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT,
+          bool SPLIT>
 __global__ __launch_bounds__(512) void k_fd_st(
     FdArgs<DIM> a, const unsigned long long* __restrict__ bits_ro,
     const unsigned long long* __restrict__ vex_ro, double t_force,
@@ -111,52 +166,47 @@ __global__ __launch_bounds__(512) void k_fd_st(
     t_force = a.tdev[0];
     t_next = a.tdev[1];
   }
+  constexpr bool F32 = MODE == kModeFp32;
   constexpr bool EXACT = MODE == kModeExact;
+  static_assert(!F32 || DIM == 3 || SPLIT, "2D: k_fd_t, k_fd_w6");
+  typedef typename std::conditional<F32, float, double>::type Real;
   typedef StRec<DIM, MODE, NOFAIL> Rec;
-  const int bn = int(blockDim.x);
+  const int bn = SPLIT ? a.tile : int(blockDim.x);
+  const int parts = SPLIT ? a.parts : 1;
   const int nsl = bn >> 6;  // slices of the tile
   const int64_t nblk = (a.nslices * 64 + bn - 1) / bn;
   const int64_t lb = xcd_block(nblk);
   if (lb >= nblk) return;
   extern __shared__ double st_smem[];
   Rec* const halo_lds = reinterpret_cast<Rec*>(st_smem);
+  double org[3] = {0., 0., 0.};
+  if constexpr (F32)
+    load3<DIM>(reinterpret_cast<const typename VT<DIM>::T*>(a.blk_org)[lb],
+               org);
   const int64_t hb = a.halo_ptr[lb];
   const int hn = int(a.halo_ptr[lb + 1] - hb);
-  for (int t = int(threadIdx.x) - 1; t < hn; t += int(blockDim.x)) {
-    Rec r;
-    if (t < 0) {  // record 0
-      for (int d = 0; d < DIM; d++) r.u[d] = 0.;
-      r.c = 0;
-      for (int d = 0; d < DIM; d++) r.x[d] = 1e15;
-      if constexpr (NOFAIL) r.flags = 0u;
-      halo_lds[0] = r;
-      continue;
-    }
-    const uint32_t g = uint32_t(a.halo[hb + t]);
-    double xg[3], ug[3];
-    load3<DIM>(ld32(a.x, g), xg);
-    load3<DIM>(ld32(a.u, g), ug);
-    const double vg = ld32(a.vol, g);
-    for (int d = 0; d < DIM; d++) {
-      r.x[d] = xg[d];
-      r.u[d] = ug[d];
-    }
-    r.c = EXACT ? vg : vg * a.m.c4_infl;
-    if constexpr (NOFAIL) r.flags = ld32(a.flags, g);
-    halo_lds[t + 1] = r;
-  }
-  __syncthreads();
+  // Loads are issued ahead of their first use: the first halo entry, the
+  // slice's bounds, the node's values and the first slot entries before the
+  // staging (a launch on a small model is a chain of memory latencies).
+  auto halo_id = [&](int t) -> uint32_t {
+    return t >= 0 && t < hn ? uint32_t(a.halo[hb + t]) : 0u;
+  };
+  const int ht = int(threadIdx.x) - 1;
+  uint32_t hg = halo_id(ht);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t s = lb * nsl + wave;
-  if (s >= a.nslices) return;  // whole wavefront
+  const int sl = SPLIT ? wave % nsl : wave;  // slice of the tile
+  const int part = SPLIT ? wave / nsl : 0;
+  const int64_t s = lb * nsl + sl;
+  const bool slice_ok = s < a.nslices;
   const int64_t i = s * 64 + lane;
-  const bool valid = i < a.n;
-  const int64_t cb = a.sl_ptr[s];
-  const int width = int((a.sl_ptr[s + 1] - cb) >> 6);
+  const bool valid = slice_ok && i < a.n;
+  const int64_t cb = slice_ok ? a.sl_ptr[s] : 0;
+  const int width = slice_ok ? int((a.sl_ptr[s + 1] - cb) >> 6) : 0;
   const int64_t bb = cb >> 6;
   const int len = valid ? int(a.rowlen[i]) : 0;
   double xi[3] = {0., 0., 0.}, ui[3] = {0., 0., 0.};
+  double vi[3] = {0., 0., 0.};  // (few wavefronts a CU: fetched early)
   double voli = 1.;
   uint32_t fl = 0;
   if (valid) {
@@ -164,8 +214,19 @@ __global__ __launch_bounds__(512) void k_fd_st(
     load3<DIM>(a.u[i], ui);
     voli = a.vol[i];
     fl = a.flags[i];
+    if constexpr (SPLIT)
+      if (part == 0) load3<DIM>(a.v[i], vi);
   }
   const bool int_i = !(fl & kFlagNonInterior);
+  // FP32-force: the node's fixed-point position and scaled displacement
+  typename std::conditional<DIM == 3, int32_t, float>::type xqi[3] = {0, 0,
+                                                                      0};
+  double uis[3] = {0., 0., 0.};
+  if constexpr (F32)
+    for (int d = 0; d < DIM; d++) {
+      st_pos(xi[d], org[d], a.m.sigma, xqi[d]);
+      uis[d] = ui[d] * a.m.tau;
+    }
   const unsigned long long* __restrict__ bits_in = bits_ro + bb;
   const unsigned long long* __restrict__ vex_in = vex_ro + bb;
   // slot entries through a buffer resource over the slice (fetches past it
@@ -178,25 +239,70 @@ __global__ __launch_bounds__(512) void k_fd_st(
         col_rsrc, lane * int(sizeof(uint16_t)), k * 64 * int(sizeof(uint16_t)),
         0));
   };
+  const int stride = U * parts;
+  int k0 = U * part;
+  uint32_t jn[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) jn[q] = slot_entry(k0 + q);
+  // the halo
+  for (int t = ht; t < hn; t += int(blockDim.x)) {
+    Rec r;
+    if (t < 0) {  // record 0
+      for (int d = 0; d < DIM; d++) r.u[d] = 0.;
+      r.c = 0;
+      for (int d = 0; d < DIM; d++) {
+        if constexpr (F32 && DIM == 3) r.xq[d] = 0x7fffffff;
+        else if constexpr (F32) r.xq[d] = 1e15f;
+        else r.x[d] = 1e15;
+      }
+      if constexpr (NOFAIL) r.flags = 0u;
+      halo_lds[0] = r;
+      hg = halo_id(t + int(blockDim.x));
+      continue;
+    }
+    // (the next halo entry is fetched before this one's node values)
+    const uint32_t g = hg;
+    hg = halo_id(t + int(blockDim.x));
+    double xg[3], ug[3];
+    load3<DIM>(ld32(a.x, g), xg);
+    load3<DIM>(ld32(a.u, g), ug);
+    const double vg = ld32(a.vol, g);
+    for (int d = 0; d < DIM; d++) {
+      if constexpr (F32) {
+        st_pos(xg[d], org[d], a.m.sigma, r.xq[d]);
+        r.u[d] = ug[d] * a.m.tau;
+      } else {
+        r.x[d] = xg[d];
+        r.u[d] = ug[d];
+      }
+    }
+    // (FP32-force 3D: rounded once; 2D: the product k_fd_t forms)
+    if constexpr (F32 && DIM == 3) r.c = float(vg * a.m.c4_infl_s);
+    else if constexpr (F32) r.c = float(vg) * a.m.c4f_infl_s;
+    else r.c = EXACT ? vg : vg * a.m.c4_infl;
+    if constexpr (NOFAIL) r.flags = ld32(a.flags, g);
+    halo_lds[t + 1] = r;
+  }
+  __syncthreads();
+  if (!SPLIT && !slice_ok) return;  // (split tiles meet at barriers)
   const unsigned long long int_m =
       NOFAIL ? __builtin_amdgcn_ballot_w64(int_i) : ~0ull;
   // one chunk of U slots from slot k0: the bonds' forces (exact mode: F[q])
   // or the slot pairs' sums (fast modes: F[m])
   constexpr int NF = EXACT ? U : U / 2;
-  uint32_t jn[U];
-  auto chunk = [&](int k0, double (&F)[NF][DIM]) {
+  auto chunk = [&](int k0, int k_next, Real (&F)[NF][DIM]) {
     uint32_t jc[U];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       jc[q] = jn[q];
-      jn[q] = slot_entry(k0 + U + q);
+      jn[q] = slot_entry(k_next + q);
     }
     unsigned long long w[U], vx[U], brk[U], band[U], ex[U];
     unsigned long long ex_any = 0ull;
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       w[q] = bits_in[k0 + q];
-      vx[q] = vex_in[k0 + q];
+      vx[q] = F32 ? 0ull : vex_in[k0 + q];
     }
 #pragma unroll
     for (int q = 0; q < U; ++q) {
@@ -214,20 +320,40 @@ __global__ __launch_bounds__(512) void k_fd_st(
       else
         km.brk = ~0ull;
       brk[q] = km.brk;
-      double dx[DIM], du[DIM];
-      for (int d = 0; d < DIM; d++) {
-        dx[d] = r->x[d] - xi[d];
-        du[d] = r->u[d] - ui[d];
+      if constexpr (F32) {
+        float dx[3] = {0.f, 0.f, 0.f}, dv[3] = {0.f, 0.f, 0.f};
+        float G[3] = {0.f, 0.f, 0.f};
+        for (int d = 0; d < DIM; d++) {
+          dx[d] = st_diff(r->xq[d], xqi[d]);
+          dv[d] = float(r->u[d] - uis[d]);
+          if (q % 2 == 1) G[d] = F[q / 2][d];
+        }
+        unsigned long long nb;
+        if (q % 2 == 1)
+          bond_fp32_scaled<DIM, INF, NOFAIL, true>(
+              a.m, dx[0], dx[1], dx[2], dv[0], dv[1], dv[2], r->c, km, nb,
+              band[q], ex[q], G);
+        else
+          bond_fp32_scaled<DIM, INF, NOFAIL, false>(
+              a.m, dx[0], dx[1], dx[2], dv[0], dv[1], dv[2], r->c, km, nb,
+              band[q], ex[q], G);
+        for (int d = 0; d < DIM; d++) F[q / 2][d] = G[d];
+      } else {
+        double dx[DIM], du[DIM];
+        for (int d = 0; d < DIM; d++) {
+          dx[d] = r->x[d] - xi[d];
+          du[d] = r->u[d] - ui[d];
+        }
+        if constexpr (EXACT)
+          bond_exact_fast<DIM, INF, NOFAIL, SHORT>(a.m, dx, du, r->c, km,
+                                                   band[q], ex[q], F[q]);
+        else if (q % 2 == 1)
+          bond_fp64_staged<DIM, INF, NOFAIL, SHORT, true>(
+              a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
+        else
+          bond_fp64_staged<DIM, INF, NOFAIL, SHORT, false>(
+              a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
       }
-      if constexpr (EXACT)
-        bond_exact_fast<DIM, INF, NOFAIL, SHORT>(a.m, dx, du, r->c, km,
-                                                 band[q], ex[q], F[q]);
-      else if (q % 2 == 1)
-        bond_fp64_staged<DIM, INF, NOFAIL, SHORT, true>(
-            a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
-      else
-        bond_fp64_staged<DIM, INF, NOFAIL, SHORT, false>(
-            a.m, dx, du, r->c, km, band[q], ex[q], F[q / 2]);
       ex_any |= ex[q];
     }
     if (ex_any != 0ull) {  // rare: whole wavefronts skip it
@@ -245,9 +371,11 @@ __global__ __launch_bounds__(512) void k_fd_st(
               a, g, xi, ui, voli,
               __builtin_amdgcn_inverse_ballot_w64(brk[q]), fs, Fd);
           fsn = fs && !fs0;
+          // (FP32-force: a bond force is an FP32 value; a contact force is
+          // rounded to FP32 here like every force of that mode)
           for (int d = 0; d < DIM; d++) {
             if constexpr (EXACT) F[q][d] = Fd[d];
-            else F[q / 2][d] += Fd[d];
+            else F[q / 2][d] += Real(Fd[d]);
           }
         }
         // new broken bits: every lane stores the same word
@@ -258,63 +386,147 @@ __global__ __launch_bounds__(512) void k_fd_st(
     }
   };
   double acc[3] = {0., 0., 0.};
+  if constexpr (SPLIT && !F32) {
+    // rounds of parts x U slots: the summands (exact mode: forces, FP64 mode:
+    // pair sums) through LDS, added in list order by the wavefront of the
+    // (slice, component) task
+    double* const buf = reinterpret_cast<double*>(
+        reinterpret_cast<char*>(st_smem) + a.halo_bytes);
+    const int nv = NF * parts;  // summands of a lane's component in a round
+    int wmax = 0;
+    for (int q = 0; q < nsl; q++) {
+      const int64_t t = lb * nsl + q;
+      if (t < a.nslices)
+        wmax = max(wmax, int((a.sl_ptr[t + 1] - a.sl_ptr[t]) >> 6));
+    }
+    const int nw = nsl * parts;
+    const int ntask = nsl * DIM;
+    constexpr int MT = 2;  // tasks a wavefront (parts >= 2, DIM <= 3)
+    double sum[MT] = {0., 0.};
+    int tw[MT];
 #pragma unroll
-  for (int q = 0; q < U; ++q) jn[q] = slot_entry(q);
-  for (int k0 = 0; k0 < width; k0 += U) {
-    double F[NF][DIM];
-    chunk(k0, F);
+    for (int t = 0; t < MT; t++) {
+      const int task = wave + t * nw;
+      const int64_t ts = lb * nsl + task / DIM;
+      tw[t] = task < ntask && ts < a.nslices
+                  ? int((a.sl_ptr[ts + 1] - a.sl_ptr[ts]) >> 6)
+                  : 0;
+    }
+    for (int base = 0; base < wmax; base += stride, k0 += stride) {
+      if (k0 < width) {
+        double F[NF][DIM];
+        chunk(k0, k0 + stride, F);
 #pragma unroll
-    for (int m = 0; m < NF; ++m)
-      for (int d = 0; d < DIM; d++) acc[d] += F[m][d];
+        for (int m = 0; m < NF; ++m)
+          for (int d = 0; d < DIM; d++)
+            buf[((sl * DIM + d) * nv + part * NF + m) * 64 + lane] = F[m][d];
+      }
+      __syncthreads();
+      // (slots past a row are exact zeros; chunks past a slice were not
+      // written)
+#pragma unroll
+      for (int t = 0; t < MT; t++) {
+        const int cnt = min(nv, (tw[t] - base + U - 1) / U * NF);
+        const double* const v = buf + (wave + t * nw) * nv * 64 + lane;
+        for (int m = 0; m < cnt; m++) sum[t] += v[m * 64];
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      const int task = wave + t * nw;
+      if (task < ntask) buf[task * 64 + lane] = sum[t];
+    }
+    __syncthreads();
+    if (part == 0)
+      for (int d = 0; d < DIM; d++) acc[d] = buf[(sl * DIM + d) * 64 + lane];
+  } else {
+    for (; k0 < width; k0 += stride) {
+      Real F[NF][DIM];
+      chunk(k0, k0 + stride, F);
+#pragma unroll
+      for (int m = 0; m < NF; ++m)
+        for (int d = 0; d < DIM; d++) acc[d] += double(F[m][d]);
+    }
+    if constexpr (SPLIT) {
+      // the parts' sums, added in the order of the parts
+      double* const buf = reinterpret_cast<double*>(
+          reinterpret_cast<char*>(st_smem) + a.halo_bytes);
+      if (part > 0)
+        for (int d = 0; d < DIM; d++)
+          buf[((sl * (parts - 1) + part - 1) * DIM + d) * 64 + lane] = acc[d];
+      __syncthreads();
+      if (part == 0)
+        for (int p = 0; p < parts - 1; p++)
+          for (int d = 0; d < DIM; d++)
+            acc[d] += buf[((sl * (parts - 1) + p) * DIM + d) * 64 + lane];
+    }
   }
-  if (!valid) return;
-  st_tail<DIM>(a, i, fl, xi, ui, acc, t_force, t_next);
+  if (!valid || part != 0) return;
+  if constexpr (!SPLIT) load3<DIM>(a.v[i], vi);
+  st_tail<DIM>(a, i, fl, xi, ui, vi, acc, t_force, t_next);
 }
 
-inline size_t st_rec_bytes(int dim, bool nofail) {
-  return size_t(2 * dim + 1) * 8 + (nofail ? 8 : 0);
+// LDS bytes behind the halo records of a split launch: the FP64 modes' round
+// buffer, the FP32-force mode's sums.
+inline size_t st_round_bytes(int dim, int precision, int tile, int parts) {
+  const size_t per = precision == kModeExact  ? size_t(kStSplitU * parts)
+                     : precision == kModeFp64 ? size_t(kStSplitU / 2 * parts)
+                                              : size_t(parts - 1);
+  return size_t(tile / 64) * dim * per * 64 * 8;
 }
 
-// Launch of the staged kernel for the configured tile (fd_st2.hip).
+// Bytes of a halo record.
+inline size_t st_rec_bytes(int dim, int precision, bool nofail) {
+  return (precision == kModeFp32 ? sizeof(StRec32<3, false>)
+                                 : size_t(2 * dim + 1) * 8) +
+         (nofail && !(dim == 2 && precision == kModeFp32) ? 8 : 0);
+}
+
+// Launch of the staged kernel for the configured tile (fd_st2.hip,
+// fd_st3.hip).
 void st_launch2(nlm_ctx* c, const FdArgs<2>& a, double tf, double tn, int U);
+void st_launch3(nlm_ctx* c, const FdArgs<3>& a, double tf, double tn, int U);
 // Whether the kernels' static LDS size is 0, as their addressing needs.
 bool st_lds_base_zero();
 
 // Instances of one dimension and mode.
-template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT>
+template <int DIM, int MODE, int INF, int U, bool NOFAIL, bool SHORT,
+          bool SPLIT>
 void st_go(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
   static_assert(sizeof(StRec<DIM, MODE, NOFAIL>) % 8 == 0, "record");
   const unsigned g = grid_xcd(c->fd.sell.nslices * 64, a.tile);
-  const size_t lds = size_t(a.halo_bytes);
+  size_t lds = size_t(a.halo_bytes);
+  if constexpr (SPLIT) lds += st_round_bytes(DIM, MODE, a.tile, a.parts);
   allow_lds(reinterpret_cast<const void*>(
-                &k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT>),
+                &k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT, SPLIT>),
             lds);
-  hipLaunchKernelGGL((k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT>),
-                     dim3(g), dim3(unsigned(a.tile)), lds,
+  hipLaunchKernelGGL((k_fd_st<DIM, MODE, INF, U, NOFAIL, SHORT, SPLIT>),
+                     dim3(g), dim3(unsigned(a.tile * a.parts)), lds,
                      c->stream, a, a.bits, a.vexw, tf, tn);
 }
 
-template <int DIM, int MODE, int U, bool SHORT, bool NOFAIL>
+template <int DIM, int MODE, int U, bool SPLIT, bool SHORT, bool NOFAIL>
 void st_inf(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
   const int inf = c->fd.rnp.inf_type;
   if (inf == 0)
-    st_go<DIM, MODE, 0, U, NOFAIL, SHORT>(c, a, tf, tn);
+    st_go<DIM, MODE, 0, U, NOFAIL, SHORT, SPLIT>(c, a, tf, tn);
   else if (inf == 1)
-    st_go<DIM, MODE, 1, U, NOFAIL, SHORT>(c, a, tf, tn);
+    st_go<DIM, MODE, 1, U, NOFAIL, SHORT, SPLIT>(c, a, tf, tn);
   else
-    st_go<DIM, MODE, 2, U, NOFAIL, SHORT>(c, a, tf, tn);
+    st_go<DIM, MODE, 2, U, NOFAIL, SHORT, SPLIT>(c, a, tf, tn);
 }
 
-template <int DIM, int MODE, int U>
+template <int DIM, int MODE, int U, bool SPLIT>
 void st_opt(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn) {
   // the exponent's range form is chosen where the break test bounds it
   // (exp_short); models with no-fail regions keep the general form
   if (a.has_nofail)
-    st_inf<DIM, MODE, U, false, true>(c, a, tf, tn);
-  else if (a.m.x_break_lo <= kExpShortMax)
-    st_inf<DIM, MODE, U, true, false>(c, a, tf, tn);
+    st_inf<DIM, MODE, U, SPLIT, false, true>(c, a, tf, tn);
+  else if (MODE != kModeFp32 && a.m.x_break_lo <= kExpShortMax)
+    st_inf<DIM, MODE, U, SPLIT, MODE != kModeFp32, false>(c, a, tf, tn);
   else
-    st_inf<DIM, MODE, U, false, false>(c, a, tf, tn);
+    st_inf<DIM, MODE, U, SPLIT, false, false>(c, a, tf, tn);
 }
 
 }  // namespace nlm

@@ -68,7 +68,7 @@ void parallel_chunks(int64_t count, F body) {
 }  // namespace
 
 void build_layout(int dim, int64_t n, const double* x, double cell,
-                  const int64_t* rp_ref, const int32_t* col_ref,
+                  const int64_t* rp_ref, const int32_t* col_ref, int bs,
                   HostLayout& L) {
   // --- permutation ------------------------------------------------------
   double lo[3] = {1e300, 1e300, 1e300};
@@ -143,9 +143,9 @@ void build_layout(int dim, int64_t n, const double* x, double cell,
     }
   });
 
-  // --- halos of 256-node blocks ----------------------------------------------
-  L.nblocks = (nslices + 3) / 4;
-  build_halos(n, nslices, L.sl_ptr.data(), L.colS.data(), 4, L.halo_ptr,
+  // --- halos of blocks of bs slices -------------------------------------------
+  L.nblocks = (nslices + bs - 1) / bs;
+  build_halos(n, nslices, L.sl_ptr.data(), L.colS.data(), bs, L.halo_ptr,
               L.halo, L.colL, L.halo_max);
 }
 

@@ -17,7 +17,7 @@ struct HostLayout {
   std::vector<int64_t> sl_ptr;   // slice starts (entries, multiples of 64)
   std::vector<int32_t> colS;     // slice entries, internal ids
   std::vector<uint16_t> rowlen;
-  int64_t nblocks = 0;           // blocks of 4 slices (256 nodes)
+  int64_t nblocks = 0;           // blocks of bs slices (64 bs nodes)
   std::vector<int64_t> halo_ptr;
   std::vector<int32_t> halo;     // per block: sorted internal ids
   std::vector<uint16_t> colL;    // slice entries, halo-local indices
@@ -25,9 +25,10 @@ struct HostLayout {
 };
 
 // Builds the layout for n nodes at x (AoS Point3) with the reference-order
-// CSR (rp_ref, col_ref); cell is the Morton cell edge (the mesh size).
+// CSR (rp_ref, col_ref); cell is the Morton cell edge (the mesh size); bs:
+// slices of a halo block (build_halos).
 void build_layout(int dim, int64_t n, const double* x, double cell,
-                  const int64_t* rp_ref, const int32_t* col_ref,
+                  const int64_t* rp_ref, const int32_t* col_ref, int bs,
                   HostLayout& L);
 
 // Halos of blocks of bs consecutive slices (64 bs nodes, one workgroup of

@@ -113,6 +113,7 @@ struct RnpDev {
   // lower bound of the break test's guard band on beta r S^2 (+inf when bonds
   // never break)
   double c4_infl, up_rcp_h, x_break_lo;
+  double c4_infl_s;        // c4_infl sigma / tau (3D FP32-force records)
 };
 
 // ElasticState constants as used by the kernels.
@@ -196,7 +197,8 @@ struct FdState {
   int cur = 0;  // which of u[]/v[] holds the current state
   int unroll = 4;  // neighbor slots per chunk in the fused step kernel
   int tile = 256;  // nodes per workgroup of the LDS-staged kernel (its halo
-                   // block): 128, 256 or 512
+                   // block): 128, 256 or 512 (k_fd_st also 64)
+  int parts = 1;   // wavefronts that share a slice's rows (k_fd_st)
   DevBuf row_ptr, col;  // CSR in internal ids (int64, int32)
   SellDev sell;
   // internal node order (see layout.cpp): perm[a] = reference id of a

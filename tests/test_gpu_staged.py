@@ -8,20 +8,27 @@ Bars, per node, relative to sum_j |F_ij| of the oracle's bond forces:
     and host values differ by at most 2 ulp in each bond force, and the
     rounding of the running sum that follows from it (half an ulp per
     addition, up to 24 slots): 2 + 12 ulp, taken as 16 x 2^-52;
+  (3D: rows of up to 92 slots, 2 + 46 ulp, taken as 64 x 2^-52;)
   FP64: about 20 roundings of half an ulp per bond force (fused operations,
     the third-order reciprocal root below one ulp entering three times) and
-    the same sum: 64 x 2^-52.
+    the same sum: 64 x 2^-52 (3D: 92 additions in pairs, 96 x 2^-52);
+  FP32-force (3D): fixed-point positions to 2^-28 of the tile's extent
+    (about 10 h, 4e-8 of a bond), 25 FP32 roundings of 2^-24 and the rsq and
+    exp2 approximations of 2^-23: 2e-6.
 """
 import numpy as np
 import pytest
 
 from conftest import progress
 from nlmech_amd import problems as pr
-from nlmech_amd.capi import NLM_PREC_FP64, NLM_PREC_FP64_EXACT
+from nlmech_amd.capi import (NLM_PREC_FP32_FORCE, NLM_PREC_FP64,
+                             NLM_PREC_FP64_EXACT)
 
 pytestmark = pytest.mark.gpu
 
 ULP = 2.0 ** -52
+BAR3 = {NLM_PREC_FP64_EXACT: 64 * ULP, NLM_PREC_FP64: 96 * ULP,
+        NLM_PREC_FP32_FORCE: 2e-6}
 BAR = {NLM_PREC_FP64_EXACT: 16 * ULP, NLM_PREC_FP64: 64 * ULP}
 
 
@@ -67,3 +74,102 @@ def test_staged_force(oracle, precision, mat, shape):
         assert bonds.sum() > b0
     err = np.abs(f - o.get_state()[2]).max(1)
     assert np.all(err <= BAR[precision] * scale), (err / scale).max() / ULP
+
+
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("shape,mat", [((4, 4, 4), dict()),
+                                       ((13, 11, 9), dict()),
+                                       ((13, 11, 9), dict(check_sc=10.0)),
+                                       ((9, 9, 9), dict(inf_type=1,
+                                                        inf_params=()))],
+                         ids=["64", "1287", "sc10", "linear"])
+def test_staged_force_3d(oracle, precision, shape, mat):
+    progress(f"[gpu] staged force 3D {shape} {mat} mode {precision}")
+    h = 1e-3
+    x, vol = pr.grid3d(*shape, h, jitter=0.05, seed=4)
+    p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                   dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3, **mat),
+                   shape=shape)
+    if shape == (9, 9, 9):
+        p.interior = np.ones(p.n, np.uint8)
+        p.interior[::7] = 0
+    rng = np.random.default_rng(2)
+    u = rng.normal(scale=6e-6, size=(p.n, 3))
+    o = oracle.OracleFD(p)
+    o.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+    scale = o.force_abs_sum()
+    o.compute_forces()
+    f, bonds = force_of(p, precision, u)
+    assert np.array_equal(bonds, o.get_bonds())
+    if "check_sc" not in mat:
+        assert bonds.sum() > 0
+    err = np.abs(f - o.get_state()[2]).max(1)
+    assert np.all(err <= BAR3[precision] * scale), (err / scale).max()
+
+
+# Trajectories over the sizes at which the rule for tiles and split rows
+# changes (slices of 64 nodes: 256, 800, 2500, 3000), through the whole step:
+# the FP64 modes agree with the oracle, and a tile set by hand (with its own
+# split) gives the same bits, because split rows are added in list order.
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(128, 127), (128, 129), (226, 226),
+                                   (230, 227), (438, 438), (440, 439)],
+                         ids=["254", "258", "799", "816", "2998", "3019"])
+def test_split_rows(oracle, precision, shape):
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] split rows {shape} mode {precision}")
+    p = pr.plate2d(*shape, 1e-3, 3, 1e-7, 12, pull=30.0, jitter=0.02)
+    o = oracle.OracleFD(p)
+    o.init()
+    o.step(12)
+    ur = o.get_state()[0]
+    outs = []
+    for tile in (None, 128, 256, 512):
+        with GpuFD(p, precision=precision) as g:
+            if tile:
+                g.set_tile(tile)
+            g.init()
+            g.step(12)
+            outs.append(g.get_state() + (g.get_bonds(),))
+    u, _, _, bonds = outs[0]
+    if precision == NLM_PREC_FP32_FORCE:
+        assert np.linalg.norm(u - ur) <= 1e-6 * np.linalg.norm(ur)
+        return
+    assert np.array_equal(bonds, o.get_bonds()) and bonds.sum() > 0
+    assert np.linalg.norm(u - ur) <= 1e-13 * np.linalg.norm(ur)
+    for other in outs[1:]:
+        for a, b in zip(outs[0], other):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(25, 25, 26), (26, 26, 25), (37, 37, 37),
+                                   (54, 54, 55)],
+                         ids=["254", "265", "792", "2506"])
+def test_split_rows_3d(oracle, precision, shape):
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] split rows 3D {shape} mode {precision}")
+    h = 1e-3
+    x, vol = pr.grid3d(*shape, h, jitter=0.02, seed=4)
+    p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                   dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3),
+                   v0=np.random.default_rng(3).normal(size=x.shape))
+    o = oracle.OracleFD(p)
+    o.init()
+    o.step(4)
+    u_ref = o.get_state()[0]
+    with GpuFD(p, precision=precision) as g:
+        g.init()
+        g.step(4)
+        u, bonds = g.get_state()[0], g.get_bonds()
+    f32 = precision == NLM_PREC_FP32_FORCE
+    assert (np.linalg.norm(u - u_ref) <=
+            (1e-6 if f32 else 1e-13) * np.linalg.norm(u_ref))
+    if not f32:
+        assert np.array_equal(bonds, o.get_bonds())
