@@ -43,7 +43,7 @@ struct FdArgs {
   int has_nofail;
   const double* __restrict__ node_rate;  // node-list BC rates (or null)
   const double* __restrict__ tdev;       // step times from device memory
-  int kind;            // KIND_* of the launch (k_fd_st)
+  int kind;            // KIND_* of the launch (k_fd_st; of the fused step)
   int tile;            // nodes of a workgroup's tile
   int parts;           // wavefronts that share a slice's rows (k_fd_st)
   int64_t halo_bytes;  // LDS bytes of the halo records (k_fd_st)
@@ -107,6 +107,9 @@ constexpr int KIND_FORCE = 0;
 constexpr int KIND_CD = 1;
 constexpr int kStSplitU = 2;       // slots a chunk of split rows (k_fd_st)
 constexpr int KIND_FORCE_ADD = 2;  // f += internal force
+// the fused velocity-Verlet step: the force at t_force, the end of its step
+// and the start of the next (FDModel::integrateVerlet, fDModel.cpp:446-525)
+constexpr int KIND_VERLET = 3;
 
 // Fourth dword of a raw buffer resource on gfx9 targets (32-bit untyped
 // accesses, range-checked against the record count).
@@ -119,6 +122,18 @@ template <class T>
 __device__ __forceinline__ T ld32(const T* __restrict__ base, uint32_t idx) {
   return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
                                      idx * uint32_t(sizeof(T)));
+}
+
+// A free dof of the fused velocity-Verlet step: v += fact f ends the step,
+// v += fact f and u += dt v start the next.
+template <int DIM>
+__device__ __forceinline__ void verlet_dof(const FdArgs<DIM>& a, double f,
+                                           double uo, double vo, double& un,
+                                           double& vn) {
+  const double df = a.fact * f;
+  vn = vo + df;
+  vn += df;
+  un = uo + a.dt * vn;
 }
 
 // Central-difference tail of a fused step for node i: f is the total force

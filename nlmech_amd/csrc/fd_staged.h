@@ -22,7 +22,7 @@
 // sums at the end in the order of the parts.
 //
 // Launch kinds (a.kind, wavefront-uniform): force, force added to f, the
-// fused central-difference step.
+// fused central-difference step and the fused velocity-Verlet step.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -109,9 +109,13 @@ __device__ __forceinline__ void st_tail(const FdArgs<DIM>& a, int64_t i,
     const uint32_t id = (fl >> (kFlagUbcShift + 4 * d)) & 0xfu;
     if (id == 0) {
       const double uo = ui[d];
-      // u += fact*f + dt*v; v = (u - u_old)/dt  (fDModel.cpp:386-394)
-      un[d] = uo + (a.fact * f[d] + a.dt * vi[d]);
-      vn[d] = (un[d] - uo) / a.dt;
+      if (a.kind == KIND_VERLET) {
+        verlet_dof(a, f[d], uo, vi[d], un[d], vn[d]);
+      } else {
+        // u += fact*f + dt*v; v = (u - u_old)/dt  (fDModel.cpp:386-394)
+        un[d] = uo + (a.fact * f[d] + a.dt * vi[d]);
+        vn[d] = (un[d] - uo) / a.dt;
+      }
     } else {
       double du, dv;
       ubc_dof(a, id, i, d, xi, t_next, du, dv);

@@ -173,3 +173,43 @@ def test_split_rows_3d(oracle, precision, shape):
             (1e-6 if f32 else 1e-13) * np.linalg.norm(u_ref))
     if not f32:
         assert np.array_equal(bonds, o.get_bonds())
+
+
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("shape", [(9, 8), (130, 127), (9, 8, 7)],
+                         ids=["72", "16510", "3d"])
+def test_fused_verlet_steps(precision, shape):
+    """The fused velocity-Verlet launches of one call (steps 2..n) give the
+    bits of n calls of one step, whose update and force are launches of their
+    own; a crack activated on the way and a force BC included."""
+    from nlmech_amd.capi import NLM_TIME_VELOCITY_VERLET
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] fused verlet {shape} mode {precision}")
+    h, dim = 1e-3, len(shape)
+    if dim == 2:
+        p = pr.plate2d(*shape, h, 3, 1e-7, 1, notch_len=0.0, pull=30.0,
+                       layers=2, jitter=0.05)
+        y = (shape[1] // 2 - 0.5) * h
+        p.cracks = [pr.CrackSpec(1, (-0.5 * h, y), (3.5 * h, y),
+                                 activation_time=2.5e-7)]
+        p.fbc = [pr.BC("rectangle", [1], "linear", [1e15], x1=-h, x2=2.5 * h,
+                       y1=-h, y2=shape[1] * h)]
+    else:
+        x, vol = pr.grid3d(*shape, h, jitter=0.05, seed=4)
+        p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                       dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3),
+                       v0=np.random.default_rng(3).normal(size=x.shape))
+    outs = []
+    for calls in ((6,), (1,) * 6):
+        with GpuFD(p, precision=precision,
+                   scheme=NLM_TIME_VELOCITY_VERLET) as g:
+            g.init()
+            for k in calls:
+                g.step(k)
+            outs.append(g.get_state() + (g.get_bonds(), g.time()))
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    if dim == 2:
+        assert outs[0][3].sum() > 0
