@@ -1221,6 +1221,14 @@ __global__ __launch_bounds__(256) void k_es_fields(
   put(stress6, S);
 }
 
+// A node field (internal order) in reference order.
+__global__ __launch_bounds__(256) void k_out_scalar(
+    int64_t n, const double* __restrict__ src,
+    const int32_t* __restrict__ perm, double* __restrict__ dst) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) dst[perm[i]] = src[i];
+}
+
 }  // namespace
 
 }  // namespace nlm
@@ -1291,16 +1299,23 @@ extern "C" int nlm_fd_get_node_fields(nlm_ctx* c, double* theta, double* mw) {
   if (s.material != NLM_MATERIAL_ELASTIC_STATE)
     return fail(c, NLM_ERR_INVALID,
                 "nlm_fd_get_node_fields: state-based material only");
-  std::vector<double> a(s.n), b(s.n);
-  NLM_HIP(c, hipMemcpyAsync(a.data(), s.es_theta.p, sizeof(double) * s.n,
-                            hipMemcpyDeviceToHost, c->stream));
-  NLM_HIP(c, hipMemcpyAsync(b.data(), s.es_mw.p, sizeof(double) * s.n,
-                            hipMemcpyDeviceToHost, c->stream));
+  const double* const src[2] = {s.es_theta.as<double>(),
+                                s.es_mw.as<double>()};
+  double* const dst[2] = {theta, mw};
+  int rc;
+  if ((rc = reserve(c, s.out, 2 * sizeof(double) * size_t(s.n)))) return rc;
+  const unsigned g = unsigned((s.n + 255) / 256);
+  for (int k = 0; k < 2; k++)
+    if (dst[k])
+      hipLaunchKernelGGL(k_out_scalar, dim3(g), dim3(256), 0, c->stream, s.n,
+                         src[k], s.perm_dev.as<int32_t>(),
+                         s.out.as<double>() + k * s.n);
+  NLM_HIP(c, hipGetLastError());
+  for (int k = 0; k < 2; k++)
+    if (dst[k])
+      NLM_HIP(c, hipMemcpyAsync(dst[k], s.out.as<double>() + k * s.n,
+                                sizeof(double) * size_t(s.n),
+                                hipMemcpyDeviceToHost, c->stream));
   NLM_HIP(c, hipStreamSynchronize(c->stream));
-  for (int64_t k = 0; k < s.n; k++) {
-    const int64_t i = s.perm_host[k];
-    if (theta) theta[i] = a[k];
-    if (mw) mw[i] = b[k];
-  }
   return NLM_OK;
 }

@@ -811,6 +811,22 @@ __global__ __launch_bounds__(256) void k_postproc(
   if (energy) energy[o] = energy_i * voli;
 }
 
+// A node vector (internal order) as the boundary takes it: 3 components per
+// node in reference order, z = 0 in 2D.
+template <int DIM>
+__global__ __launch_bounds__(256) void k_out_vec(
+    int64_t n, const typename VT<DIM>::T* __restrict__ src,
+    const int32_t* __restrict__ perm, double* __restrict__ dst) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  double v[3];
+  load3<DIM>(src[i], v);
+  double* const o = dst + 3 * int64_t(perm[i]);
+  o[0] = v[0];
+  o[1] = v[1];
+  o[2] = v[2];
+}
+
 // External force density of every node at time t: FLoading::apply on a zero
 // force vector (fLoading.cpp:117-279), as FDModel::computePostProcFields
 // takes it for the work done (fDModel.cpp:655-662).  Internal order, 3
@@ -1924,17 +1940,37 @@ int to_dev_vec(nlm_ctx* c, const double* src, DevBuf& dst) {
                        hipMemcpyHostToDevice));
   return NLM_OK;
 }
-int from_dev_vec(nlm_ctx* c, const DevBuf& src, double* dst) {
+// Node vectors in reference order to the host: reordered on the device (a
+// host loop over the permutation took 2 to 4 ms a vector of 1e6 nodes), one
+// copy each, one wait.
+int from_dev_vecs(nlm_ctx* c, int count, const DevBuf* const* src,
+                  double* const* dst) {
   FdState& s = c->fd;
-  const int stride = s.dim == 2 ? 2 : 4;
-  std::vector<double> tmp(size_t(s.n) * stride, 0.);
-  NLM_HIP(c, hipMemcpy(tmp.data(), src.p, sizeof(double) * tmp.size(),
-                       hipMemcpyDeviceToHost));
-  for (int64_t a = 0; a < s.n; a++) {
-    const int64_t i = s.perm_host[a];
-    for (int d = 0; d < 3; d++)
-      dst[3 * i + d] = d < s.dim ? tmp[a * stride + d] : 0.;
+  const size_t vec = sizeof(double) * 3 * size_t(s.n);
+  int rc, used = 0;
+  for (int k = 0; k < count; k++) used += dst[k] != nullptr;
+  if ((rc = reserve(c, s.out, vec * size_t(std::max(used, 1))))) return rc;
+  const int32_t* perm = s.perm_dev.as<int32_t>();
+  double* o = s.out.as<double>();
+  for (int k = 0; k < count; k++) {
+    if (!dst[k]) continue;
+    if (s.dim == 2)
+      hipLaunchKernelGGL(k_out_vec<2>, dim3(node_blocks(s)), dim3(256), 0,
+                         c->stream, s.n, src[k]->as<double2>(), perm, o);
+    else
+      hipLaunchKernelGGL(k_out_vec<3>, dim3(node_blocks(s)), dim3(256), 0,
+                         c->stream, s.n, src[k]->as<double4>(), perm, o);
+    o += 3 * s.n;
   }
+  NLM_HIP(c, hipGetLastError());
+  o = s.out.as<double>();
+  for (int k = 0; k < count; k++) {
+    if (!dst[k]) continue;
+    NLM_HIP(c, hipMemcpyAsync(dst[k], o, vec, hipMemcpyDeviceToHost,
+                              c->stream));
+    o += 3 * s.n;
+  }
+  NLM_HIP(c, hipStreamSynchronize(c->stream));
   return NLM_OK;
 }
 }  // namespace
@@ -1954,12 +1990,10 @@ extern "C" int nlm_fd_set_state(nlm_ctx* c, const double* u, const double* v,
 extern "C" int nlm_fd_get_state(nlm_ctx* c, double* u, double* v, double* f) {
   int rc = check_ready(c, "nlm_fd_get_state");
   if (rc) return rc;
-  NLM_HIP(c, hipStreamSynchronize(c->stream));
   FdState& s = c->fd;
-  if (u && (rc = from_dev_vec(c, s.u[s.cur], u))) return rc;
-  if (v && (rc = from_dev_vec(c, s.v[s.cur], v))) return rc;
-  if (f && (rc = from_dev_vec(c, s.f, f))) return rc;
-  return NLM_OK;
+  const DevBuf* const src[3] = {&s.u[s.cur], &s.v[s.cur], &s.f};
+  double* const dst[3] = {u, v, f};
+  return from_dev_vecs(c, 3, src, dst);
 }
 
 extern "C" int nlm_fd_get_bonds(nlm_ctx* c, uint8_t* out) {
@@ -2150,38 +2184,33 @@ extern "C" int nlm_fd_postproc(nlm_ctx* c, float* Z, float* phi,
   if (s.material != NLM_MATERIAL_RNP_BOND)
     return fail(c, NLM_ERR_INVALID,
                 "nlm_fd_postproc: bond-based material only");
-  DevBuf dz, dp, de;
-  if ((rc = alloc(c, dz, sizeof(float) * s.n))) return rc;
-  if ((rc = alloc(c, dp, sizeof(float) * s.n))) return rc;
-  if ((rc = alloc(c, de, sizeof(double) * s.n))) return rc;
+  // fields in reference order in the context's staging, the outputs copied
+  // from there
+  const size_t n = size_t(s.n);
+  if ((rc = reserve(c, s.out, (sizeof(double) + 2 * sizeof(float)) * n)))
+    return rc;
+  double* const de = s.out.as<double>();
+  float* const dz = reinterpret_cast<float*>(de + n);
+  float* const dp = dz + n;
+  const int32_t* const perm = s.perm_dev.as<int32_t>();
   unsigned g = unsigned((s.sell.nslices * 64 + 255) / 256);
-  if (s.dim == 2) {
-    FdArgs<2> a = make_args<2>(c);
-    hipLaunchKernelGGL(k_postproc<2>, dim3(g), dim3(256), 0, c->stream, a,
-                       dz.as<float>(), dp.as<float>(), de.as<double>(),
-                       nullptr);
-  } else {
-    FdArgs<3> a = make_args<3>(c);
-    hipLaunchKernelGGL(k_postproc<3>, dim3(g), dim3(256), 0, c->stream, a,
-                       dz.as<float>(), dp.as<float>(), de.as<double>(),
-                       nullptr);
-  }
+  if (s.dim == 2)
+    hipLaunchKernelGGL(k_postproc<2>, dim3(g), dim3(256), 0, c->stream,
+                       make_args<2>(c), dz, dp, de, perm);
+  else
+    hipLaunchKernelGGL(k_postproc<3>, dim3(g), dim3(256), 0, c->stream,
+                       make_args<3>(c), dz, dp, de, perm);
   NLM_HIP(c, hipGetLastError());
-  std::vector<float> hz(s.n), hp(s.n);
-  std::vector<double> he(s.n);
-  NLM_HIP(c, hipMemcpyAsync(hz.data(), dz.p, sizeof(float) * s.n,
-                            hipMemcpyDeviceToHost, c->stream));
-  NLM_HIP(c, hipMemcpyAsync(hp.data(), dp.p, sizeof(float) * s.n,
-                            hipMemcpyDeviceToHost, c->stream));
-  NLM_HIP(c, hipMemcpyAsync(he.data(), de.p, sizeof(double) * s.n,
-                            hipMemcpyDeviceToHost, c->stream));
+  if (Z)
+    NLM_HIP(c, hipMemcpyAsync(Z, dz, sizeof(float) * n, hipMemcpyDeviceToHost,
+                              c->stream));
+  if (phi)
+    NLM_HIP(c, hipMemcpyAsync(phi, dp, sizeof(float) * n,
+                              hipMemcpyDeviceToHost, c->stream));
+  if (energy)
+    NLM_HIP(c, hipMemcpyAsync(energy, de, sizeof(double) * n,
+                              hipMemcpyDeviceToHost, c->stream));
   NLM_HIP(c, hipStreamSynchronize(c->stream));
-  for (int64_t a = 0; a < s.n; a++) {
-    const int64_t i = s.perm_host[a];
-    if (Z) Z[i] = hz[a];
-    if (phi) phi[i] = hp[a];
-    if (energy) energy[i] = he[a];
-  }
   return NLM_OK;
 }
 

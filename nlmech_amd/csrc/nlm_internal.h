@@ -221,6 +221,8 @@ struct FdState {
   hipGraphExec_t graph = nullptr;
   int graph_chunk = 0;
   int graph_cur = -1;  // value of cur when the graph was captured
+  DevBuf out;    // device staging of the calls that return node fields, in
+                 // reference order; grows to the largest call
   DevBuf bctab;  // BcTable
   BcTable bc_host{};
   std::vector<uint8_t> fix_host;
@@ -357,6 +359,11 @@ inline int alloc(nlm_ctx* c, DevBuf& b, size_t bytes) {
   }
   b.bytes = bytes;
   return NLM_OK;
+}
+
+// A workspace of at least `bytes` (kept when it is large enough).
+inline int reserve(nlm_ctx* c, DevBuf& b, size_t bytes) {
+  return b.p && b.bytes >= bytes ? NLM_OK : alloc(c, b, bytes);
 }
 
 // Grid helper: ceil-divide and pad to a multiple of 8 for the XCD remap.

@@ -287,9 +287,8 @@ class GpuFD:
 
     def get_state(self):
         n = self.p.n
-        u = np.zeros((n, 3))
-        v = np.zeros((n, 3))
-        f = np.zeros((n, 3))
+        # (the call writes every entry)
+        u, v, f = (np.empty((n, 3)) for _ in range(3))
         self._call("nlm_fd_get_state", ptr(u, C.c_double), ptr(v, C.c_double),
                    ptr(f, C.c_double))
         return u, v, f
@@ -450,8 +449,8 @@ class GpuFD:
 
     def node_fields(self):
         """State-based material: (dilatation, weighted volume) per node."""
-        th = np.zeros(self.p.n)
-        mw = np.zeros(self.p.n)
+        th = np.empty(self.p.n)
+        mw = np.empty(self.p.n)
         self._call("nlm_fd_get_node_fields", ptr(th, C.c_double),
                    ptr(mw, C.c_double))
         return th, mw
@@ -473,9 +472,9 @@ class GpuFD:
 
     def postproc(self):
         n = self.p.n
-        Z = np.zeros(n, np.float32)
-        phi = np.zeros(n, np.float32)
-        e = np.zeros(n)
+        Z = np.empty(n, np.float32)
+        phi = np.empty(n, np.float32)
+        e = np.empty(n)
         self._call("nlm_fd_postproc", ptr(Z, C.c_float), ptr(phi, C.c_float),
                    ptr(e, C.c_double))
         return Z, phi, e
