@@ -84,75 +84,6 @@ __device__ __forceinline__ double es_dil_exact(const EsDev& m,
   return c3 * lx * ext * c * volj;
 }
 
-// Pass 1, FP64: same decision, cancellation-free extension.  exn: the
-// decision lies in a guard band and must be redone by es_dil_exact.
-template <int DIM>
-__device__ __forceinline__ double es_dil_fp64(const EsDev& m, const double* xi,
-                                              const double* ui,
-                                              const double* xj,
-                                              const double* uj, double volj,
-                                              double c3, bool fs0, bool& fs,
-                                              bool& exn) {
-  double dx0 = xj[0] - xi[0], dx1 = xj[1] - xi[1];
-  double dx2 = DIM == 3 ? xj[2] - xi[2] : 0.;
-  double du0 = uj[0] - ui[0], du1 = uj[1] - ui[1];
-  double du2 = DIM == 3 ? uj[2] - ui[2] : 0.;
-  double dd = __builtin_fma(dx1, dx1, dx0 * dx0);
-  double g = __builtin_fma(du1, __builtin_fma(2., dx1, du1),
-                           du0 * __builtin_fma(2., dx0, du0));
-  if (DIM == 3) {
-    dd = __builtin_fma(dx2, dx2, dd);
-    g = __builtin_fma(du2, __builtin_fma(2., dx2, du2), g);
-  }
-  double rx = rsqrt_f64(dd);
-  double lx = dd * rx;
-  double yy = dd + g;
-  double ly = yy * rsqrt_f64(yy);
-  double ext = g / (ly + lx);
-  double s = ext * rx;
-  bool bex = m.breaking && !fs0 &&
-             fabs(s - m.sc_break) <= kEsGuard64 * m.sc_break;
-  fs = fs0 || (m.breaking && s > m.sc_break);
-  bool vex = fabs(lx - m.low_band) <= kEsGuard64 * m.low_band;
-  exn = bex || vex;
-  double c = lx > m.low_band ? (m.check_up - lx) * m.rcp_h : 1.;
-  return c3 * lx * ext * c * volj;
-}
-
-// Pass 1, FP32F.
-template <int DIM>
-__device__ __forceinline__ double es_dil_fp32(const EsDev& m, const double* xi,
-                                              const double* ui,
-                                              const double* xj,
-                                              const double* uj, double volj,
-                                              float c3, bool fs0, bool& fs,
-                                              bool& exn) {
-  float dx0 = float(xj[0] - xi[0]), dx1 = float(xj[1] - xi[1]);
-  float dx2 = DIM == 3 ? float(xj[2] - xi[2]) : 0.f;
-  float du0 = float(uj[0] - ui[0]), du1 = float(uj[1] - ui[1]);
-  float du2 = DIM == 3 ? float(uj[2] - ui[2]) : 0.f;
-  float dd = __builtin_fmaf(dx1, dx1, dx0 * dx0);
-  float g = __builtin_fmaf(du1, __builtin_fmaf(2.f, dx1, du1),
-                           du0 * __builtin_fmaf(2.f, dx0, du0));
-  if (DIM == 3) {
-    dd = __builtin_fmaf(dx2, dx2, dd);
-    g = __builtin_fmaf(du2, __builtin_fmaf(2.f, dx2, du2), g);
-  }
-  float rx = __builtin_amdgcn_rsqf(dd);
-  float lx = dd * rx;
-  float yy = dd + g;
-  float ly = yy * __builtin_amdgcn_rsqf(yy);
-  float ext = g * __builtin_amdgcn_rcpf(ly + lx);
-  float s = ext * rx;
-  bool bex = m.breaking && !fs0 &&
-             fabsf(s - m.sc_break_f) <= kEsGuard32 * m.sc_break_f;
-  fs = fs0 || (m.breaking && s > m.sc_break_f);
-  bool vex = fabsf(lx - m.low_band_f) <= 3e-5f * m.low_band_f;
-  exn = bex || vex;
-  float c = fminf((m.check_up_f - lx) * m.rcp_h_f, 1.0f);
-  return double(c3 * lx * ext * c * float(volj));
-}
-
 // Pass 2, EXACT: V_j T_ij and V_j T_ji of getBondEF for the two directions
 // of one bond, given the per-node coefficients (3D: P = (9/m) K; 2D: P = C,
 // Q = alpha_d) and dilatations of both ends.

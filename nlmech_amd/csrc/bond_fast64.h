@@ -122,6 +122,14 @@ __device__ __forceinline__ double quot(double a, double b, double y) {
   return __builtin_fma(__builtin_fma(-b, q, a), y, q);
 }
 
+// a / b to about an ulp (b well inside the exponent range).
+__device__ __forceinline__ double quot_near(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
 // Influence function as the exact mode evaluates it (r / horizon rounded
 // like the IEEE quotient).
 template <int INF>

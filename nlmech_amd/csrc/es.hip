@@ -29,105 +29,12 @@
 #include <vector>
 
 #include "bond_es.h"
+#include "es_staged.h"
 #include "fd_common.h"
 #include "nlm_internal.h"
 
 namespace nlm {
 namespace {
-
-template <int DIM>
-struct EsArgs {
-  FdArgs<DIM> f;
-  const double* __restrict__ mw;
-  double* __restrict__ theta;
-  double* __restrict__ P;
-  double* __restrict__ Q;
-  EsDev m;
-};
-
-// One halo node staged in LDS by the tiled passes (3D): reference position,
-// displacement, volume and the force coefficient (pass 2) in one 64-byte
-// record.
-struct alignas(16) EsRec {
-  double x0, x1, x2;
-  double u0, u1, u2;
-  double vol, P;
-};
-
-// Stages the halo of layout block lb (every node its four slices reference)
-// in LDS; WITH_P also copies the force coefficient of pass 1.
-template <bool WITH_P>
-__device__ __forceinline__ void es_stage_halo(const FdArgs<3>& a,
-                                              const double* __restrict__ P,
-                                              int64_t lb, EsRec* smem) {
-  const int64_t hb = a.halo_ptr[lb];
-  const int hn = int(a.halo_ptr[lb + 1] - hb);
-  for (int t = threadIdx.x; t < hn; t += int(blockDim.x)) {
-    const uint32_t g = uint32_t(a.halo[hb + t]);
-    const double4 xx = ld32(a.x, g);
-    const double4 uu = ld32(a.u, g);
-    EsRec r;
-    r.x0 = xx.x;
-    r.x1 = xx.y;
-    r.x2 = xx.z;
-    r.u0 = uu.x;
-    r.u1 = uu.y;
-    r.u2 = uu.z;
-    r.vol = ld32(a.vol, g);
-    r.P = WITH_P ? ld32(P, g) : 0.;
-    smem[t] = r;
-  }
-  __syncthreads();
-}
-
-__device__ __forceinline__ const EsRec& es_rec(const EsRec* smem, uint32_t j) {
-  return *reinterpret_cast<const EsRec*>(reinterpret_cast<const char*>(smem) +
-                                         j * uint32_t(sizeof(EsRec)));
-}
-
-// The fast passes stage the halo as two arrays: FP64 position and
-// displacement (48 bytes a node) and the volume and force coefficient (in
-// FP32 in the FP32-force mode, which rounds both anyway).  The 12-dword
-// stride of the first spreads a wavefront's reads over four times as many
-// LDS bank groups as a 16-dword record, at no more LDS.
-struct alignas(16) EsXU {
-  double x[3];
-  double u[3];
-};
-template <class R>
-struct EsVP {
-  R vol;
-  R P;
-};
-template <int MODE>
-using EsVPOf =
-    EsVP<typename std::conditional<MODE == kModeFp32, float, double>::type>;
-
-template <bool WITH_P, class VP>
-__device__ __forceinline__ void es_stage_halo_split(
-    const FdArgs<3>& a, const double* __restrict__ P, int64_t lb, EsXU* xu,
-    VP* vp) {
-  const int64_t hb = a.halo_ptr[lb];
-  const int hn = int(a.halo_ptr[lb + 1] - hb);
-  for (int t = threadIdx.x; t < hn; t += int(blockDim.x)) {
-    const uint32_t g = uint32_t(a.halo[hb + t]);
-    const double4 xx = ld32(a.x, g);
-    const double4 uu = ld32(a.u, g);
-    EsXU r;
-    r.x[0] = xx.x;
-    r.x[1] = xx.y;
-    r.x[2] = xx.z;
-    r.u[0] = uu.x;
-    r.u[1] = uu.y;
-    r.u[2] = uu.z;
-    xu[t] = r;
-    VP q;
-    q.vol = decltype(q.vol)(ld32(a.vol, g));
-    q.P = WITH_P ? decltype(q.P)(ld32(P, g)) : decltype(q.P)(0);
-    vp[t] = q;
-  }
-  __syncthreads();
-}
 
 // The FP32-force passes stage each halo node as its displacement in FP64
 // (24 bytes) and its position as a fixed-point offset from the block's
@@ -210,41 +117,41 @@ __global__ __launch_bounds__(256) void k_es_mw(FdArgs<DIM> a,
 template <int DIM, int MODE, int U, bool TILED>
 __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_dil(
     EsArgs<DIM> e, const unsigned long long* __restrict__ bits_ro) {
-  static_assert(!TILED || DIM == 3, "the LDS-staged passes are 3D");
+  static_assert(!TILED || (DIM == 3 && MODE == kModeFp32),
+                "the staged form is 3D FP32-force (others: k_es_dil_st)");
   const FdArgs<DIM>& a = e.f;
   // staged passes: the workgroup's nodes (its size: 128, 256 or 512, the
   // tuned tile) are one block of the layout's halos
-  const int bn = TILED ? int(blockDim.x) : 256;
+  const int bn = TILED ? a.tile : 256;
   const int64_t nblk = (a.nslices * 64 + bn - 1) / bn;
   const int64_t lb = xcd_block(nblk);
   if (lb >= nblk) return;
-  extern __shared__ EsRec es_smem[];
-  // fast staged passes: split arrays (FP64 mode: FP64 x, u; volume.
-  // FP32-force mode: FP64 u; FP32 block-relative x and volume)
-  constexpr bool R32 = TILED && MODE == kModeFp32;
-  constexpr bool SPLIT = TILED && MODE == kModeFp64;
-  typedef EsVPOf<MODE> VP;
-  EsXU* const es_xu = reinterpret_cast<EsXU*>(es_smem);
-  VP* const es_vp = reinterpret_cast<VP*>(es_xu + a.halo_cap);
+  extern __shared__ double es_smem[];
+  constexpr bool R32 = TILED;
   EsU64* const es_u64 = reinterpret_cast<EsU64*>(es_smem);
   EsXV32* const es_xv = reinterpret_cast<EsXV32*>(es_u64 + a.halo_cap);
   double4 org = make_double4(0., 0., 0., 0.);
   if constexpr (R32) {
     org = reinterpret_cast<const double4*>(a.blk_org)[lb];
     es_stage_halo_r32<false>(a, e.P, lb, org, e.m, es_u64, es_xv, nullptr);
-  } else if constexpr (SPLIT) {
-    es_stage_halo_split<false>(a, e.P, lb, es_xu, es_vp);
-  } else if constexpr (TILED) {
-    es_stage_halo<false>(a, e.P, lb, es_smem);
   }
-  const int lane = threadIdx.x & 63;
-  const int64_t s =
-      lb * (bn >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (s >= a.nslices) return;  // whole wavefront
+  // staged: `parts` wavefronts share a slice (split_rows.h), their FP64 sums
+  // added in the order of the parts
+  SplitPos sp;
+  sp.lane = threadIdx.x & 63;
+  sp.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  sp.nsl = bn >> 6;
+  sp.parts = TILED ? a.parts : 1;
+  sp.sl = TILED ? sp.wave % sp.nsl : sp.wave;
+  sp.part = TILED ? sp.wave / sp.nsl : 0;
+  const int lane = sp.lane;
+  const int64_t s = lb * sp.nsl + sp.sl;
+  const bool slice_ok = s < a.nslices;
+  if (!TILED && !slice_ok) return;  // whole wavefront
   const int64_t i = s * 64 + lane;
-  const bool valid = i < a.n;
-  const int64_t cb = a.sl_ptr[s];
-  const int width = int((a.sl_ptr[s + 1] - cb) >> 6);
+  const bool valid = slice_ok && i < a.n;
+  const int64_t cb = slice_ok ? a.sl_ptr[s] : 0;
+  const int width = slice_ok ? int((a.sl_ptr[s + 1] - cb) >> 6) : 0;
   const int64_t bb = cb >> 6;
   const int len = valid ? int(a.rowlen[i]) : 0;
   double xi[3] = {0., 0., 0.}, ui[3] = {0., 0., 0.};
@@ -285,13 +192,14 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_dil(
   const double sc3 = R32 ? c3 * e.m.q * e.m.q : c3;
   uint32_t jn[U];
 #pragma unroll
-  for (int q = 0; q < U; ++q) jn[q] = slot_index(q);
-  for (int k0 = 0; k0 < width; k0 += U) {
+  for (int q = 0; q < U; ++q) jn[q] = slot_index(U * sp.part + q);
+  const int stride = U * sp.parts;
+  for (int k0 = U * sp.part; k0 < width; k0 += stride) {
     uint32_t jc[U];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       jc[q] = jn[q];
-      jn[q] = slot_index(k0 + U + q);
+      jn[q] = slot_index(k0 + stride + q);
     }
     double xj[U][3], uj[U][3], vj[U];
     float dxf[U][3], duf[U][3];
@@ -306,22 +214,6 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_dil(
           duf[q][d] = float(ru.u[d] - uqi[d]);
         }
         vj[q] = double(rx.vol);
-      } else if constexpr (SPLIT) {
-        const EsXU& r = es_xu[jc[q]];
-        for (int d = 0; d < 3; d++) {
-          xj[q][d] = r.x[d];
-          uj[q][d] = r.u[d];
-        }
-        vj[q] = double(es_vp[jc[q]].vol);
-      } else if constexpr (TILED) {
-        const EsRec& r = es_rec(es_smem, jc[q]);
-        xj[q][0] = r.x0;
-        xj[q][1] = r.x1;
-        xj[q][2] = r.x2;
-        uj[q][0] = r.u0;
-        uj[q][1] = r.u1;
-        uj[q][2] = r.u2;
-        vj[q] = r.vol;
       } else {
         load3<DIM>(ld32(a.x, jc[q]), xj[q]);
         load3<DIM>(ld32(a.u, jc[q]), uj[q]);
@@ -470,25 +362,8 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_dil(
       const bool act = k0 + q < len;
       const bool fs0 = __builtin_amdgcn_inverse_ballot_w64(w[q]);
       bool fs = fs0;
-      double d;
-      if constexpr (MODE == kModeExact) {
-        d = es_dil_exact(e.m, xi, ui, xj[q], uj[q], vj[q], c3, fs);
-      } else {
-        bool exn;
-        if constexpr (MODE == kModeFp64)
-          d = es_dil_fp64<DIM>(e.m, xi, ui, xj[q], uj[q], vj[q], c3, fs0, fs,
-                               exn);
-        else
-          d = es_dil_fp32<DIM>(e.m, xi, ui, xj[q], uj[q], vj[q], c3f, fs0,
-                               fs, exn);
-        exn = exn && act;
-        if (__ballot(exn) != 0ull) {
-          if (exn) {
-            fs = fs0;
-            d = es_dil_exact(e.m, xi, ui, xj[q], uj[q], vj[q], c3, fs);
-          }
-        }
-      }
+      const double d =
+          es_dil_exact(e.m, xi, ui, xj[q], uj[q], vj[q], c3, fs);
       if (act && !fs) th += d;
       const bool newly = act && fs && !fs0;
       if (k0 + q < width) {
@@ -497,25 +372,17 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_dil(
       }
     }
   }
+  if constexpr (TILED) {
+    if (sp.parts > 1) {
+      double t1[1] = {thf};
+      split_parts<1>(reinterpret_cast<double*>(es_xv + a.halo_cap), sp, t1);
+      thf = t1[0];
+    }
+    if (sp.part != 0) return;
+  }
   th += sc3 * thf;
   if (!valid) return;
-  e.theta[i] = th;
-  if constexpr (DIM == 3) {
-    // EXACT keeps alpha_s = (9/m) K (ElasticState.cpp:230-233); the fast
-    // modes fold t_ij = alpha_s theta_i |X| / 3 into P_i |X|.
-    e.P[i] = MODE == kModeExact ? (9. / mwi) * e.m.K : 3. * e.m.K * th / mwi;
-  } else if (e.m.one_d) {
-    // 1D: t_ij = (E/m_i) e_ij (ElasticState.cpp:187-193)
-    e.P[i] = 0.;
-    e.Q[i] = e.m.E / mwi;
-  } else {
-    const double as = (9. / mwi) * e.m.Kc;
-    const double ad = (8. / mwi) * e.m.mu;
-    const double C = 2. * e.m.f2d * as - (3. - 2. * e.m.f2d) * ad;
-    // fast modes: t_ij = theta_i (C/9 - alpha_d/3) |X| + alpha_d e_ij
-    e.P[i] = MODE == kModeExact ? C : th * (C / 9. - ad / 3.);
-    e.Q[i] = ad;
-  }
+  es_coefficients<DIM, MODE>(e, i, th, mwi);
 }
 
 // Pass 2: bond forces of both directions gathered at node i, force BCs,
@@ -528,22 +395,15 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_force(
     t_force = e.f.tdev[0];
     t_next = e.f.tdev[1];
   }
-  static_assert(!TILED || (DIM == 3 && MODE != kModeExact),
-                "the LDS-staged force pass is 3D, fast modes");
+  static_assert(!TILED || (DIM == 3 && MODE == kModeFp32),
+                "the staged form is 3D FP32-force (others: k_es_force_st)");
   const FdArgs<DIM>& a = e.f;
-  const int bn = TILED ? int(blockDim.x) : 256;
+  const int bn = TILED ? a.tile : 256;
   const int64_t nblk = (a.nslices * 64 + bn - 1) / bn;
   const int64_t lb = xcd_block(nblk);
   if (lb >= nblk) return;
-  extern __shared__ EsRec es_smem[];
-  // fast staged passes: split arrays (FP64 mode: FP64 x, u; volume and
-  // force coefficient.  FP32-force mode: FP64 u; FP32 block-relative x and
-  // volume; FP32 force coefficient)
-  constexpr bool R32 = TILED && MODE == kModeFp32;
-  constexpr bool SPLIT = TILED && MODE == kModeFp64;
-  typedef EsVPOf<MODE> VP;
-  EsXU* const es_xu = reinterpret_cast<EsXU*>(es_smem);
-  VP* const es_vp = reinterpret_cast<VP*>(es_xu + a.halo_cap);
+  extern __shared__ double es_smem[];
+  constexpr bool R32 = TILED;
   EsU64* const es_u64 = reinterpret_cast<EsU64*>(es_smem);
   EsXV32* const es_xv = reinterpret_cast<EsXV32*>(es_u64 + a.halo_cap);
   float* const es_p32 = reinterpret_cast<float*>(es_xv + a.halo_cap);
@@ -551,19 +411,24 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_force(
   if constexpr (R32) {
     org = reinterpret_cast<const double4*>(a.blk_org)[lb];
     es_stage_halo_r32<true>(a, e.P, lb, org, e.m, es_u64, es_xv, es_p32);
-  } else if constexpr (SPLIT) {
-    es_stage_halo_split<true>(a, e.P, lb, es_xu, es_vp);
-  } else if constexpr (TILED) {
-    es_stage_halo<true>(a, e.P, lb, es_smem);
   }
-  const int lane = threadIdx.x & 63;
-  const int64_t s =
-      lb * (bn >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (s >= a.nslices) return;
+  // staged: `parts` wavefronts share a slice (split_rows.h), their FP64 sums
+  // added in the order of the parts
+  SplitPos sp;
+  sp.lane = threadIdx.x & 63;
+  sp.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  sp.nsl = bn >> 6;
+  sp.parts = TILED ? a.parts : 1;
+  sp.sl = TILED ? sp.wave % sp.nsl : sp.wave;
+  sp.part = TILED ? sp.wave / sp.nsl : 0;
+  const int lane = sp.lane;
+  const int64_t s = lb * sp.nsl + sp.sl;
+  const bool slice_ok = s < a.nslices;
+  if (!TILED && !slice_ok) return;  // whole wavefront
   const int64_t i = s * 64 + lane;
-  const bool valid = i < a.n;
-  const int64_t cb = a.sl_ptr[s];
-  const int width = int((a.sl_ptr[s + 1] - cb) >> 6);
+  const bool valid = slice_ok && i < a.n;
+  const int64_t cb = slice_ok ? a.sl_ptr[s] : 0;
+  const int width = slice_ok ? int((a.sl_ptr[s + 1] - cb) >> 6) : 0;
   const int64_t bb = cb >> 6;
   const int len = valid ? int(a.rowlen[i]) : 0;
   constexpr bool kExact = MODE == kModeExact;
@@ -604,13 +469,14 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_force(
   double acc[3] = {0., 0., 0.}, oth[3] = {0., 0., 0.};
   uint32_t jn[U];
 #pragma unroll
-  for (int q = 0; q < U; ++q) jn[q] = slot_index(q);
-  for (int k0 = 0; k0 < width; k0 += U) {
+  for (int q = 0; q < U; ++q) jn[q] = slot_index(U * sp.part + q);
+  const int stride = U * sp.parts;
+  for (int k0 = U * sp.part; k0 < width; k0 += stride) {
     uint32_t jc[U];
 #pragma unroll
     for (int q = 0; q < U; ++q) {
       jc[q] = jn[q];
-      jn[q] = slot_index(k0 + U + q);
+      jn[q] = slot_index(k0 + stride + q);
     }
     double xj[U][3], uj[U][3], vj[U], Pj[U], Qj[U], thj[U];
     float dxf[U][3], duf[U][3];
@@ -627,29 +493,6 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_force(
         }
         vj[q] = double(rx.vol);
         Pj[q] = double(es_p32[j]);
-        Qj[q] = 0.;
-        thj[q] = 0.;
-      } else if constexpr (SPLIT) {
-        const EsXU& r = es_xu[j];
-        for (int d = 0; d < 3; d++) {
-          xj[q][d] = r.x[d];
-          uj[q][d] = r.u[d];
-        }
-        const VP vpj = es_vp[j];
-        vj[q] = double(vpj.vol);
-        Pj[q] = double(vpj.P);
-        Qj[q] = 0.;
-        thj[q] = 0.;
-      } else if constexpr (TILED) {
-        const EsRec& r = es_rec(es_smem, j);
-        xj[q][0] = r.x0;
-        xj[q][1] = r.x1;
-        xj[q][2] = r.x2;
-        uj[q][0] = r.u0;
-        uj[q][1] = r.u1;
-        uj[q][2] = r.u2;
-        vj[q] = r.vol;
-        Pj[q] = r.P;
         Qj[q] = 0.;
         thj[q] = 0.;
       } else {
@@ -783,6 +626,11 @@ __global__ __launch_bounds__(TILED ? 512 : 256) void k_es_force(
         for (int d = 0; d < DIM; d++) acc[d] += double(pf[mm][d]);
     }
   }
+  if constexpr (TILED) {
+    if (sp.parts > 1)
+      split_parts<3>(reinterpret_cast<double*>(es_p32 + a.halo_cap), sp, acc);
+    if (sp.part != 0) return;
+  }
   if (!valid) return;
   double f[3] = {0., 0., 0.};
   if (BASE_F) {
@@ -806,34 +654,54 @@ EsArgs<DIM> make_es_args(nlm_ctx* c) {
   e.P = s.es_P.as<double>();
   e.Q = s.es_Q.as<double>();
   e.m = s.es;
+  e.stride = 0;
   return e;
 }
 
-// LDS bytes of a tiled launch: one record per halo entry (the fast passes:
-// the two split arrays; the exact pass 1 keeps one record).
+// Halo record sizes that decide whether a tile's halo fits the LDS: the 3D
+// FP32-force passes' arrays, 64 bytes in the FP64 modes (a pass of theirs
+// whose own records need more takes the direct gathers).
 size_t es_record_bytes(int precision) {
-  const size_t fast = precision == kModeFp32
-                          ? sizeof(EsU64) + sizeof(EsXV32) + sizeof(float)
-                          : sizeof(EsXU) + sizeof(EsVPOf<kModeFp64>);
-  return precision == kModeExact ? sizeof(EsRec) : fast;
+  return precision == kModeFp32
+             ? sizeof(EsU64) + sizeof(EsXV32) + sizeof(float)
+             : 64;
 }
 size_t es_lds_bytes(const FdState& s) {
   return size_t(s.halo_max + 1) * es_record_bytes(s.precision);
 }
+// LDS bytes of a 3D FP32-force pass: its arrays (halo_cap entries, even) and
+// the parts' sums.
+size_t es_lds32(const FdState& s, bool force) {
+  return size_t((s.halo_max + 1) & ~int64_t(1)) *
+             (sizeof(EsU64) + sizeof(EsXV32) + (force ? sizeof(float) : 0)) +
+         split_parts_bytes(s.tile, s.parts, force ? 3 : 1);
+}
+
+// Whether a pass runs as k_es_dil_st / k_es_force_st: every staged model but
+// the 3D FP32-force ones, where the pass's records fit the LDS.
+bool st_pass(const nlm_ctx* c, const FdState& s, bool force) {
+  return s.es_tiled && s.use_tiled &&
+         !(s.dim == 3 && s.precision == kModeFp32) &&
+         es_st_lds(s.dim, s.precision, s.halo_max, s.tile, s.parts, force,
+                   size_t(s.es_lds_max))
+                 .bytes <= size_t(s.es_lds_max);
+}
 
 template <int DIM, int MODE>
 void launch_dil(nlm_ctx* c, const EsArgs<DIM>& e) {
+  if (st_pass(c, c->fd, false)) return es_st_dil<DIM>(c, e);
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
-  if constexpr (DIM == 3) {
+  if constexpr (DIM == 3 && MODE == kModeFp32) {
     if (c->fd.es_tiled && c->fd.use_tiled) {
       // one workgroup per tile of the layout's halos
       const int bn = c->fd.tile;
       const unsigned gt = grid_xcd(c->fd.sell.nslices * 64, bn);
-      const size_t lds = es_lds_bytes(c->fd);
+      const size_t lds = es_lds32(c->fd, false);
       allow_lds(reinterpret_cast<const void*>(k_es_dil<DIM, MODE, 4, true>),
                 lds);
-      hipLaunchKernelGGL((k_es_dil<DIM, MODE, 4, true>), dim3(gt), dim3(bn),
-                         lds, c->stream, e, e.f.bits);
+      hipLaunchKernelGGL((k_es_dil<DIM, MODE, 4, true>), dim3(gt),
+                         dim3(unsigned(bn * c->fd.parts)), lds, c->stream, e,
+                         e.f.bits);
       return;
     }
   }
@@ -843,18 +711,23 @@ void launch_dil(nlm_ctx* c, const EsArgs<DIM>& e) {
 
 template <int DIM, int MODE, int KIND, bool BASE_F, int U>
 void launch_force_k(nlm_ctx* c, const EsArgs<DIM>& e, double tf, double tn) {
+  if (st_pass(c, c->fd, true)) {
+    EsArgs<DIM> b = e;
+    b.f.kind = KIND == KIND_CD ? KIND_CD : BASE_F ? KIND_FORCE_ADD : KIND_FORCE;
+    return es_st_force<DIM>(c, b, tf, tn);
+  }
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
-  if constexpr (DIM == 3 && MODE != kModeExact) {
+  if constexpr (DIM == 3 && MODE == kModeFp32) {
     if (c->fd.es_tiled && c->fd.use_tiled) {
       const int bn = c->fd.tile;
       const unsigned gt = grid_xcd(c->fd.sell.nslices * 64, bn);
-      const size_t lds = es_lds_bytes(c->fd);
+      const size_t lds = es_lds32(c->fd, true);
       allow_lds(reinterpret_cast<const void*>(
                     k_es_force<DIM, MODE, KIND, BASE_F, U, true>),
                 lds);
       hipLaunchKernelGGL((k_es_force<DIM, MODE, KIND, BASE_F, U, true>),
-                         dim3(gt), dim3(bn), lds, c->stream, e, e.f.bits, tf,
-                         tn);
+                         dim3(gt), dim3(unsigned(bn * c->fd.parts)), lds,
+                         c->stream, e, e.f.bits, tf, tn);
       return;
     }
   }
@@ -939,13 +812,13 @@ int es_prepare(nlm_ctx* c) {
   NLM_HIP(c, hipMemsetAsync(s.es_theta.p, 0, nb, c->stream));
   NLM_HIP(c, hipMemsetAsync(s.es_P.p, 0, nb, c->stream));
   NLM_HIP(c, hipMemsetAsync(s.es_Q.p, 0, nb, c->stream));
-  // LDS-staged passes: 3D, when one block's halo fits the device's LDS
+  // LDS-staged passes, when one block's halo fits the device's LDS
   int lds_max = 0;
   NLM_HIP(c, hipDeviceGetAttribute(&lds_max,
                                    hipDeviceAttributeMaxSharedMemoryPerBlock,
                                    c->device));
-  s.es_tiled = s.dim == 3 && s.halo_max > 0 &&
-               es_lds_bytes(s) <= size_t(lds_max);
+  s.es_lds_max = lds_max;
+  s.es_tiled = s.halo_max > 0 && es_lds_bytes(s) <= size_t(lds_max);
   const unsigned g = unsigned((s.n + 255) / 256);
   if (s.dim == 2)
     hipLaunchKernelGGL(k_es_mw<2>, dim3(g), dim3(256), 0, c->stream,

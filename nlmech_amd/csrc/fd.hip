@@ -1276,6 +1276,36 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
   return {256, 1};
 }
 
+// The same for the state-based passes.  Microseconds per step (both passes)
+// at the lines, and of the passes before (2D: direct gathers, 3D: 256-node
+// tiles, whole rows):
+//   2D exact / FP64 / FP32-force, 100 x 100 nodes (157 slices): 64 x 8 12.3 /
+//     11.3 / 10.4, before 28.1 / 19.1 / 16.3; 301 x 257 (1209): 64 x 4 23.3 /
+//     20.1 / 15.2, 256 x 1 28.6 / 23.9 / 19.8, before 40.0 / 26.9 / 23.0;
+//     600 x 500 (4688): 256 x 1 58.2 / 47.9 / 35.5, 64 x 4 65.3 / 54.8 /
+//     38.8, before 84.8 / 57.6 / 46.5;
+//   3D exact / FP64 / FP32-force, 20 x 18 x 22 (124): 64 x 8 25.6 / 20.3 /
+//     15.9, before 92 / 51 / 43; 47 x 39 x 33 (945): 256 x 1 65.3 / 53.2 /
+//     46.7, 128 x 4 72.5 / 47.9 / 30.9, before 96.4 / 56.3 / 46.0; 80 x 80 x
+//     80 (8000): 256 x 1 317 / 241 / 166, 128 x 4 465 / 261 / 154, 256 x 2
+//     499 / 338 / 140, before 523 / 269 / 166.
+StageRule es_stage_rule(int dim, int precision, int64_t nslices) {
+  const bool f32 = precision == NLM_PREC_FP32_FORCE;
+  if (nslices <= 400) return {64, 8};
+  if (dim == 2) {
+    if (nslices <= 2500) return {64, 4};
+    return f32 ? StageRule{128, 2} : StageRule{256, 1};
+  }
+  if (f32) return nslices <= 2500 ? StageRule{128, 4} : StageRule{256, 2};
+  if (precision == NLM_PREC_FP64 && nslices <= 2500) return {128, 4};
+  return {256, 1};
+}
+// Parts at a tile set by hand: at most 512 threads a workgroup.
+int es_stage_parts(int dim, int precision, int64_t nslices, int tile) {
+  const StageRule r = es_stage_rule(dim, precision, nslices);
+  return std::max(1, std::min(r.parts, 512 / tile));
+}
+
 // Parts at a tile other than the rule's own (a tile set by hand, or one that
 // fits the LDS): at most 512 threads a workgroup; in the FP64 modes tiles of
 // 256 nodes and more keep whole rows (their rounds over four slices cost
@@ -1384,6 +1414,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   const size_t rec = halo_rec_bytes(dim, p->precision, has_nofail);
   StageRule rule{256, 1};
   if (!es_mat) rule = stage_rule(dim, p->precision, (n + 63) / 64);
+  else rule = es_stage_rule(dim, p->precision, (n + 63) / 64);
   int tile = rule.tile;
   build_layout(dim, n, p->x, mesh_h, h_row, h_col, tile / 64, L);
   bool fits = (L.halo_max + 1) * int64_t(bond3 ? rec : kHaloRecBudget) <=
@@ -1425,7 +1456,8 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   if ((rc = up(s.halo, L.halo.data(), sizeof(int32_t) * L.halo.size()))) return rc;
   s.halo_max = L.halo_max;
   s.tile = tile;
-  s.parts = es_mat ? 1 : stage_parts(dim, p->precision, L.nslices, tile);
+  s.parts = es_mat ? rule.parts
+                   : stage_parts(dim, p->precision, L.nslices, tile);
   // the staged bond-based kernels
   s.tiled = !es_mat && L.halo_max > 0 && fits;
   // k_fd_st's arithmetic takes beta > 0 and lengths far inside the exponent
@@ -1451,6 +1483,12 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     const std::vector<uint16_t> colL_off = staged_entries(
         L.colL, rec, L.sl_ptr.data(), L.nslices, L.rowlen.data(), n);
     if ((rc = up(s.colL, colL_off.data(), sizeof(uint16_t) * nent))) return rc;
+  } else if (es_mat && (dim == 2 || p->precision != NLM_PREC_FP32_FORCE)) {
+    // (k_es_dil_st, k_es_force_st: record indices, 0 the record of padded
+    // slots)
+    const std::vector<uint16_t> idx = staged_entries(
+        L.colL, 1, L.sl_ptr.data(), L.nslices, L.rowlen.data(), n);
+    if ((rc = up(s.colL, idx.data(), sizeof(uint16_t) * nent))) return rc;
   } else if ((rc = up(s.colL, L.colL.data(), sizeof(uint16_t) * nent))) {
     return rc;
   }
@@ -2435,11 +2473,17 @@ int retile(nlm_ctx* c, int bn) {
     NLM_HIP(c, hipDeviceGetAttribute(&lds_max,
                                      hipDeviceAttributeMaxSharedMemoryPerBlock,
                                      c->device));
-    if (hmax > 65535 ||
+    if (hmax > 65534 ||
         es_halo_lds_bytes(s.precision, hmax) > size_t(lds_max))
       return fail(c, NLM_ERR_INVALID,
                   "tile of " + std::to_string(bn) +
                       " nodes: its largest halo exceeds the LDS budget");
+    if (s.precision != NLM_PREC_FP32_FORCE) {
+      std::vector<uint16_t> rl(static_cast<size_t>(n));
+      NLM_HIP(c, hipMemcpy(rl.data(), s.sell.rowlen.p, sizeof(uint16_t) * n,
+                           hipMemcpyDeviceToHost));
+      colL = staged_entries(colL, 1, slp.data(), ns, rl.data(), n);
+    }
   }
   // origins: the centre of each block's bounding box
   const int dim = s.dim == 3 ? 3 : 2;
@@ -2489,7 +2533,8 @@ int retile(nlm_ctx* c, int bn) {
     return rc;
   s.halo_max = hmax;
   s.tile = bn;
-  if (!es) s.parts = stage_parts(s.dim, s.precision, ns, bn);
+  s.parts = es ? es_stage_parts(s.dim, s.precision, ns, bn)
+               : stage_parts(s.dim, s.precision, ns, bn);
   if (es) es_set_quantum(s.es, org_range);
   return NLM_OK;
 }

@@ -215,6 +215,7 @@ struct FdState {
   int64_t halo_max = 0;
   bool tiled = false;   // LDS-staged step kernel usable
   bool es_tiled = false;  // LDS-staged state-based passes usable
+  int es_lds_max = 0;     // the device's LDS per workgroup
   bool use_tiled = true;
   DevBuf node_rate;  // double[3n] internal order: node-list BC rates
   DevBuf tdev;       // (t_force, t_next) read by graph-captured steps
