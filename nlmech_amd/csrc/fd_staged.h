@@ -15,11 +15,9 @@
 // Split rows.  One wavefront per 64-node slice leaves a small model a few
 // wavefronts per CU that walk their rows serially (100 x 100 nodes: 157
 // slices on 1024 SIMDs), and the 3D halos leave a CU two tiles.  With SPLIT,
-// `parts` wavefronts share a slice: part p takes the slot chunks p, p +
-// parts, ...  In the FP64 modes the summands pass through LDS in rounds of
-// parts x U slots and are added in list order, so their bits depend
-// on neither the split nor the tile; the FP32-force mode adds the parts' FP64
-// sums at the end in the order of the parts.
+// `parts` wavefronts share a slice (split_rows.h): in the FP64 modes with the
+// sums of one wavefront walking the row, so their bits depend on neither the
+// split nor the tile.
 //
 // Launch kinds (a.kind, wavefront-uniform): force, force added to f, the
 // fused central-difference step and the fused velocity-Verlet step.
@@ -34,6 +32,7 @@
 #include "device_common.h"
 #include "fd_common.h"
 #include "nlm_internal.h"
+#include "split_rows.h"
 
 namespace nlm {
 
@@ -389,61 +388,15 @@ __global__ __launch_bounds__(512) void k_fd_st(
       }
     }
   };
-  double acc[3] = {0., 0., 0.};
+  double acc[DIM] = {};
+  double* const buf = reinterpret_cast<double*>(
+      reinterpret_cast<char*>(st_smem) + a.halo_bytes);
+  const SplitPos sp{sl, part, parts, nsl, wave, lane};
   if constexpr (SPLIT && !F32) {
-    // rounds of parts x U slots: the summands (exact mode: forces, FP64 mode:
-    // pair sums) through LDS, added in list order by the wavefront of the
-    // (slice, component) task
-    double* const buf = reinterpret_cast<double*>(
-        reinterpret_cast<char*>(st_smem) + a.halo_bytes);
-    const int nv = NF * parts;  // summands of a lane's component in a round
-    int wmax = 0;
-    for (int q = 0; q < nsl; q++) {
-      const int64_t t = lb * nsl + q;
-      if (t < a.nslices)
-        wmax = max(wmax, int((a.sl_ptr[t + 1] - a.sl_ptr[t]) >> 6));
-    }
-    const int nw = nsl * parts;
-    const int ntask = nsl * DIM;
-    constexpr int MT = 2;  // tasks a wavefront (parts >= 2, DIM <= 3)
-    double sum[MT] = {0., 0.};
-    int tw[MT];
-#pragma unroll
-    for (int t = 0; t < MT; t++) {
-      const int task = wave + t * nw;
-      const int64_t ts = lb * nsl + task / DIM;
-      tw[t] = task < ntask && ts < a.nslices
-                  ? int((a.sl_ptr[ts + 1] - a.sl_ptr[ts]) >> 6)
-                  : 0;
-    }
-    for (int base = 0; base < wmax; base += stride, k0 += stride) {
-      if (k0 < width) {
-        double F[NF][DIM];
-        chunk(k0, k0 + stride, F);
-#pragma unroll
-        for (int m = 0; m < NF; ++m)
-          for (int d = 0; d < DIM; d++)
-            buf[((sl * DIM + d) * nv + part * NF + m) * 64 + lane] = F[m][d];
-      }
-      __syncthreads();
-      // (slots past a row are exact zeros; chunks past a slice were not
-      // written)
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        const int cnt = min(nv, (tw[t] - base + U - 1) / U * NF);
-        const double* const v = buf + (wave + t * nw) * nv * 64 + lane;
-        for (int m = 0; m < cnt; m++) sum[t] += v[m * 64];
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int t = 0; t < MT; t++) {
-      const int task = wave + t * nw;
-      if (task < ntask) buf[task * 64 + lane] = sum[t];
-    }
-    __syncthreads();
-    if (part == 0)
-      for (int d = 0; d < DIM; d++) acc[d] = buf[(sl * DIM + d) * 64 + lane];
+    const int64_t s0 = lb * nsl;
+    split_ordered<DIM, NF, U>(chunk, buf, sp, a.sl_ptr + s0,
+                              int(min(int64_t(nsl), a.nslices - s0)), width,
+                              acc);
   } else {
     for (; k0 < width; k0 += stride) {
       Real F[NF][DIM];
@@ -452,32 +405,19 @@ __global__ __launch_bounds__(512) void k_fd_st(
       for (int m = 0; m < NF; ++m)
         for (int d = 0; d < DIM; d++) acc[d] += double(F[m][d]);
     }
-    if constexpr (SPLIT) {
-      // the parts' sums, added in the order of the parts
-      double* const buf = reinterpret_cast<double*>(
-          reinterpret_cast<char*>(st_smem) + a.halo_bytes);
-      if (part > 0)
-        for (int d = 0; d < DIM; d++)
-          buf[((sl * (parts - 1) + part - 1) * DIM + d) * 64 + lane] = acc[d];
-      __syncthreads();
-      if (part == 0)
-        for (int p = 0; p < parts - 1; p++)
-          for (int d = 0; d < DIM; d++)
-            acc[d] += buf[((sl * (parts - 1) + p) * DIM + d) * 64 + lane];
-    }
+    if constexpr (SPLIT) split_parts<DIM>(buf, sp, acc);
   }
   if (!valid || part != 0) return;
   if constexpr (!SPLIT) load3<DIM>(a.v[i], vi);
   st_tail<DIM>(a, i, fl, xi, ui, vi, acc, t_force, t_next);
 }
 
-// LDS bytes behind the halo records of a split launch: the FP64 modes' round
-// buffer, the FP32-force mode's sums.
+// LDS bytes behind the halo records of a split launch.
 inline size_t st_round_bytes(int dim, int precision, int tile, int parts) {
-  const size_t per = precision == kModeExact  ? size_t(kStSplitU * parts)
-                     : precision == kModeFp64 ? size_t(kStSplitU / 2 * parts)
-                                              : size_t(parts - 1);
-  return size_t(tile / 64) * dim * per * 64 * 8;
+  if (precision == kModeFp32) return split_parts_bytes(tile, parts, dim);
+  return split_ordered_bytes(tile, parts, dim,
+                             precision == kModeExact ? kStSplitU
+                                                     : kStSplitU / 2);
 }
 
 // Bytes of a halo record.
