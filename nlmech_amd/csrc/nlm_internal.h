@@ -218,7 +218,7 @@ struct FdState {
   int es_lds_max = 0;     // the device's LDS per workgroup
   bool use_tiled = true;
   DevBuf node_rate;  // double[3n] internal order: node-list BC rates
-  DevBuf tdev;       // (t_force, t_next) read by graph-captured steps
+  DevBuf tdev;       // times of the graph-captured steps
   hipGraphExec_t graph = nullptr;
   int graph_chunk = 0;
   int graph_cur = -1;  // value of cur when the graph was captured
