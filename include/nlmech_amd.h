@@ -394,7 +394,10 @@ const char* nlm_fd_kernel_name(nlm_ctx* ctx);
  * = 0 on the free dofs (QuasiStaticModel::solver, QuasiStaticModel.cpp:
  * 527-592; computeResidual :597-646).  The tangent is the analytic derivative
  * of the bond force (on the neighbor sparsity, 2x2 blocks); each Newton
- * system is solved by BiCGSTAB to a relative residual. */
+ * system is solved to a relative residual by conjugate gradients in the
+ * volume-weighted inner product (the analytic tangent with precond NONE or
+ * JACOBI, where it is self-adjoint) or by BiCGSTAB (every other case, and
+ * where conjugate gradients break down or reach the iteration limit). */
 #define NLM_QS_TANGENT_FULL 0      /* exact derivative, all 2x2 entries */
 #define NLM_QS_TANGENT_COMPONENT 1 /* same-component entries only, the
                                       entries the reference's central-
@@ -426,7 +429,7 @@ typedef struct {
   int max_newton;     /* SolverDeck Max_Iteration */
   int tangent;        /* NLM_QS_TANGENT_* */
   int precond;        /* NLM_QS_PRECOND_* */
-  double lin_tol;     /* BiCGSTAB: ||r|| <= lin_tol ||b|| */
+  double lin_tol;     /* Krylov solve: ||r|| <= lin_tol ||b|| */
   int lin_max_iter;
   int predictor;      /* 1: linearized first iteration with the prescribed
                          increment as Dirichlet data (no force evaluation at
@@ -448,7 +451,7 @@ typedef struct {
   double residual;       /* ||R||_2 after the last load step */
   double residual0;      /* ||R_0|| of the last load step */
   double ms_total;
-  double ms_linear;      /* BiCGSTAB iterations */
+  double ms_linear;      /* Krylov iterations */
   double ms_precond;     /* preconditioner construction (incl. network) */
   double ms_tangent;     /* tangent assembly */
 } nlm_qs_stats;
@@ -471,13 +474,13 @@ int nlm_qs_get_precond(nlm_ctx* ctx, double* blocks, double* diag);
 /* z = R A_c^-1 R^T r: the coarse correction of the two-level preconditioner
  * on the assembled tangent (r, z AoS double[3n]). */
 int nlm_qs_coarse_apply(nlm_ctx* ctx, const double* r, double* z);
-/* BiCGSTAB launch mode (no counterpart in the reference): on (default),
+/* Krylov launch mode (no counterpart in the reference): on (default),
  * each batch of 8 iterations is one replay of a captured HIP graph; off,
  * the same kernels are launched one by one.  Results are identical.  The
  * environment variable NLM_QS_GRAPH=0 makes off the default of new
  * contexts. */
 int nlm_qs_set_graph(nlm_ctx* ctx, int on);
-/* BiCGSTAB configuration (no counterpart in the reference): graph as
+/* Krylov configuration (no counterpart in the reference): graph as
  * nlm_qs_set_graph; bond_scalar (default on): the products with the
  * analytic bond tangent (NLM_QS_TANGENT_FULL / _COMPONENT) read one scalar
  * per bond, g with -B_ij = g dx dx^T (dx the reference bond vector), and

@@ -9,8 +9,10 @@
 // difference Jacobian that keeps only same-component entries (:363-454);
 // NLM_QS_TANGENT_COMPONENT keeps the same entries of the exact derivative.
 //
-// Krylov solve.  BiCGSTAB on A_ff (prescribed dofs held at zero in every
-// vector, their rows masked in every product).  The scalars live on the
+// Krylov solve.  Conjugate gradients in the volume-weighted inner product for
+// the analytic tangent with point Jacobi or none, BiCGSTAB otherwise, on A_ff
+// (prescribed dofs held at zero in every vector, their rows masked in every
+// product).  The scalars live on the
 // device: each kernel that needs a dot product reduces the 256-node blocks'
 // partial sums itself (every workgroup in the same order, so all agree), and
 // workgroup 0 records the scalar for later kernels.  Convergence sets a flag
@@ -915,6 +917,204 @@ __global__ __launch_bounds__(256) void k_bicg_x(VecArgs a, int k) {
   block_partials<2>(v, P, blockIdx.x);
 }
 
+// Conjugate gradients ---------------------------------------------------------
+// The analytic bond tangent times the nodes' volumes is symmetric (A_ij holds
+// V_j, the bond's other factors belong to the pair), so A_ff is self-adjoint
+// in the inner product <x, y> = sum_i V_i x_i.y_i and, away from softening,
+// positive; so is point Jacobi.  Conjugate gradients in that product take one
+// product with the tangent an iteration and two launches, BiCGSTAB two and
+// five.  A solve that breaks down or does not converge within the iteration
+// limit is done again by BiCGSTAB.
+//
+// Iteration it: k_cg_mv forms p = z + beta p (into the other p buffer) and q =
+// A z + beta A p with partial <p, q>; k_cg_x takes alpha, x += alpha p, r -=
+// alpha q, z = M r with partials <r, z>, (r, r).  Buffers of VecArgs: p and s
+// the two p's, v = q, ph = z.  Both kernels are chains of memory latencies on
+// small models (about 5 us each at 1e4 nodes): the row's loads wait neither
+// for the partials nor for the iteration's number.  Point Jacobi, 1e-8, two
+// load steps, BiCGSTAB before: 100 x 100 nodes 1180 x 9.9 us (837 x 19.2), 200
+// x 200 2323 x 12.4 (1780 x 22.5), 300 x 300 3484 x 20.2 (2717 x 34.6).
+
+// z = M r: point Jacobi (PRE 1) or r (PRE 0).
+template <int PRE>
+__device__ __forceinline__ double2 cg_z(const VecArgs& a, int64_t i,
+                                        double2 r) {
+  if (PRE == 0) return r;
+  const double2 di = a.dinv[i];
+  return make_double2(di.x * r.x, di.y * r.y);
+}
+
+template <int PRE>
+__global__ __launch_bounds__(256) void k_cg_init(VecArgs a, QsArgs q,
+                                                 const double2* __restrict__ b) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  double v[2] = {0., 0.};
+  if (i < a.n) {
+    double2 r = b[i];
+    const uint32_t fl = a.flags[i];
+    if (dof_fixed(fl, 0)) r.x = 0.;
+    if (dof_fixed(fl, 1)) r.y = 0.;
+    const double2 z = cg_z<PRE>(a, i, r), o = make_double2(0., 0.);
+    a.r[i] = r;
+    a.ph[i] = z;
+    a.p[i] = o;
+    a.s[i] = o;
+    a.x[i] = o;
+    v[0] = q.vol[i] * (r.x * z.x + r.y * z.y);
+    v[1] = r.x * r.x + r.y * r.y;
+  }
+  double* const P[2] = {a.P0, a.P1};
+  block_partials<2>(v, P, blockIdx.x);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    a.ctl[0] = 0;
+    a.ctl[1] = 0;
+    a.ctl[2] = 1;
+  }
+}
+
+// BS: the tangent's form (k_qs_spmv4).  One workgroup per slice, wavefront w
+// taking slots w, w + 4, ...
+template <int BS>
+__global__ __launch_bounds__(256) void k_cg_mv(
+    VecArgs a, QsArgs q, const double4* __restrict__ blk,
+    const double4* __restrict__ dg, const double* __restrict__ bg, int k) {
+  const int done = a.ctl[0];
+  const int it = a.ctl[2] + k;
+  const double rho2[2] = {a.sc.rho_p(0), a.sc.rho_p(1)};
+  const int64_t s = xcd_block(q.nslices);
+  if (s >= q.nslices) return;
+  const int lane = threadIdx.x & 63;
+  const int wq = threadIdx.x >> 6;
+  const int64_t i = s * 64 + lane;
+  const bool valid = i < a.n;
+  const int64_t cb = q.sl_ptr[s];
+  const int width = int((q.sl_ptr[s + 1] - cb) >> 6);
+  const double2 none = make_double2(0., 0.);
+  const double2 xi = valid ? q.x[i] : none;
+  // the partials' loads first; beta is their ratio, so the products of z and
+  // of the old p are formed apart (A z + beta A p) and the row's loads wait
+  // for nothing
+  double red[2] = {0., 0.};
+  for (int64_t t = threadIdx.x; t < a.nb; t += 256) {
+    red[0] += a.P0[t];
+    red[1] += a.P1[t];
+  }
+  // (kBicgBatch is even: the parity of it is that of k + 1)
+  const double2* const po = k & 1 ? a.p : a.s;
+  double2* const pn = k & 1 ? a.s : a.p;
+  double2 az = none, ap = none;
+  auto slot = [&](int64_t e) {
+    const int32_t j = q.col[e];
+    const double2 z = a.ph[j], p = po[j];
+    if (BS == 0) {
+      const double4 B = blk[e];
+      az.x += B.x * z.x + B.y * z.y;
+      az.y += B.z * z.x + B.w * z.y;
+      ap.x += B.x * p.x + B.y * p.y;
+      ap.y += B.z * p.x + B.w * p.y;
+    } else {
+      const double2 xj = q.x[j];
+      const double g = bg[e], d0 = xj.x - xi.x, d1 = xj.y - xi.y;
+      if (BS == 1) {
+        const double wz = g * (d0 * z.x + d1 * z.y);
+        const double wp = g * (d0 * p.x + d1 * p.y);
+        az.x += wz * d0;
+        az.y += wz * d1;
+        ap.x += wp * d0;
+        ap.y += wp * d1;
+      } else {
+        az.x += g * d0 * d0 * z.x;
+        az.y += g * d1 * d1 * z.y;
+        ap.x += g * d0 * d0 * p.x;
+        ap.y += g * d1 * d1 * p.y;
+      }
+    }
+  };
+#pragma unroll 4
+  for (int kk = wq; kk < width; kk += 4) slot(cb + int64_t(kk) * 64 + lane);
+  block_reduce<2>(red);
+  if (done || it > a.max_it) return;
+  const double rho = red[0], rr = red[1];
+  const bool conv = !(rr > a.sc.tol2());
+  const bool brk = !conv && !(rho > 0.);
+  if (s == 0 && threadIdx.x == 0) {
+    a.sc.rho_p((it - 1) & 1) = rho;
+    a.sc.rr(it - 1) = rr;
+    if (conv || brk) {
+      a.ctl[0] = conv ? 1 : 2;
+      a.ctl[1] = it - 1;
+    }
+  }
+  if (conv || brk) return;
+  const double beta = it > 1 ? rho / rho2[it & 1] : 0.;
+  double2 acc = make_double2(az.x + beta * ap.x, az.y + beta * ap.y);
+  __shared__ double2 part[3][64];
+  if (wq > 0) part[wq - 1][lane] = acc;
+  __syncthreads();
+  if (wq != 0) return;
+  acc.x += part[0][lane].x + part[1][lane].x + part[2][lane].x;
+  acc.y += part[0][lane].y + part[1][lane].y + part[2][lane].y;
+  double pq = 0.;
+  if (valid) {
+    const double2 z = a.ph[i], p = po[i];
+    const double2 pi =
+        make_double2(z.x + beta * p.x, z.y + beta * p.y);
+    const double4 D = dg[i];
+    acc.x += D.x * pi.x + D.y * pi.y;
+    acc.y += D.z * pi.x + D.w * pi.y;
+    const uint32_t fl = a.flags[i];
+    if (dof_fixed(fl, 0)) acc.x = 0.;
+    if (dof_fixed(fl, 1)) acc.y = 0.;
+    pn[i] = pi;
+    a.v[i] = acc;
+    pq = q.vol[i] * (pi.x * acc.x + pi.y * acc.y);
+  }
+  for (int off = 32; off > 0; off >>= 1) pq += __shfl_xor(pq, off);
+  if (lane == 0) a.P2[s] = pq;
+}
+
+template <int PRE>
+__global__ __launch_bounds__(256) void k_cg_x(VecArgs a, QsArgs q, int k) {
+  const int done = a.ctl[0];
+  const int it = a.ctl[2] + k;
+  const double rho1[2] = {a.sc.rho_p(0), a.sc.rho_p(1)};
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const bool own = i < a.n;
+  const double2 none = make_double2(0., 0.);
+  const double2* const pn = k & 1 ? a.s : a.p;
+  const double2 p = own ? pn[i] : none, v = own ? a.v[i] : none,
+                x = own ? a.x[i] : none, r0 = own ? a.r[i] : none;
+  const double vol = own ? q.vol[i] : 0.;
+  double pq[1];
+  {
+    const double* const P[1] = {a.P2};
+    block_sums<1>(P, a.nbs, pq);
+  }
+  if (done || it > a.max_it) return;
+  const bool brk = !(pq[0] > 0.);
+  if (brk) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      a.ctl[0] = 2;
+      a.ctl[1] = it - 1;
+    }
+    return;
+  }
+  const double alpha = rho1[(it - 1) & 1] / pq[0];
+  double w[2] = {0., 0.};
+  if (own) {
+    a.x[i] = make_double2(x.x + alpha * p.x, x.y + alpha * p.y);
+    const double2 r =
+        make_double2(r0.x - alpha * v.x, r0.y - alpha * v.y);
+    const double2 z = cg_z<PRE>(a, i, r);
+    a.r[i] = r;
+    a.ph[i] = z;
+    w[0] = vol * (r.x * z.x + r.y * z.y);
+    w[1] = r.x * r.x + r.y * r.y;
+  }
+  double* const P[2] = {a.P0, a.P1};
+  block_partials<2>(w, P, blockIdx.x);
+}
+
 // Newton helpers ------------------------------------------------------------
 
 // R = f on free dofs (f = f_int + b), 0 on prescribed; partial (R, R).
@@ -1128,13 +1328,16 @@ VecArgs vec_args(nlm_ctx* c) {
   return a;
 }
 
-// BiCGSTAB iterations per host check (and per graph replay).
-constexpr int kBicgBatch = 8;
+// Krylov iterations per host check (and per graph replay).
+constexpr int kBicgBatch = 8;  // (even: k_cg_mv)
+static_assert(kBicgBatch % 2 == 0, "p buffers by the parity of k");
 
 // Everything a captured BiCGSTAB batch depends on.
 struct BicgKey {
   VecArgs a;
   QsArgs qa;
+  int method;  // 0: BiCGSTAB, 1: conjugate gradients
+  int form;    // the tangent's form (k_qs_spmv4's BS)
   int precond;
   int coarse;
   int m;
@@ -1425,6 +1628,102 @@ int coarse_setup(nlm_ctx* c) {
   return NLM_OK;
 }
 
+// The squared norm of the masked right-hand side (its partials in P1) and the
+// convergence bound for the device.
+int start_solve(nlm_ctx* c, const VecArgs& a, double tol, double* bb) {
+  if (int rc = partial_sum(c, a.P1, bb)) return rc;
+  const double tol2 = tol * tol * *bb;
+  NLM_HIP(c, hipMemcpyAsync(c->qs.scal.p, &tol2, sizeof(double),
+                            hipMemcpyHostToDevice, c->stream));
+  NLM_HIP(c, hipStreamSynchronize(c->stream));
+  return NLM_OK;
+}
+
+// Runs batches of kBicgBatch iterations (launch_batch, replayed from a
+// captured graph when the context says so) until the device reports the end
+// or a.max_it is reached.
+template <class Launch>
+int run_batches(nlm_ctx* c, const VecArgs& a, BicgKey& key,
+                const Launch& launch_batch, double bb, int* iters,
+                double* relres, bool* ok) {
+  QsState& q = c->qs;
+  const int max_iter = a.max_it, batch = kBicgBatch;
+  int rc;
+  int ctl[2] = {0, 0};
+  hipGraphExec_t exec = nullptr;
+  if (q.use_graph) {
+    // the captured batch depends on every kernel argument: recapture when
+    // any of them changed since the last capture
+    std::memcpy(&key.a, &a, sizeof(a));
+    const QsArgs qa = qs_args(c);
+    std::memcpy(&key.qa, &qa, sizeof(qa));
+    key.form = q.bond_scalar ? q.bs_mode : 0;
+    key.blk = q.blk.p;
+    key.diag = q.diag.p;
+    key.g = node_grid(c->fd);
+    const unsigned char* kb = reinterpret_cast<const unsigned char*>(&key);
+    if (!q.bicg_graph || q.bicg_key.size() != sizeof(key) ||
+        std::memcmp(kb, q.bicg_key.data(), sizeof(key)) != 0) {
+      if (q.bicg_graph) (void)hipGraphExecDestroy(q.bicg_graph);
+      q.bicg_graph = nullptr;
+      hipGraph_t gr = nullptr;
+      NLM_HIP(c, hipStreamBeginCapture(c->stream,
+                                       hipStreamCaptureModeThreadLocal));
+      launch_batch();
+      NLM_HIP(c, hipStreamEndCapture(c->stream, &gr));
+      hipError_t e = hipGraphInstantiate(&q.bicg_graph, gr, nullptr, nullptr,
+                                         0);
+      (void)hipGraphDestroy(gr);
+      if (e != hipSuccess) {
+        q.bicg_graph = nullptr;
+        return fail(c, NLM_ERR_HIP, "Krylov solve: graph instantiation failed");
+      }
+      q.bicg_key.assign(kb, kb + sizeof(key));
+    }
+    exec = q.bicg_graph;
+  }
+  // One batch stays queued ahead of the host's check of the previous one,
+  // so the device does not idle through the round trip; a batch queued
+  // after the finish (convergence, breakdown or the iteration cap) runs as
+  // no-ops.  Each batch's control words land in their own pinned slot.
+  const int nbatch = (max_iter + batch - 1) / batch;
+  hipEvent_t ev[2] = {q.e0, q.e1};
+  auto queue = [&](int b) -> int {
+    if (exec)
+      NLM_HIP(c, hipGraphLaunch(exec, c->stream));
+    else
+      launch_batch();
+    NLM_HIP(c, hipGetLastError());
+    NLM_HIP(c, hipMemcpyAsync(q.hctl + 2 * (b & 1), q.ctl.p, 2 * sizeof(int),
+                              hipMemcpyDeviceToHost, c->stream));
+    NLM_HIP(c, hipEventRecord(ev[b & 1], c->stream));
+    return NLM_OK;
+  };
+  if ((rc = queue(0))) return rc;
+  for (int b = 0; b < nbatch; b++) {
+    if (b + 1 < nbatch && (rc = queue(b + 1))) return rc;
+    NLM_HIP(c, hipEventSynchronize(ev[b & 1]));
+    ctl[0] = q.hctl[2 * (b & 1)];
+    ctl[1] = q.hctl[2 * (b & 1) + 1];
+    if (ctl[0]) break;
+  }
+  NLM_HIP(c, hipStreamSynchronize(c->stream));
+  double rr = 0.;
+  int done_it = max_iter;
+  if (ctl[0]) {
+    done_it = ctl[1];
+    const size_t off = 8 + 3 * size_t(q.max_iter_alloc) + size_t(done_it);
+    NLM_HIP(c, hipMemcpy(&rr, q.scal.as<double>() + off, sizeof(double),
+                         hipMemcpyDeviceToHost));
+  } else {
+    if ((rc = partial_sum(c, a.P1, &rr))) return rc;
+  }
+  *iters = done_it;
+  *relres = std::sqrt(rr / bb);
+  *ok = ctl[0] == 1;
+  return NLM_OK;
+}
+
 // BiCGSTAB on A_ff x = b (q.b -> q.x).  Returns iterations, relative
 // residual and whether it converged.
 int bicgstab(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
@@ -1449,11 +1748,7 @@ int bicgstab(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
                      q.b.as<double2>());
   NLM_HIP(c, hipGetLastError());
   double bb = 0.;
-  if ((rc = partial_sum(c, a.P1, &bb))) return rc;
-  const double tol2 = tol * tol * bb;
-  NLM_HIP(c, hipMemcpyAsync(q.scal.p, &tol2, sizeof(double),
-                            hipMemcpyHostToDevice, c->stream));
-  NLM_HIP(c, hipStreamSynchronize(c->stream));
+  if ((rc = start_solve(c, a, tol, &bb))) return rc;
   if (bb == 0.) {
     *iters = 0;
     *relres = 0.;
@@ -1462,7 +1757,6 @@ int bicgstab(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
   }
   const double2* rh = q.rh.as<double2>();
   a.max_it = max_iter;
-  int ctl[2] = {0, 0};
   const int batch = kBicgBatch;
   // one batch: iterations ctl[2] .. ctl[2] + batch - 1 (no-ops past
   // max_iter or after convergence), then the batch start moves on
@@ -1516,88 +1810,94 @@ int bicgstab(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
     hipLaunchKernelGGL(k_iter_advance, dim3(1), dim3(64), 0, c->stream, a.ctl,
                        batch);
   };
-  hipGraphExec_t exec = nullptr;
-  if (q.use_graph) {
-    // the captured batch depends on every kernel argument: recapture when
-    // any of them changed since the last capture
-    BicgKey key;
-    std::memset(&key, 0, sizeof(key));
-    std::memcpy(&key.a, &a, sizeof(a));
-    const QsArgs qa = qs_args(c);
-    std::memcpy(&key.qa, &qa, sizeof(qa));
-    key.precond = precond;
-    key.coarse = coarse;
-    key.m = q.m;
-    key.cinv = q.cinv;
-    key.blk = q.blk.p;
-    key.diag = q.diag.p;
-    key.mblk = q.mhalf.p;
-    key.mdiag = q.mdiag.p;
-    key.zcp = q.zcp.p;
-    key.zcs = q.zcs.p;
-    key.g = g;
-    key.gmv = gmv;
-    const unsigned char* kb = reinterpret_cast<const unsigned char*>(&key);
-    if (!q.bicg_graph || q.bicg_key.size() != sizeof(key) ||
-        std::memcmp(kb, q.bicg_key.data(), sizeof(key)) != 0) {
-      if (q.bicg_graph) (void)hipGraphExecDestroy(q.bicg_graph);
-      q.bicg_graph = nullptr;
-      hipGraph_t gr = nullptr;
-      NLM_HIP(c, hipStreamBeginCapture(c->stream,
-                                       hipStreamCaptureModeThreadLocal));
-      launch_batch();
-      NLM_HIP(c, hipStreamEndCapture(c->stream, &gr));
-      hipError_t e = hipGraphInstantiate(&q.bicg_graph, gr, nullptr, nullptr,
-                                         0);
-      (void)hipGraphDestroy(gr);
-      if (e != hipSuccess) {
-        q.bicg_graph = nullptr;
-        return fail(c, NLM_ERR_HIP, "BiCGSTAB: graph instantiation failed");
-      }
-      q.bicg_key.assign(kb, kb + sizeof(key));
-    }
-    exec = q.bicg_graph;
-  }
-  // One batch stays queued ahead of the host's check of the previous one,
-  // so the device does not idle through the round trip; a batch queued
-  // after the finish (convergence, breakdown or the iteration cap) runs as
-  // no-ops.  Each batch's control words land in their own pinned slot.
-  const int nbatch = (max_iter + batch - 1) / batch;
-  hipEvent_t ev[2] = {q.e0, q.e1};
-  auto queue = [&](int b) -> int {
-    if (exec)
-      NLM_HIP(c, hipGraphLaunch(exec, c->stream));
-    else
-      launch_batch();
-    NLM_HIP(c, hipGetLastError());
-    NLM_HIP(c, hipMemcpyAsync(q.hctl + 2 * (b & 1), q.ctl.p, 2 * sizeof(int),
-                              hipMemcpyDeviceToHost, c->stream));
-    NLM_HIP(c, hipEventRecord(ev[b & 1], c->stream));
+  BicgKey key;
+  std::memset(&key, 0, sizeof(key));
+  key.precond = precond;
+  key.coarse = coarse;
+  key.m = q.m;
+  key.cinv = q.cinv;
+  key.mblk = q.mhalf.p;
+  key.mdiag = q.mdiag.p;
+  key.zcp = q.zcp.p;
+  key.zcs = q.zcs.p;
+  key.gmv = gmv;
+  return run_batches(c, a, key, launch_batch, bb, iters, relres, ok);
+}
+
+// Conjugate gradients on A_ff x = b (q.b -> q.x) in the volume-weighted inner
+// product, for the analytic tangent with point Jacobi or none.
+int conjugate_gradients(nlm_ctx* c, int precond, double tol, int max_iter,
+                        int* iters, double* relres, bool* ok) {
+  FdState& s = c->fd;
+  QsState& q = c->qs;
+  int rc;
+  if ((rc = qs_alloc(c, max_iter))) return rc;
+  VecArgs a = vec_args(c);
+  a.max_it = max_iter;
+  const QsArgs qa = qs_args(c);
+  const unsigned g = node_grid(s);
+  const unsigned gsl = unsigned((s.sell.nslices + 7) / 8 * 8);
+  const bool jacobi = precond == NLM_QS_PRECOND_JACOBI;
+  if (jacobi)
+    hipLaunchKernelGGL(k_cg_init<1>, dim3(g), dim3(256), 0, c->stream, a, qa,
+                       q.b.as<double2>());
+  else
+    hipLaunchKernelGGL(k_cg_init<0>, dim3(g), dim3(256), 0, c->stream, a, qa,
+                       q.b.as<double2>());
+  NLM_HIP(c, hipGetLastError());
+  double bb = 0.;
+  if ((rc = start_solve(c, a, tol, &bb))) return rc;
+  if (bb == 0.) {
+    *iters = 0;
+    *relres = 0.;
+    *ok = true;
     return NLM_OK;
+  }
+  const int bs = q.bond_scalar ? q.bs_mode : 0;
+  const double4* blk = q.blk.as<double4>();
+  const double4* dg = q.diag.as<double4>();
+  const double* bg = q.bg.as<double>();
+  auto launch_batch = [&]() {
+    for (int k = 0; k < kBicgBatch; k++) {
+      if (bs == 1)
+        hipLaunchKernelGGL(k_cg_mv<1>, dim3(gsl), dim3(256), 0, c->stream, a,
+                           qa, blk, dg, bg, k);
+      else if (bs == 2)
+        hipLaunchKernelGGL(k_cg_mv<2>, dim3(gsl), dim3(256), 0, c->stream, a,
+                           qa, blk, dg, bg, k);
+      else
+        hipLaunchKernelGGL(k_cg_mv<0>, dim3(gsl), dim3(256), 0, c->stream, a,
+                           qa, blk, dg, bg, k);
+      if (jacobi)
+        hipLaunchKernelGGL(k_cg_x<1>, dim3(g), dim3(256), 0, c->stream, a, qa,
+                           k);
+      else
+        hipLaunchKernelGGL(k_cg_x<0>, dim3(g), dim3(256), 0, c->stream, a, qa,
+                           k);
+    }
+    hipLaunchKernelGGL(k_iter_advance, dim3(1), dim3(64), 0, c->stream, a.ctl,
+                       kBicgBatch);
   };
-  if ((rc = queue(0))) return rc;
-  for (int b = 0; b < nbatch; b++) {
-    if (b + 1 < nbatch && (rc = queue(b + 1))) return rc;
-    NLM_HIP(c, hipEventSynchronize(ev[b & 1]));
-    ctl[0] = q.hctl[2 * (b & 1)];
-    ctl[1] = q.hctl[2 * (b & 1) + 1];
-    if (ctl[0]) break;
+  BicgKey key;
+  std::memset(&key, 0, sizeof(key));
+  key.method = 1;
+  key.precond = precond;
+  return run_batches(c, a, key, launch_batch, bb, iters, relres, ok);
+}
+
+// Solves A_ff x = b (q.b -> q.x): conjugate gradients where the tangent and
+// the preconditioner are self-adjoint (the analytic tangent; none or point
+// Jacobi), BiCGSTAB otherwise and where conjugate gradients end without
+// convergence.
+int linear_solve(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
+                 double* relres, bool* ok) {
+  if ((precond == NLM_QS_PRECOND_NONE || precond == NLM_QS_PRECOND_JACOBI) &&
+      c->qs.tangent != NLM_QS_TANGENT_FD) {
+    const int rc =
+        conjugate_gradients(c, precond, tol, max_iter, iters, relres, ok);
+    if (rc || *ok) return rc;
   }
-  NLM_HIP(c, hipStreamSynchronize(c->stream));
-  double rr = 0.;
-  int done_it = max_iter;
-  if (ctl[0]) {
-    done_it = ctl[1];
-    const size_t off = 8 + 3 * size_t(q.max_iter_alloc) + size_t(done_it);
-    NLM_HIP(c, hipMemcpy(&rr, q.scal.as<double>() + off, sizeof(double),
-                         hipMemcpyDeviceToHost));
-  } else {
-    if ((rc = partial_sum(c, a.P1, &rr))) return rc;
-  }
-  *iters = done_it;
-  *relres = std::sqrt(rr / bb);
-  *ok = ctl[0] == 1;
-  return NLM_OK;
+  return bicgstab(c, precond, tol, max_iter, iters, relres, ok);
 }
 
 // ||R||_2 of the residual of the current force (q.b <- R).
@@ -1850,7 +2150,7 @@ extern "C" int nlm_qs_linear_solve(nlm_ctx* c, const double* b, double* x,
   int it = 0;
   double rr = 0.;
   bool ok = false;
-  if ((rc = bicgstab(c, precond, tol, max_iter, &it, &rr, &ok))) return rc;
+  if ((rc = linear_solve(c, precond, tol, max_iter, &it, &rr, &ok))) return rc;
   if (iters) *iters = it;
   if (relres) *relres = rr;
   return dev_to_aos(c, q.x, x);
@@ -1896,7 +2196,7 @@ extern "C" int nlm_qs_solve(nlm_ctx* c, const nlm_qs_options* o,
     int it = 0;
     double rr = 0.;
     bool ok = false;
-    int r = bicgstab(c, o->precond, o->lin_tol, o->lin_max_iter, &it, &rr,
+    int r = linear_solve(c, o->precond, o->lin_tol, o->lin_max_iter, &it, &rr,
                      &ok);
     stats.ms_linear += ms_since(t0);
     stats.linear_iters += it;
