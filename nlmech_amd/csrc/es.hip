@@ -677,6 +677,11 @@ size_t es_lds32(const FdState& s, bool force) {
          split_parts_bytes(s.tile, s.parts, force ? 3 : 1);
 }
 
+bool staged32(const FdState& s, bool force) {
+  return s.es_tiled && s.use_tiled &&
+         es_lds32(s, force) <= size_t(s.es_lds_max);
+}
+
 // Whether a pass runs as k_es_dil_st / k_es_force_st: every staged model but
 // the 3D FP32-force ones, where the pass's records fit the LDS.
 bool st_pass(const nlm_ctx* c, const FdState& s, bool force) {
@@ -692,7 +697,7 @@ void launch_dil(nlm_ctx* c, const EsArgs<DIM>& e) {
   if (st_pass(c, c->fd, false)) return es_st_dil<DIM>(c, e);
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
   if constexpr (DIM == 3 && MODE == kModeFp32) {
-    if (c->fd.es_tiled && c->fd.use_tiled) {
+    if (staged32(c->fd, false)) {
       // one workgroup per tile of the layout's halos
       const int bn = c->fd.tile;
       const unsigned gt = grid_xcd(c->fd.sell.nslices * 64, bn);
@@ -718,7 +723,7 @@ void launch_force_k(nlm_ctx* c, const EsArgs<DIM>& e, double tf, double tn) {
   }
   unsigned g = grid_xcd(force_blocks(c->fd) * 256, 256);
   if constexpr (DIM == 3 && MODE == kModeFp32) {
-    if (c->fd.es_tiled && c->fd.use_tiled) {
+    if (staged32(c->fd, true)) {
       const int bn = c->fd.tile;
       const unsigned gt = grid_xcd(c->fd.sell.nslices * 64, bn);
       const size_t lds = es_lds32(c->fd, true);
