@@ -1097,7 +1097,7 @@ int do_steps(nlm_ctx* c, int nsteps, double* ms_fused) {
   if (ms_fused) NLM_HIP(c, hipEventRecord(s.ev0, c->stream));
   // one launch a step: the force, the end of its step and the start of the
   // next (velocity Verlet, 333 x 217 nodes, FP64: 24.4 us with three launches,
-  // their update kernels 8 us of it)
+  // their update kernels 8 us of it; 15 us now)
   for (int k = 1; k < nsteps; k++) {
     double tn = s.time + s.dt;
     launch_fused_dispatch<DIM>(c, s.time, tn);

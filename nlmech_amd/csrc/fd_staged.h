@@ -9,8 +9,9 @@
 // the common path carries no row-length mask.  The kernel is bound by FP64
 // instructions; bond_fast64.h says what a bond costs.  Per step, before and
 // after that arithmetic (and the records without the row-length mask):
-// 400 x 397 nodes, horizon 4 h, exact mode 57 -> 28 us; 619 x 451 nodes,
-// FP64 mode, four slots a chunk 48 -> 31 us.
+// 400 x 397 nodes, horizon 4 h, exact mode 57 -> 27 us; 619 x 451 nodes,
+// FP64 mode, four slots a chunk 48 -> 32 us; 1000 x 1000, 103 -> 82 us (FP64),
+// 256 -> 119 us (exact).
 //
 // Split rows.  One wavefront per 64-node slice leaves a small model a few
 // wavefronts per CU that walk their rows serially (100 x 100 nodes: 157
