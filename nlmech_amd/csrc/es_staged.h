@@ -5,8 +5,8 @@
 //
 // A workgroup stages its tile's halo in LDS and reads neighbors through
 // 16-bit indices; record 0 is a zero-volume record far from every node that
-// padded slots and fetches past a slice address.  `parts` wavefronts share a
-// slice (split_rows.h): in the FP64 modes with the sums of one wavefront
+// padded slots and fetches past a slice address (their terms are masked by the
+// row's length).  `parts` wavefronts share a slice (split_rows.h): in the FP64 modes with the sums of one wavefront
 // walking the row, so their bits depend on neither the tile nor the split.
 //
 // The exact mode takes its square roots and quotients from one Goldschmidt
@@ -316,9 +316,12 @@ __global__ __launch_bounds__(512) void k_es_dil_st(
       }
       // one vote on the guard band's lower bound: a bond that may break is
       // decided, and its term taken, by the exact evaluation after the chunk
-      band[q] = ~w[q] & v_lo;
-      ex[q] = v_vex | band[q];
-      const unsigned long long keep = ~w[q] & ~ex[q];
+      // (record 0 alone does not make a slot past the row 0: a node without
+      // neighbors has an infinite c3)
+      const unsigned long long act = __builtin_amdgcn_ballot_w64(k0 + q < len);
+      band[q] = act & ~w[q] & v_lo;
+      ex[q] = (act & v_vex) | band[q];
+      const unsigned long long keep = act & ~w[q] & ~ex[q];
       term = __builtin_amdgcn_inverse_ballot_w64(keep) ? term : Real(0);
       if constexpr (EXACT) F[q][0] = term;
       else if (q % 2 == 0) F[q / 2][0] = term;
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(512) void k_es_dil_st(
       for (int q = 0; q < U; ++q) {
         if (ex[q] == 0ull) continue;
         bool fsn = false;
-        if (__builtin_amdgcn_inverse_ballot_w64(ex[q]) && k0 + q < len) {
+        if (__builtin_amdgcn_inverse_ballot_w64(ex[q])) {
           const uint32_t g = uint32_t(a.halo[r.hb + jc[q] - 1]);
           const bool fs0 = __builtin_amdgcn_inverse_ballot_w64(w[q]);
           bool fs = fs0;
@@ -448,7 +451,12 @@ __global__ __launch_bounds__(512) void k_es_force_st(
                      X2 = xs[2] - xi[2];
         return es_corr_exact(e.m, sqrt(X0 * X0 + X1 * X1 + X2 * X2));
       };
-      const bool live = !__builtin_amdgcn_inverse_ballot_w64(w[q]);
+      // Slots past the row are masked: against record 0 the FP32 product
+      // (P_i + P_j) |X| overflows on fine meshes (P goes with h^-4), and a
+      // node without neighbors has P and Q infinite or NaN.  (The mask is one
+      // comparison and one scalar AND a slot.)
+      const unsigned long long act = __builtin_amdgcn_ballot_w64(k0 + q < len);
+      const bool live = __builtin_amdgcn_inverse_ballot_w64(act & ~w[q]);
       if constexpr (EXACT) {
         // es_force_exact's operations in its order
         double Y[DIM], yy = 0., dd = 0.;
