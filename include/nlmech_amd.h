@@ -44,7 +44,12 @@ typedef struct nlm_ctx nlm_ctx;
 /* Precision modes of the bond-force kernels. */
 #define NLM_PREC_FP64_EXACT 0 /* reference operation order, no FMA, IEEE div */
 #define NLM_PREC_FP64 1       /* FP64, break test as the reference, FMA elsewhere */
-#define NLM_PREC_FP32_FORCE 2 /* FP64 state / stretch / break test, FP32 force */
+#define NLM_PREC_FP32_FORCE 2 /* FP64 state, sums and break decisions near the
+                                 critical stretch; a bond's position and
+                                 displacement differences, stretch and force
+                                 in FP32 (staged kernels: positions relative
+                                 to a tile, FP32 in 2D, 32-bit fixed point in
+                                 3D) */
 
 /* Time integrators, inp::ModelDeck::d_timeDiscretization
  * (src/inp/input.cpp:137-147). */

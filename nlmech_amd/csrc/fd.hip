@@ -1518,8 +1518,8 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     for (int d = 0; d < dim; d++) borg[stride * b + d] = 0.5 * (lo[d] + hi[d]);
   }
   // largest offset of a block's node or halo node from the block's origin
-  // (per component): the range of the fixed-point positions of the
-  // state-based FP32-force passes
+  // (per component): the range of the fixed-point positions of the 3D
+  // FP32-force kernels
   double org_range = 0.;
   for (int64_t b = 0; b < L.nblocks; b++) {
     auto span = [&](int64_t a) {
@@ -1651,42 +1651,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
                      ? m.beta * (m.break_lo * m.krbar_sq)
                      : std::numeric_limits<double>::infinity();
   m.vex_tol_f = float(3e-5 * m.low_band);
-  {
-    const double b2 = m.beta * 1.4426950408889634;  // beta log2 e
-    if (b2 > 0.) {  // (beta > 0 for RNP bonds)
-      // 3D: 1/sigma is the quantum of the fixed-point positions, the
-      // smallest with every offset from a tile's origin (at most org_range)
-      // below 2^30 that keeps tau a power of two (between one and four times
-      // org_range / 2^30)
-      const double e = dim == 3
-                           ? std::floor(0.5 * std::log2(b2 * 0x1p+30 /
-                                                        std::max(org_range,
-                                                                 m.h)))
-                           : std::round(0.5 * std::log2(b2));
-      m.tau = std::ldexp(1.0, int(e));
-      m.sigma = m.tau * m.tau / b2;
-      // 3D: sigma moved by up to 2^-25 so that 1/(sigma h), the constant of
-      // the volume correction, is an FP32 number (rounded, it is an error of
-      // every bond at the horizon's edge that does not average out: forces of
-      // the 72 x 64 x 56 block 4.4e-7 off instead of 2.6e-7); the exponent
-      // beta r S^2 takes that relative error instead
-      if (dim == 3) m.sigma = 1.0 / (double(float(1.0 / (m.sigma * m.h))) * m.h);
-    } else {
-      m.tau = m.sigma = 1.0;
-    }
-    const double bl = m.tau * m.tau / m.sigma;  // beta log2 e
-    m.c4_infl_s = m.c4_infl * m.sigma / m.tau;
-    m.c4f_infl_s = float(double(m.c4f_infl) * m.sigma / m.tau);
-    m.rcp_h_s = float(1.0 / (m.sigma * m.h));
-    m.rcp_sigma_f = float(1.0 / m.sigma);
-    m.break_lo_s = m.irreversible ? float(double(m.break_lo_f) * bl)
-                                  : std::numeric_limits<float>::infinity();
-    // r within 3e-5 (relative) of low_band <=> r^2 within about 6e-5 of
-    // low_band^2; the band on r^2 is taken a little wider
-    const double lows = m.sigma * m.low_band;
-    m.low_dd_f = float(lows * lows);
-    m.vex_dd_tol_f = float(6.1e-5 * lows * lows);
-  }
+  double bond_max = 0.;  // largest component of a bond
   {
     // Bonds whose reference length lies within 3e-5 (relative) of the
     // volume-correction edge: a static mask per (slice, slot), padded like
@@ -1708,6 +1673,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
             for (int d = 0; d < dim; d++) {
               const double e = hx[g * stride + d] - hx[a * stride + d];
               d2 += e * e;
+              bond_max = std::max(bond_max, std::fabs(e));
             }
             if (std::fabs(std::sqrt(d2) - m.low_band) <= tol)
               word |= 1ull << lane;
@@ -1719,6 +1685,49 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     if ((rc = up(s.vexw, vw.data(), sizeof(unsigned long long) * vw.size())))
       return rc;
     NLM_HIP(c, hipStreamSynchronize(st));
+  }
+  {
+    const double b2 = m.beta * 1.4426950408889634;  // beta log2 e
+    if (b2 > 0.) {  // (beta > 0 for RNP bonds)
+      // 3D: 1/sigma is the quantum of the fixed-point positions, the
+      // smallest with every component of a bond below 2^31 of them that keeps
+      // tau a power of two (between one and four times bond_max / 2^31)
+      const double e =
+          dim == 3 ? std::floor(0.5 * std::log2(b2 * 0x1.f8p+30 /
+                                                std::max(bond_max, m.h)))
+                   : std::round(0.5 * std::log2(b2));
+      m.tau = std::ldexp(1.0, int(e));
+      m.sigma = m.tau * m.tau / b2;
+      // 3D: sigma moved by up to 2^-25 so that 1/(sigma h), the constant of
+      // the volume correction, is an FP32 number (rounded, it is an error of
+      // every bond at the horizon's edge that does not average out: forces of
+      // the 72 x 64 x 56 block 4.4e-7 off instead of 2.6e-7); the exponent
+      // beta r S^2 takes that relative error instead
+      if (dim == 3) m.sigma = 1.0 / (double(float(1.0 / (m.sigma * m.h))) * m.h);
+      // Direct gathers where the fixed-point positions (even numbers of
+      // quanta) would be coarser than 2^-25 h, about the FP32 rounding of a
+      // bond's length (bonds longer than 7.8 h), and where an offset from a
+      // tile's origin leaves their range (2^52 quanta: a gap of about 1e7 h
+      // inside a tile).
+      if (bond3 && p->precision == NLM_PREC_FP32_FORCE &&
+          (!(2.0 / m.sigma <= 0x1p-25 * m.h) ||
+           !(org_range * m.sigma < 0x1p+52)))
+        s.tiled = false;
+    } else {
+      m.tau = m.sigma = 1.0;
+    }
+    const double bl = m.tau * m.tau / m.sigma;  // beta log2 e
+    m.c4_infl_s = m.c4_infl * m.sigma / m.tau;
+    m.c4f_infl_s = float(double(m.c4f_infl) * m.sigma / m.tau);
+    m.rcp_h_s = float(1.0 / (m.sigma * m.h));
+    m.rcp_sigma_f = float(1.0 / m.sigma);
+    m.break_lo_s = m.irreversible ? float(double(m.break_lo_f) * bl)
+                                  : std::numeric_limits<float>::infinity();
+    // r within 3e-5 (relative) of low_band <=> r^2 within about 6e-5 of
+    // low_band^2; the band on r^2 is taken a little wider
+    const double lows = m.sigma * m.low_band;
+    m.low_dd_f = float(lows * lows);
+    m.vex_dd_tol_f = float(6.1e-5 * lows * lows);
   }
   s.unroll = 4;
   if (es_mat) {

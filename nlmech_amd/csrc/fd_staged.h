@@ -64,9 +64,12 @@ struct alignas(8) StRec32 {
   uint32_t flags;
   uint32_t pad[2];
 };
-// 3D: the position as a fixed-point offset from the tile's origin in units of
-// the quantum 1/sigma, so a bond's position difference is an exact integer
-// difference rounded once to FP32.
+// 3D: the position as a fixed-point offset from the tile's origin, an even
+// number of quanta 1/sigma modulo 2^32.  A bond's components stay below 2^31
+// quanta, so its position difference is an exact integer difference whatever
+// the tile's extent (a tile of the Morton order may span a gap between two
+// bodies), rounded once to FP32.  Record 0's position is odd: it coincides
+// with no node.
 template <bool NOFAIL>
 struct alignas(8) StRec32<3, NOFAIL> {
   double u[3];
@@ -146,10 +149,12 @@ __device__ __forceinline__ void st_deferred(const FdArgs<DIM>& a, uint32_t g,
 }
 
 // A coordinate as the FP32-force records hold it: its offset from the tile's
-// origin times sigma, in fixed point (3D) or FP32 (2D).
+// origin times sigma, in fixed point (3D: the low word of 1.5 2^52 + half of
+// it is that half, rounded, modulo 2^32) or FP32 (2D).
 __device__ __forceinline__ void st_pos(double x, double o, double sigma,
                                        int32_t& q) {
-  q = __double2int_rn((x - o) * sigma);
+  const double t = __builtin_fma(x - o, 0.5 * sigma, 0x1.8p+52);
+  q = int32_t(uint32_t(__double2loint(t)) << 1);
 }
 __device__ __forceinline__ void st_pos(double x, double o, double sigma,
                                        float& q) {

@@ -101,8 +101,9 @@ struct RnpDev {
   // tau^2 / sigma = beta log2(e), so the product (tau S / sigma)(tau S r)
   // they form is beta log2(e) r S^2: the exponent of exp2 and the break
   // ratio at once
-  double tau;              // power of two nearest sqrt(beta log2 e)
-  double sigma;            // tau^2 / (beta log2 e), in [1/2, 2]
+  double tau;              // power of two (2D: nearest sqrt(beta log2 e))
+  double sigma;            // tau^2 / (beta log2 e): 2D in [1/2, 2], 3D the
+                           // reciprocal of the fixed-point quantum
   float c4f_infl_s;        // c4f_infl sigma / tau
   float rcp_h_s;           // 1 / (sigma h)
   float rcp_sigma_f;       // 1 / sigma

@@ -12,9 +12,9 @@ Bars, per node, relative to sum_j |F_ij| of the oracle's bond forces:
   FP64: about 20 roundings of half an ulp per bond force (fused operations,
     the third-order reciprocal root below one ulp entering three times) and
     the same sum: 64 x 2^-52 (3D: 92 additions in pairs, 96 x 2^-52);
-  FP32-force (3D): fixed-point positions to 2^-28 of the tile's extent
-    (about 10 h, 4e-8 of a bond), 25 FP32 roundings of 2^-24 and the rsq and
-    exp2 approximations of 2^-23: 2e-6.
+  FP32-force (3D): fixed-point positions rounded by at most 2^-28 of the
+    longest bond (3 h: 1e-8 h, twice a bond), 25 FP32 roundings of 2^-24 and
+    the rsq and exp2 approximations of 2^-23: 2e-6.
 """
 import numpy as np
 import pytest
@@ -83,8 +83,9 @@ def test_staged_force(oracle, precision, mat, shape):
                                        ((13, 11, 9), dict()),
                                        ((13, 11, 9), dict(check_sc=10.0)),
                                        ((9, 9, 9), dict(inf_type=1,
-                                                        inf_params=()))],
-                         ids=["64", "1287", "sc10", "linear"])
+                                                        inf_params=())),
+                                       ((33, 33, 33), dict())],
+                         ids=["64", "1287", "sc10", "linear", "35937"])
 def test_staged_force_3d(oracle, precision, shape, mat):
     progress(f"[gpu] staged force 3D {shape} {mat} mode {precision}")
     h = 1e-3
@@ -105,6 +106,38 @@ def test_staged_force_3d(oracle, precision, shape, mat):
     assert np.array_equal(bonds, o.get_bonds())
     if "check_sc" not in mat:
         assert bonds.sum() > 0
+    err = np.abs(f - o.get_state()[2]).max(1)
+    assert np.all(err <= BAR3[precision] * scale), (err / scale).max()
+
+
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("gap", [1e2, 1e4, 1e6, 3e7])
+def test_separated_bodies_3d(oracle, precision, gap):
+    """Two bodies `gap` mesh sizes apart, one tile spanning the gap: a bond's
+    force depends on its own length, not on the tile's extent (the last gap
+    leaves the fixed-point range: direct gathers)."""
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] separated bodies gap {gap} mode {precision}")
+    h = 1e-3
+    x, vol = pr.grid3d(13, 11, 9, h, jitter=0.05, seed=4)
+    x2, vol2 = pr.grid3d(9, 10, 11, h, jitter=0.05, seed=5)
+    x2[:, 0] += gap * h
+    x, vol = np.concatenate([x, x2]), np.concatenate([vol, vol2])
+    p = pr.Problem(name="bodies", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                   dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3))
+    u = np.random.default_rng(2).normal(scale=6e-6, size=(p.n, 3))
+    csr = oracle.neighbors(p.x, p.horizon, "brute")
+    o = oracle.OracleFD(p, csr=csr)
+    o.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+    scale = o.force_abs_sum()
+    o.compute_forces()
+    with GpuFD(p, precision=precision, csr=csr) as g:
+        g.set_state(u=u, f=np.zeros((p.n, 3)))
+        g.compute_forces()
+        f, bonds = g.get_state()[2], g.get_bonds()
+    assert np.array_equal(bonds, o.get_bonds()) and bonds.sum() > 0
     err = np.abs(f - o.get_state()[2]).max(1)
     assert np.all(err <= BAR3[precision] * scale), (err / scale).max()
 
