@@ -1494,13 +1494,18 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   }
   // node arrays in internal order
   const int stride = dim == 2 ? 2 : 4;
+  s.far = 0.;
   std::vector<double> hx(size_t(n) * stride, 0.);
   std::vector<double> hv(n);
   for (int64_t a = 0; a < n; a++) {
     int64_t i = L.perm[a];
-    for (int d = 0; d < dim; d++) hx[a * stride + d] = p->x[3 * i + d];
+    for (int d = 0; d < dim; d++) {
+      hx[a * stride + d] = p->x[3 * i + d];
+      s.far = std::max(s.far, std::fabs(p->x[3 * i + d]));
+    }
     hv[a] = p->vol[i];
   }
+  s.far = 1e6 * (s.far + horizon);
   // Per tile: the centre of its nodes' bounding box, the origin of
   // the FP32 block-relative positions (double2 per block in 2D, double4 in
   // 3D).

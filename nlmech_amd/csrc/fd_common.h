@@ -47,6 +47,7 @@ struct FdArgs {
   int tile;            // nodes of a workgroup's tile
   int parts;           // wavefronts that share a slice's rows (k_fd_st)
   int64_t halo_bytes;  // LDS bytes of the halo records (k_fd_st)
+  double far;          // coordinates of the staged kernels' record 0
 };
 
 // Displacement and velocity of a prescribed dof at time t: ULoading::apply
@@ -211,6 +212,7 @@ inline FdArgs<DIM> make_args(nlm_ctx* c) {
   a.tile = s.tile;
   a.parts = s.parts;
   a.halo_bytes = 0;
+  a.far = s.far;
   return a;
 }
 

@@ -262,7 +262,7 @@ __global__ __launch_bounds__(512) void k_fd_st(
       for (int d = 0; d < DIM; d++) {
         if constexpr (F32 && DIM == 3) r.xq[d] = 0x7fffffff;
         else if constexpr (F32) r.xq[d] = 1e15f;
-        else r.x[d] = 1e15;
+        else r.x[d] = a.far;
       }
       if constexpr (NOFAIL) r.flags = 0u;
       halo_lds[0] = r;

@@ -200,6 +200,9 @@ struct FdState {
   int tile = 256;  // nodes per workgroup of the LDS-staged kernel (its halo
                    // block): 128, 256 or 512 (k_fd_st also 64)
   int parts = 1;   // wavefronts that share a slice's rows (k_fd_st)
+  double far = 0.;  // coordinates of the FP64 staged records' record 0: 1e6
+                    // times the model's extent, so far from every node at
+                    // any scale and within the range of the products
   DevBuf row_ptr, col;  // CSR in internal ids (int64, int32)
   SellDev sell;
   // internal node order (see layout.cpp): perm[a] = reference id of a

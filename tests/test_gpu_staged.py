@@ -110,6 +110,26 @@ def test_staged_force_3d(oracle, precision, shape, mat):
     assert np.all(err <= BAR3[precision] * scale), (err / scale).max()
 
 
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64],
+                         ids=["exact", "fp64"])
+def test_coordinates_of_the_far_record(oracle, precision):
+    """Nodes at coordinates of 1e15: the record of the padded slots lies away
+    from the nodes whatever their coordinates."""
+    progress(f"[gpu] coordinates of 1e15 mode {precision}")
+    p = pr.plate2d(9, 8, 1.0, 3, 1e-4, 1, notch_len=0.0, layers=0, jitter=0.0)
+    p.x[:, :2] += 1e15 - 4.0
+    u = np.zeros((p.n, 3))
+    u[:, :2] = np.random.default_rng(2).normal(scale=1e-4, size=(p.n, 2))
+    o = oracle.OracleFD(p, csr=oracle.neighbors(p.x, p.horizon, "brute"))
+    o.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+    scale = o.force_abs_sum()
+    o.compute_forces()
+    f, bonds = force_of(p, precision, u)
+    assert np.array_equal(bonds, o.get_bonds())
+    err = np.abs(f - o.get_state()[2]).max(1)
+    assert np.all(err <= BAR[precision] * scale), (err / scale).max() / ULP
+
+
 @pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
                                        NLM_PREC_FP32_FORCE],
                          ids=["exact", "fp64", "fp32"])
