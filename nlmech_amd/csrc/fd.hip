@@ -1661,6 +1661,8 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     // Bonds whose reference length lies within 3e-5 (relative) of the
     // volume-correction edge: a static mask per (slice, slot), padded like
     // the bond bits; the step kernels send them to the exact evaluation.
+    // Bonds of coincident nodes too: the exact mode's common path has no
+    // finite direction for them (broken, their force is 0).
     // The band is far wider than the fast paths' rounding of the length.
     std::vector<unsigned long long> vw(size_t(nent / 64 + 8), 0ull);
     if (!es_mat) {
@@ -1680,7 +1682,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
               d2 += e * e;
               bond_max = std::max(bond_max, std::fabs(e));
             }
-            if (std::fabs(std::sqrt(d2) - m.low_band) <= tol)
+            if (d2 == 0. || std::fabs(std::sqrt(d2) - m.low_band) <= tol)
               word |= 1ull << lane;
           }
           vw[size_t(e0 / 64 + k)] = word;

@@ -110,6 +110,45 @@ def test_staged_force_3d(oracle, precision, shape, mat):
     assert np.all(err <= BAR3[precision] * scale), (err / scale).max()
 
 
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_coincident_nodes(oracle, precision, dim):
+    """Two nodes at one place, the bond between them broken: it has no force."""
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] coincident nodes {dim}D mode {precision}")
+    h = 1e-3
+    if dim == 2:
+        p = specimen((9, 8))
+    else:
+        x, vol = pr.grid3d(7, 6, 5, h, jitter=0.05, seed=4)
+        p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                       dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3))
+    i, j = 30, 31
+    p.x[j] = p.x[i]
+    u = np.zeros((p.n, 3))
+    u[:, :dim] = np.random.default_rng(2).normal(scale=1e-6, size=(p.n, dim))
+    o = oracle.OracleFD(p)
+    bonds = o.get_bonds()
+    rows = np.repeat(np.arange(p.n), np.diff(o.row_ptr))
+    pair = ((rows == i) & (o.col == j)) | ((rows == j) & (o.col == i))
+    assert pair.sum() == 2
+    bonds[pair] = 1
+    o.set_bonds(bonds)
+    o.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+    o.compute_forces()
+    ref = o.get_state()[2]
+    assert np.all(np.isfinite(ref))
+    with GpuFD(p, precision=precision) as g:
+        g.set_bonds(bonds)
+        g.set_state(u=u, f=np.zeros((p.n, 3)))
+        g.compute_forces()
+        f = g.get_state()[2]
+    bar = 2e-6 if precision == NLM_PREC_FP32_FORCE else BAR3[precision]
+    assert np.abs(f - ref).max() <= bar * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64],
                          ids=["exact", "fp64"])
 def test_coordinates_of_the_far_record(oracle, precision):
@@ -117,7 +156,7 @@ def test_coordinates_of_the_far_record(oracle, precision):
     from the nodes whatever their coordinates."""
     progress(f"[gpu] coordinates of 1e15 mode {precision}")
     p = pr.plate2d(9, 8, 1.0, 3, 1e-4, 1, notch_len=0.0, layers=0, jitter=0.0)
-    p.x[:, :2] += 1e15 - 4.0
+    p.x[:, :2] += 1e15  # (a corner, a row with padded slots, at the place)
     u = np.zeros((p.n, 3))
     u[:, :2] = np.random.default_rng(2).normal(scale=1e-4, size=(p.n, 2))
     o = oracle.OracleFD(p, csr=oracle.neighbors(p.x, p.horizon, "brute"))
