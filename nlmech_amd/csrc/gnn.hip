@@ -958,10 +958,7 @@ int gnn_forward(nlm_ctx* c) {
   int rc;
   if ((rc = gnn_size(c))) return rc;
   const int64_t n = s.n, ne = s.sell.nentries;
-  if (!q.mblk.p || q.mblk.bytes < sizeof(float4) * ne) {
-    if ((rc = alloc(c, q.mblk, sizeof(float4) * ne + 256))) return rc;
-    if ((rc = alloc(c, q.mdiag, sizeof(float4) * n + 256))) return rc;
-  }
+  if ((rc = precond_alloc(c))) return rc;
   const GraphArgs ga = graph_args(c);
   const unsigned gn = unsigned((n + 255) / 256);
   const unsigned gs = unsigned((s.sell.nslices + 3) / 4);

@@ -371,6 +371,13 @@ inline int reserve(nlm_ctx* c, DevBuf& b, size_t bytes) {
   return b.p && b.bytes >= bytes ? NLM_OK : alloc(c, b, bytes);
 }
 
+// Drops the previous model's tangent, preconditioner, colors, aggregates and
+// captured batch of the quasi-static solver, and the graph network's reverse
+// entries (qs.hip).
+void qs_new_model(nlm_ctx* c);
+// Sizes the learned preconditioner's blocks for the model (qs.hip).
+int precond_alloc(nlm_ctx* c);
+
 // Grid helper: ceil-divide and pad to a multiple of 8 for the XCD remap.
 inline unsigned grid_xcd(int64_t items, int block) {
   int64_t g = (items + block - 1) / block;

@@ -1221,6 +1221,13 @@ QsArgs qs_args(nlm_ctx* c) {
   return a;
 }
 
+// Destroys the captured Krylov batches.
+void drop_batches(QsState& q) {
+  if (q.bicg_graph) (void)hipGraphExecDestroy(q.bicg_graph);
+  q.bicg_graph = nullptr;
+  q.bicg_key.clear();
+}
+
 int qs_check(nlm_ctx* c, const char* fn) {
   if (!c) return NLM_ERR_INVALID;
   if (!c->fd.ready)
@@ -1257,43 +1264,40 @@ int tangent_check(nlm_ctx* c, int tangent, const char* fn) {
 int qs_alloc(nlm_ctx* c, int max_iter) {
   FdState& s = c->fd;
   QsState& q = c->qs;
-  const int64_t n = s.n;
-  const size_t nent = size_t(s.sell.nentries);
+  const size_t n = size_t(s.n), nent = size_t(s.sell.nentries);
+  q.nb = (s.n + 255) / 256;
   int rc;
-  const bool grow_vec = !q.blk.p || q.blk.bytes < nent * sizeof(double4);
-  if ((grow_vec || max_iter + 2 > q.max_iter_alloc) && q.bicg_graph) {
-    // buffers the captured batch references are about to be replaced: the
-    // executable graph goes first, so no live graph ever refers to freed
-    // memory
-    (void)hipGraphExecDestroy(q.bicg_graph);
-    q.bicg_graph = nullptr;
-    q.bicg_key.clear();
-  }
-  if (grow_vec) {
-    if ((rc = alloc(c, q.blk, nent * sizeof(double4) + 256))) return rc;
-    if ((rc = alloc(c, q.bg, nent * sizeof(double) + 256))) return rc;
-    if ((rc = alloc(c, q.diag, n * sizeof(double4) + 256))) return rc;
-    if ((rc = alloc(c, q.dinv, n * sizeof(double2) + 256))) return rc;
-    DevBuf* vec[] = {&q.r, &q.rh, &q.p, &q.v, &q.s, &q.t, &q.x,
-                     &q.ph, &q.sh, &q.b, &q.y, &q.dup, &q.u0};
-    for (DevBuf* d : vec)
-      if ((rc = alloc(c, *d, n * sizeof(double2) + 256))) return rc;
-    q.nb = (n + 255) / 256;
-    if ((rc = alloc(c, q.part, (2 * q.nb + 2 * s.sell.nslices) *
-                                   sizeof(double) + 256)))
-      return rc;
-    if ((rc = alloc(c, q.ctl, 64))) return rc;
-    if (!q.e0) NLM_HIP(c, hipEventCreate(&q.e0));
-    if (!q.e1) NLM_HIP(c, hipEventCreate(&q.e1));
-    if (!q.hctl)
-      NLM_HIP(c, hipHostMalloc(reinterpret_cast<void**>(&q.hctl),
-                               4 * sizeof(int), hipHostMallocDefault));
-  }
+  // Every buffer against its own size: a context may be set up again with
+  // more nodes but fewer neighbors.  A captured batch goes before a buffer
+  // it references, so no live graph ever refers to freed memory.
+  auto fit = [&](DevBuf& b, size_t bytes) -> int {
+    if (b.p && b.bytes >= bytes) return NLM_OK;
+    drop_batches(q);
+    return alloc(c, b, bytes);
+  };
+  if ((rc = fit(q.blk, nent * sizeof(double4) + 256)) ||
+      (rc = fit(q.bg, nent * sizeof(double) + 256)) ||
+      (rc = fit(q.diag, n * sizeof(double4) + 256)) ||
+      (rc = fit(q.dinv, n * sizeof(double2) + 256)))
+    return rc;
+  DevBuf* vec[] = {&q.r, &q.rh, &q.p, &q.v, &q.s, &q.t, &q.x,
+                   &q.ph, &q.sh, &q.b, &q.y, &q.dup, &q.u0};
+  for (DevBuf* d : vec)
+    if ((rc = fit(*d, n * sizeof(double2) + 256))) return rc;
+  if ((rc = fit(q.part, (2 * size_t(q.nb) + 2 * size_t(s.sell.nslices)) *
+                                sizeof(double) + 256)) ||
+      (rc = fit(q.ctl, 64)))
+    return rc;
+  if (!q.e0) NLM_HIP(c, hipEventCreate(&q.e0));
+  if (!q.e1) NLM_HIP(c, hipEventCreate(&q.e1));
+  if (!q.hctl)
+    NLM_HIP(c, hipHostMalloc(reinterpret_cast<void**>(&q.hctl),
+                             4 * sizeof(int), hipHostMallocDefault));
   if (max_iter + 2 > q.max_iter_alloc) {
-    q.max_iter_alloc = max_iter + 2;
-    if ((rc = alloc(c, q.scal, (8 + 4 * size_t(q.max_iter_alloc)) *
-                                   sizeof(double))))
+    if ((rc = fit(q.scal,
+                  (8 + 4 * size_t(max_iter + 2)) * sizeof(double))))
       return rc;
+    q.max_iter_alloc = max_iter + 2;
   }
   return NLM_OK;
 }
@@ -1543,11 +1547,7 @@ int precond_bf16(nlm_ctx* c) {
   const int64_t nent = c->fd.sell.nentries;
   int rc;
   if (!q.mhalf.p || q.mhalf.bytes < sizeof(Bf4) * nent) {
-    if (q.bicg_graph) {  // it may reference the buffer being replaced
-      (void)hipGraphExecDestroy(q.bicg_graph);
-      q.bicg_graph = nullptr;
-      q.bicg_key.clear();
-    }
+    drop_batches(q);  // they may reference the buffer being replaced
     if ((rc = alloc(c, q.mhalf, sizeof(Bf4) * nent + 256))) return rc;
   }
   hipLaunchKernelGGL(k_blocks_bf16, dim3(unsigned((nent + 255) / 256)),
@@ -1922,6 +1922,28 @@ double ms_since(std::chrono::steady_clock::time_point t0) {
 
 }  // namespace
 
+int precond_alloc(nlm_ctx* c) {
+  QsState& q = c->qs;
+  const size_t nent = size_t(c->fd.sell.nentries), n = size_t(c->fd.n);
+  const size_t bb = sizeof(float4) * nent + 256, db = sizeof(float4) * n + 256;
+  if (!q.mblk.p || q.mblk.bytes < bb || !q.mdiag.p || q.mdiag.bytes < db)
+    drop_batches(q);
+  if (int rc = reserve(c, q.mblk, bb)) return rc;
+  return reserve(c, q.mdiag, db);
+}
+
+void qs_new_model(nlm_ctx* c) {
+  QsState& q = c->qs;
+  drop_batches(q);
+  q.assembled = q.has_m = q.mhalf_ok = false;
+  q.bs_mode = 0;
+  q.ncolors = 0;
+  q.adj_ptr.release();  // (coarse_setup sizes what goes with it)
+  q.cinv = nullptr;
+  q.m = 0;
+  c->gnn.n = c->gnn.ne = 0;
+}
+
 // Preconditioner construction by the graph network (gnn.hip); returns
 // NLM_ERR_STATE when no network is attached to the context.
 int gnn_predict_precond(nlm_ctx* c);
@@ -2025,10 +2047,7 @@ extern "C" int nlm_qs_set_precond(nlm_ctx* c, const double* blocks,
   if ((rc = qs_alloc(c, 8))) return rc;
   NLM_HIP(c, hipStreamSynchronize(c->stream));
   const int64_t nent = s.sell.nentries;
-  if (!q.mblk.p || q.mblk.bytes < sizeof(float4) * nent) {
-    if ((rc = alloc(c, q.mblk, sizeof(float4) * nent + 256))) return rc;
-    if ((rc = alloc(c, q.mdiag, sizeof(float4) * s.n + 256))) return rc;
-  }
+  if ((rc = precond_alloc(c))) return rc;
   std::vector<float4> hb(nent, make_float4(0.f, 0.f, 0.f, 0.f)), hd(s.n);
   std::vector<int64_t> slp(s.sell.nslices + 1), roff(s.n);
   std::vector<uint16_t> rl(s.n);

@@ -83,3 +83,65 @@ def test_falls_back(kind):
         assert rr > 1e-8 or res <= 1e-7
         if kind == "one_way":
             assert rr <= 1e-8
+
+
+def setup_again(g, p):
+    """Another problem set up on the context of g (which is used up)."""
+    from nlmech_amd import capi
+    from nlmech_amd.engine import GpuFD
+
+    class Lib:  # hands out the context there is
+        def __getattr__(self, name):
+            return getattr(g.lib, name)
+
+        def nlm_ctx_create(self, h, device):
+            h._obj.value, g.ctx = g.ctx.value, None
+            return 0
+
+    load = capi.load
+    capi.load = Lib
+    try:
+        return GpuFD(p, precision=NLM_PREC_FP64_EXACT)
+    finally:
+        capi.load = load
+
+
+def solves(g, p):
+    """Every solver's answers, on the model as it stands."""
+    b = np.zeros((p.n, 3))
+    b[:, :2] = np.random.default_rng(4).standard_normal((p.n, 2))
+    g.qs_assemble(0)
+    out = [g.qs_linear_solve(b, precond=pc, tol=1e-10, max_iter=300)
+           for pc in (1, 1 | 16, 0)]
+    st = g.qs_solve(2, lin_max_iter=600)
+    out.append((st["linear_iters"], st["newton_iters"], st["residual"]))
+    return [v for o in out for v in o] + list(g.get_state())
+
+
+@pytest.mark.parametrize("kind", ["smaller", "more_nodes_fewer_bonds"])
+def test_second_model_on_a_context(kind):
+    """A context set up again gives a fresh context's answers, bit for bit: a
+    smaller model (fewer partial sums), one with more nodes and slices but
+    fewer bonds (buffers larger than the first model's although the tangent
+    is smaller); what the first model left is not solved with."""
+    from nlmech_amd.capi import NLM_QS_PRECOND_COARSE, NlmError
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] second model on a context: {kind}")
+    assert NLM_QS_PRECOND_COARSE == 16
+    if kind == "smaller":
+        first, second = pr.qs_plate(40, jitter=0.05), pr.qs_plate(12)
+    else:
+        first = pr.qs_plate(20, ratio=6, jitter=0.05)
+        second = pr.qs_plate(36, ratio=2, jitter=0.05)
+    with GpuFD(second, precision=NLM_PREC_FP64_EXACT) as g:
+        nnz2 = g.nnz
+        want = solves(g, second)
+    g = GpuFD(first, precision=NLM_PREC_FP64_EXACT)
+    assert (g.nnz > nnz2) and (first.n > second.n) == (kind == "smaller")
+    solves(g, first)
+    g = setup_again(g, second)
+    with pytest.raises(NlmError):
+        g.qs_linear_solve(np.zeros((second.n, 3)))
+    for a, b in zip(want, solves(g, second)):
+        assert np.array_equal(a, b)
+    g.close()
