@@ -402,7 +402,9 @@ const char* nlm_fd_kernel_name(nlm_ctx* ctx);
  * system is solved to a relative residual by conjugate gradients in the
  * volume-weighted inner product (the analytic tangent with precond NONE or
  * JACOBI, where it is self-adjoint) or by BiCGSTAB (every other case, and
- * where conjugate gradients break down or reach the iteration limit). */
+ * where conjugate gradients break down or reach the iteration limit: then
+ * for the rest of the load step; each method keeps to lin_max_iter, and the
+ * statistics count the iterations of both). */
 #define NLM_QS_TANGENT_FULL 0      /* exact derivative, all 2x2 entries */
 #define NLM_QS_TANGENT_COMPONENT 1 /* same-component entries only, the
                                       entries the reference's central-

@@ -68,7 +68,8 @@ extern "C" void nlm_ctx_destroy(nlm_ctx* c) {
   if (c->fd.ev0) (void)hipEventDestroy(c->fd.ev0);
   if (c->fd.ev1) (void)hipEventDestroy(c->fd.ev1);
   if (c->fd.graph) (void)hipGraphExecDestroy(c->fd.graph);
-  if (c->qs.bicg_graph) (void)hipGraphExecDestroy(c->qs.bicg_graph);
+  for (hipGraphExec_t g : c->qs.batch_graph)
+    if (g) (void)hipGraphExecDestroy(g);
   if (c->qs.e0) (void)hipEventDestroy(c->qs.e0);
   if (c->qs.e1) (void)hipEventDestroy(c->qs.e1);
   if (c->qs.hctl) (void)hipHostFree(c->qs.hctl);

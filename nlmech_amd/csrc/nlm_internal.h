@@ -265,18 +265,19 @@ struct QsState {
   DevBuf adj_ptr, adj, cA, cB, rc, zcp, zcs;
   double* cinv = nullptr;
   int m = 0;
-  hipEvent_t e0 = nullptr, e1 = nullptr;  // BiCGSTAB batches in flight
+  hipEvent_t e0 = nullptr, e1 = nullptr;  // Krylov batches in flight
   int* hctl = nullptr;       // pinned: control words of two batches
   // finite-difference tangent: node colors (no two nodes of one color
   // within 4 horizons), perturbation factor (eps = factor * h)
   DevBuf color;
   int ncolors = 0;
   double fd_perturbation = 1e-7;
-  // BiCGSTAB iterations run in batches replayed from a captured HIP graph;
-  // the key holds the kernel arguments of the capture
+  // Krylov iterations run in batches replayed from a captured HIP graph, one
+  // for each method (0: BiCGSTAB, 1: conjugate gradients); the key holds the
+  // kernel arguments of the capture
   bool use_graph = true;
-  hipGraphExec_t bicg_graph = nullptr;
-  std::vector<unsigned char> bicg_key;
+  hipGraphExec_t batch_graph[2] = {nullptr, nullptr};
+  std::vector<unsigned char> batch_key[2];
 };
 
 // Graph-network preconditioner: FP32 master weights, gradient, Adam

@@ -1223,9 +1223,11 @@ QsArgs qs_args(nlm_ctx* c) {
 
 // Destroys the captured Krylov batches.
 void drop_batches(QsState& q) {
-  if (q.bicg_graph) (void)hipGraphExecDestroy(q.bicg_graph);
-  q.bicg_graph = nullptr;
-  q.bicg_key.clear();
+  for (int m = 0; m < 2; m++) {
+    if (q.batch_graph[m]) (void)hipGraphExecDestroy(q.batch_graph[m]);
+    q.batch_graph[m] = nullptr;
+    q.batch_key[m].clear();
+  }
 }
 
 int qs_check(nlm_ctx* c, const char* fn) {
@@ -1336,7 +1338,7 @@ VecArgs vec_args(nlm_ctx* c) {
 constexpr int kBicgBatch = 8;  // (even: k_cg_mv)
 static_assert(kBicgBatch % 2 == 0, "p buffers by the parity of k");
 
-// Everything a captured BiCGSTAB batch depends on.
+// Everything a captured Krylov batch depends on.
 struct BicgKey {
   VecArgs a;
   QsArgs qa;
@@ -1662,25 +1664,26 @@ int run_batches(nlm_ctx* c, const VecArgs& a, BicgKey& key,
     key.diag = q.diag.p;
     key.g = node_grid(c->fd);
     const unsigned char* kb = reinterpret_cast<const unsigned char*>(&key);
-    if (!q.bicg_graph || q.bicg_key.size() != sizeof(key) ||
-        std::memcmp(kb, q.bicg_key.data(), sizeof(key)) != 0) {
-      if (q.bicg_graph) (void)hipGraphExecDestroy(q.bicg_graph);
-      q.bicg_graph = nullptr;
+    hipGraphExec_t& graph = q.batch_graph[key.method];
+    std::vector<unsigned char>& held = q.batch_key[key.method];
+    if (!graph || held.size() != sizeof(key) ||
+        std::memcmp(kb, held.data(), sizeof(key)) != 0) {
+      if (graph) (void)hipGraphExecDestroy(graph);
+      graph = nullptr;
       hipGraph_t gr = nullptr;
       NLM_HIP(c, hipStreamBeginCapture(c->stream,
                                        hipStreamCaptureModeThreadLocal));
       launch_batch();
       NLM_HIP(c, hipStreamEndCapture(c->stream, &gr));
-      hipError_t e = hipGraphInstantiate(&q.bicg_graph, gr, nullptr, nullptr,
-                                         0);
+      hipError_t e = hipGraphInstantiate(&graph, gr, nullptr, nullptr, 0);
       (void)hipGraphDestroy(gr);
       if (e != hipSuccess) {
-        q.bicg_graph = nullptr;
+        graph = nullptr;
         return fail(c, NLM_ERR_HIP, "Krylov solve: graph instantiation failed");
       }
-      q.bicg_key.assign(kb, kb + sizeof(key));
+      held.assign(kb, kb + sizeof(key));
     }
-    exec = q.bicg_graph;
+    exec = graph;
   }
   // One batch stays queued ahead of the host's check of the previous one,
   // so the device does not idle through the round trip; a batch queued
@@ -1882,22 +1885,32 @@ int conjugate_gradients(nlm_ctx* c, int precond, double tol, int max_iter,
   std::memset(&key, 0, sizeof(key));
   key.method = 1;
   key.precond = precond;
-  return run_batches(c, a, key, launch_batch, bb, iters, relres, ok);
+  rc = run_batches(c, a, key, launch_batch, bb, iters, relres, ok);
+  // (the device sees convergence one iteration later: not that of the last)
+  if (!rc && !*ok && *iters == max_iter && *relres <= tol) *ok = true;
+  return rc;
 }
 
 // Solves A_ff x = b (q.b -> q.x): conjugate gradients where the tangent and
 // the preconditioner are self-adjoint (the analytic tangent; none or point
 // Jacobi), BiCGSTAB otherwise and where conjugate gradients end without
-// convergence.
+// convergence: *cg (whether they may be tried) turns false then.  *iters are
+// the iterations of the method that gave x, *spent those of both.
 int linear_solve(nlm_ctx* c, int precond, double tol, int max_iter, int* iters,
-                 double* relres, bool* ok) {
-  if ((precond == NLM_QS_PRECOND_NONE || precond == NLM_QS_PRECOND_JACOBI) &&
+                 int* spent, double* relres, bool* ok, bool* cg) {
+  *spent = 0;
+  if (*cg &&
+      (precond == NLM_QS_PRECOND_NONE || precond == NLM_QS_PRECOND_JACOBI) &&
       c->qs.tangent != NLM_QS_TANGENT_FD) {
     const int rc =
         conjugate_gradients(c, precond, tol, max_iter, iters, relres, ok);
+    *spent = *iters;
     if (rc || *ok) return rc;
+    *cg = false;
   }
-  return bicgstab(c, precond, tol, max_iter, iters, relres, ok);
+  const int rc = bicgstab(c, precond, tol, max_iter, iters, relres, ok);
+  *spent += *iters;
+  return rc;
 }
 
 // ||R||_2 of the residual of the current force (q.b <- R).
@@ -2166,10 +2179,12 @@ extern "C" int nlm_qs_linear_solve(nlm_ctx* c, const double* b, double* x,
   if ((rc = qs_alloc(c, max_iter))) return rc;
   if (precond != base && (rc = coarse_setup(c))) return rc;
   if ((rc = aos_to_dev(c, b, q.b))) return rc;
-  int it = 0;
+  int it = 0, spent = 0;
   double rr = 0.;
-  bool ok = false;
-  if ((rc = linear_solve(c, precond, tol, max_iter, &it, &rr, &ok))) return rc;
+  bool ok = false, cg = true;
+  if ((rc = linear_solve(c, precond, tol, max_iter, &it, &spent, &rr, &ok,
+                         &cg)))
+    return rc;
   if (iters) *iters = it;
   if (relres) *relres = rr;
   return dev_to_aos(c, q.x, x);
@@ -2210,15 +2225,16 @@ extern "C" int nlm_qs_solve(nlm_ctx* c, const nlm_qs_options* o,
     stats.ms_precond += ms_since(t0);
     return r;
   };
+  bool cg = true;  // conjugate gradients, until they fail in a load step
   auto linear = [&](int* it_out) -> int {
     const auto t0 = std::chrono::steady_clock::now();
-    int it = 0;
+    int it = 0, spent = 0;
     double rr = 0.;
     bool ok = false;
-    int r = linear_solve(c, o->precond, o->lin_tol, o->lin_max_iter, &it, &rr,
-                     &ok);
+    int r = linear_solve(c, o->precond, o->lin_tol, o->lin_max_iter, &it,
+                         &spent, &rr, &ok, &cg);
     stats.ms_linear += ms_since(t0);
-    stats.linear_iters += it;
+    stats.linear_iters += spent;
     if (!ok) stats.linear_failures++;
     *it_out = it;
     return r;
@@ -2236,6 +2252,7 @@ extern "C" int nlm_qs_solve(nlm_ctx* c, const nlm_qs_options* o,
     const double t = double(s.step + 1) * o->dt;
     double rnorm = 0., r0 = 0.;
     int newton = 0, lit = 0;
+    cg = true;
     if (o->predictor) {
       // linearized first iteration at the previous equilibrium
       hipLaunchKernelGGL(k_qs_dup, dim3(g), dim3(256), 0, c->stream, s.n,

@@ -1,7 +1,8 @@
 """Conjugate gradients of the quasi-static solver: against a dense solve at
 sizes around a slice and a 256-node block, on both tangents and both forms of
-their products; a softening tangent (not positive) and a bond broken in one
-direction only (not self-adjoint) end in BiCGSTAB's answer.
+their products; a softening tangent (not positive) and bonds broken in one
+direction only (not self-adjoint) end in BiCGSTAB's answer; the iteration
+limit; a context set up for a second model.
 
 Bar: the solver stops at ||r|| <= 1e-10 ||b||; the true residual adds the
 recursion's rounding, n iterations of a few ulp: 2e-10 for these sizes.
@@ -57,16 +58,38 @@ def test_dense(nx, tangent, precond):
             assert 0 < it < 4000 and rr <= 1e-10 and res <= 2e-10
 
 
+def cg_end(A, W, b, tol, limit):
+    """How conjugate gradients in the inner product W, point Jacobi, end:
+    (iterations, True where they converge)."""
+    z = b / np.diag(A)
+    r, p, rho = b.copy(), z.copy(), W @ (b * z)
+    for it in range(limit):
+        if np.linalg.norm(r) <= tol * np.linalg.norm(b):
+            return it, True
+        q = A @ p
+        pq = W @ (p * q)
+        if not (rho > 0 and pq > 0):
+            return it, False
+        r -= rho / pq * q
+        z = r / np.diag(A)
+        rho, beta = W @ (r * z), rho
+        p = z + rho / beta * p
+    return limit, False
+
+
 @pytest.mark.parametrize("kind", ["softening", "one_way"])
 def test_falls_back(kind):
+    """Where conjugate gradients end without convergence (restated here), the
+    answer is BiCGSTAB's."""
     from nlmech_amd.engine import GpuFD
     progress(f"[gpu] cg fallback {kind}")
     p = pr.qs_plate(12, jitter=0.05, layers=1, check_sc=10.0)
+    limit = 2000
     with GpuFD(p, precision=NLM_PREC_FP64_EXACT) as g:
         if kind == "softening":
-            # strains past the force's maximum on many bonds
+            # strains past the force's maximum on some bonds
             u = np.zeros((p.n, 3))
-            u[:, :2] = np.random.default_rng(1).normal(scale=1.2e-5,
+            u[:, :2] = np.random.default_rng(1).normal(scale=3e-6,
                                                        size=(p.n, 2))
             g.set_state(u=u)
         else:
@@ -74,15 +97,50 @@ def test_falls_back(kind):
             bonds[::5] = 1
             g.set_bonds(bonds)
         g.qs_assemble(0)
+        fix = g.get_fixity()
+        free = np.stack([fix & 1, fix >> 1 & 1], 1).reshape(-1) == 0
+        A = dense(g, p)[np.ix_(free, free)]
+        W = np.repeat(p.vol, 2)[free]
+        b = np.random.default_rng(4).standard_normal((p.n, 2)).reshape(-1)
+        ends, conv = cg_end(A, W, b[free], 1e-8, limit)
+        assert not conv and (ends == limit) == (kind == "one_way")
         if kind == "softening":
             w = np.linalg.eigvalsh(dense(g, p) * np.repeat(p.vol, 2)[:, None])
             assert w[0] < -1e-3 * w[-1]
-        it, rr, res = check(g, p, 1, max_iter=20000, tol=1e-8)
-        # (BiCGSTAB may stop at its limit on an indefinite tangent; what it
-        # reports as solved is solved)
-        assert rr > 1e-8 or res <= 1e-7
-        if kind == "one_way":
-            assert rr <= 1e-8
+        it, rr, res = check(g, p, 1, max_iter=limit, tol=1e-8)
+        assert 0 < it < limit and rr <= 1e-8 and res <= 2e-8
+
+
+def test_converged_at_the_limit():
+    """Convergence in the last iteration allowed is convergence; one iteration
+    less goes to BiCGSTAB."""
+    from nlmech_amd.engine import GpuFD
+    progress("[gpu] cg converged at the iteration limit")
+    p = pr.qs_plate(17, jitter=0.05, layers=1)
+    b = np.zeros((p.n, 3))
+    b[:, :2] = np.random.default_rng(4).standard_normal((p.n, 2))
+    with GpuFD(p, precision=NLM_PREC_FP64_EXACT) as g:
+        g.qs_assemble(0)
+        for graph in (True, False):
+            g.qs_set_graph(graph)
+            x, it, rr = g.qs_linear_solve(b, tol=1e-10)
+            x1, it1, rr1 = g.qs_linear_solve(b, tol=1e-10, max_iter=it)
+            assert it1 == it and rr1 == rr and np.array_equal(x, x1)
+            _, it2, rr2 = g.qs_linear_solve(b, tol=1e-10, max_iter=it - 1)
+            assert it2 < it and rr2 <= 1e-10
+
+
+def test_failure_is_remembered_in_a_load_step():
+    """A limit that neither method reaches convergence in: conjugate gradients
+    are tried once a load step, BiCGSTAB in every Newton iteration."""
+    from nlmech_amd.engine import GpuFD
+    progress("[gpu] cg failure within a load step")
+    p = pr.qs_plate(40, jitter=0.05, pull=2e-5)
+    with GpuFD(p, precision=NLM_PREC_FP64_EXACT) as g:
+        st = g.qs_solve(2, lin_max_iter=60)
+    newton = st["newton_iters"]
+    assert newton >= 4 and st["linear_failures"] == newton
+    assert st["linear_iters"] == 60 * (2 + newton)
 
 
 def setup_again(g, p):
