@@ -180,6 +180,8 @@ SIGNATURES = {
     "nlm_fd_autotune_tiles": (C.c_int, [_P, C.POINTER(C.c_int),
                                         C.POINTER(C.c_int), _D]),
     "nlm_fd_set_tile": (C.c_int, [_P, C.c_int]),
+    "nlm_fd_get_tile": (C.c_int, [_P, C.POINTER(C.c_int),
+                                  C.POINTER(C.c_int)]),
     "nlm_fd_kernel_name": (C.c_char_p, [_P]),
     "nlm_es_params_from_deck": (C.c_int, [C.POINTER(EsDeck),
                                           C.POINTER(EsParams)]),

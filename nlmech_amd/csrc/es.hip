@@ -878,8 +878,13 @@ int es_autotune(nlm_ctx* c, int* chosen, double* best_us, double* us3) {
   NLM_HIP(c, hipEventCreate(&e0));
   NLM_HIP(c, hipEventCreate(&e1));
   const int reps = 4;
-  for (int k = 0; k < 3; k++) {
+  for (int k : {1, 0, 2}) {
     const int U = cands[k];
+    // (k_es_force_st has one width: its one time for every width)
+    if (U != 4 && st_pass(c, s, true)) {
+      if (us3) us3[k] = best;
+      continue;
+    }
     launch_any(c, KIND_CD, false, s.time, s.time + s.dt, U);
     NLM_HIP(c, hipEventRecord(e0, c->stream));
     for (int r = 0; r < reps; r++)

@@ -996,12 +996,17 @@ void launch_inf(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
   else launch_k<DIM, MODE, KIND, BASE_F, 2, 4>(c, a, tf, tn);
 }
 
+// Whether the bond-based step launches k_fd_st: the staged kernel of the FP64
+// modes, of 3D models and of split rows.
+bool staged_step(const FdState& s) {
+  return s.tiled && s.use_tiled &&
+         (s.dim == 3 || s.precision != kModeFp32 || s.parts > 1);
+}
+
 template <int DIM, int KIND, bool BASE_F>
 void launch_mode(nlm_ctx* c, const FdArgs<DIM>& a, double tf, double tn,
                  int U) {
-  // the staged kernel of the FP64 modes and of 3D models
-  if (c->fd.tiled && c->fd.use_tiled &&
-      (DIM == 3 || c->fd.precision != kModeFp32 || c->fd.parts > 1)) {
+  if (staged_step(c->fd)) {
     FdArgs<DIM> b = a;
     if (KIND != KIND_CD) b.kind = BASE_F ? KIND_FORCE_ADD : KIND_FORCE;
     b.halo_bytes =
@@ -1451,7 +1456,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     return rc;
   if ((rc = up(s.halo, L.halo.data(), sizeof(int32_t) * L.halo.size()))) return rc;
   s.halo_max = L.halo_max;
-  s.tile = tile;
+  s.tile = s.own_tile = tile;
   s.parts = es_mat ? rule.parts
                    : stage_parts(dim, p->precision, L.nslices, tile);
   // the staged bond-based kernels
@@ -2384,7 +2389,9 @@ namespace {
 // next step anyway) and a scratch copy of the bond bits, so the model state
 // is unchanged.
 // us[k]: microseconds per step with chunk width {2, 4, 8}[k] (0 = not
-// timed: the FP64-exact mode runs U = 4 only).
+// timed: the FP64-exact mode has one width, reported as 4).  Split rows have
+// one width too, the staged 3D kernel no 8: the widths that launch the same
+// kernel get its one time.
 template <int DIM>
 int time_chunks(nlm_ctx* c, double us[3]) {
   FdState& s = c->fd;
@@ -2400,10 +2407,15 @@ int time_chunks(nlm_ctx* c, double us[3]) {
   NLM_HIP(c, hipEventCreate(&e0));
   NLM_HIP(c, hipEventCreate(&e1));
   const int reps = 6;
-  for (int k = 0; k < 3; k++) {
+  const bool st = staged_step(s);
+  us[0] = us[2] = 0.;
+  for (int k : {1, 0, 2}) {
     const int U = cands[k];
-    us[k] = 0.;
     if (s.precision == NLM_PREC_FP64_EXACT && U != 4) continue;
+    if (U != 4 && st && (s.parts > 1 || (DIM == 3 && U == 8))) {
+      us[k] = us[1];
+      continue;
+    }
     for (int r = 0; r < 2; r++)
       launch_mode<DIM, KIND_CD, false>(c, a, s.time, s.time + s.dt, U);
     NLM_HIP(c, hipEventRecord(e0, c->stream));
@@ -2421,11 +2433,12 @@ int time_chunks(nlm_ctx* c, double us[3]) {
   return NLM_OK;
 }
 
+// (4 where another is no faster)
 int best_chunk(const double us[3], double* best) {
   const int cands[3] = {2, 4, 8};
   int pick = 4;
   *best = 1e300;
-  for (int k = 0; k < 3; k++)
+  for (int k : {1, 0, 2})
     if (us[k] > 0. && us[k] < *best) {
       *best = us[k];
       pick = cands[k];
@@ -2446,8 +2459,8 @@ int autotune(nlm_ctx* c, int* chosen, double* best_us) {
   return NLM_OK;
 }
 
-// Rebuilds the staged kernels' halos for tiles of bn nodes (128, 256 or
-// 512): halo lists and halo-local entries (the 2D bond-based kernel's: LDS
+// Rebuilds the staged kernels' halos for tiles of bn nodes (64 to 512): halo
+// lists and halo-local entries (the 2D bond-based kernel's: LDS
 // byte offsets), the tile origins, the LDS budget and, for the state-based
 // FP32-force passes, the fixed-point quantum (the origins' range changes
 // with the tile).  NLM_ERR_INVALID (state unchanged) when the largest halo
@@ -2591,31 +2604,41 @@ extern "C" int nlm_fd_autotune_tiles(nlm_ctx* c, int* tile, int* chunk,
     if (us) std::memcpy(us, tab, sizeof(tab));
     return NLM_OK;
   }
-  double best = 1e300;
-  int bt = s.tile, bu = s.unroll;
+  // times of a tile's chunk widths; its best and that one's time
+  auto time_tile = [&](int bn, double* us3, int* u, double* b) -> int {
+    if (int r = retile(c, bn)) return r;
+    int pick = 4;
+    double t = 0.;
+    const int r = es ? es_autotune(c, &pick, &t, us3) : time_chunks<2>(c, us3);
+    if (!r) *u = best_chunk(us3, b);
+    return r;
+  };
+  double best = 1e300, own = 1e300;
+  int bt = 0, bu = 4, ou = 4;
   for (int k = 0; k < 3; k++) {
-    if ((rc = retile(c, tiles[k]))) {
+    double b = 0.;
+    int u = 4;
+    if ((rc = time_tile(tiles[k], tab + 3 * k, &u, &b))) {
       if (rc != NLM_ERR_INVALID) return rc;
       c->err.clear();  // over the LDS budget: not a candidate
       continue;
     }
-    if (es) {
-      int pick = 4;
-      double bu = 0.;
-      if ((rc = es_autotune(c, &pick, &bu, tab + 3 * k))) return rc;
-    } else if ((rc = time_chunks<2>(c, tab + 3 * k))) {
-      return rc;
-    }
-    double b;
-    const int u = best_chunk(tab + 3 * k, &b);
     if (b < best) {
       best = b;
       bt = tiles[k];
       bu = u;
     }
   }
-  if ((rc = retile(c, bt))) return rc;
-  s.unroll = bu;
+  // the setup's own tile, where the table has it not (64 nodes, the rule's
+  // choice for small models): kept unless a pair of the table is faster
+  if (std::find(tiles, tiles + 3, s.own_tile) == tiles + 3) {
+    double own3[3] = {0., 0., 0.};
+    if ((rc = time_tile(s.own_tile, own3, &ou, &own))) return rc;
+  }
+  const bool keep = own <= best;
+  if ((rc = retile(c, keep ? s.own_tile : bt))) return rc;
+  s.unroll = keep ? ou : bu;
+  if (bt == 0) bt = s.own_tile;  // (no tile of the table fits)
   if (tile) *tile = bt;
   if (chunk) *chunk = bu;
   if (us) std::memcpy(us, tab, sizeof(tab));
@@ -2625,8 +2648,9 @@ extern "C" int nlm_fd_autotune_tiles(nlm_ctx* c, int* tile, int* chunk,
 extern "C" int nlm_fd_set_tile(nlm_ctx* c, int tile) {
   int rc = check_ready(c, "nlm_fd_set_tile");
   if (rc) return rc;
-  if (tile != 128 && tile != 256 && tile != 512)
-    return fail(c, NLM_ERR_INVALID, "nlm_fd_set_tile: 128, 256 or 512");
+  if (tile != 128 && tile != 256 && tile != 512 && tile != c->fd.own_tile)
+    return fail(c, NLM_ERR_INVALID,
+                "nlm_fd_set_tile: 128, 256, 512 or the setup's own");
   const bool es = c->fd.material == NLM_MATERIAL_ELASTIC_STATE;
   if (es ? !(c->fd.es_tiled && c->fd.dim == 3)
          : !(c->fd.tiled && c->fd.dim == 2))
@@ -2634,6 +2658,14 @@ extern "C" int nlm_fd_set_tile(nlm_ctx* c, int tile) {
                 "nlm_fd_set_tile: the model has no LDS-staged step kernel");
   c->fd.graph_chunk = 0;
   return retile(c, tile);
+}
+
+extern "C" int nlm_fd_get_tile(nlm_ctx* c, int* tile, int* parts) {
+  int rc = check_ready(c, "nlm_fd_get_tile");
+  if (rc) return rc;
+  if (tile) *tile = c->fd.tile;
+  if (parts) *parts = c->fd.parts;
+  return NLM_OK;
 }
 
 extern "C" int nlm_fd_set_unroll(nlm_ctx* c, int unroll) {

@@ -199,6 +199,7 @@ struct FdState {
   int unroll = 4;  // neighbor slots per chunk in the fused step kernel
   int tile = 256;  // nodes per workgroup of the LDS-staged kernel (its halo
                    // block): 128, 256 or 512 (k_fd_st also 64)
+  int own_tile = 256;  // the setup's choice (nlm_fd_set_tile, autotuner)
   int parts = 1;   // wavefronts that share a slice's rows (k_fd_st)
   double far = 0.;  // coordinates of the FP64 staged records' record 0: 1e6
                     // times the model's extent, so far from every node at

@@ -234,9 +234,11 @@ class GpuFD:
         self._call("nlm_fd_set_unroll", int(unroll))
 
     def autotune_tiles(self):
-        """(tile, chunk, table): the chosen staged-kernel tile and chunk
-        width and the 3 x 3 table of microseconds per step (rows: tiles 128,
-        256, 512; columns: chunks 2, 4, 8; 0 = not run)."""
+        """(tile, chunk, table): the fastest staged-kernel tile and chunk
+        width of the 3 x 3 table of microseconds per step (rows: tiles 128,
+        256, 512; columns: chunks 2, 4, 8; 0 = not run).  They are in effect
+        afterwards unless a small model's own tile of 64 is faster
+        (get_tile)."""
         t, u = C.c_int(), C.c_int()
         us = np.zeros(9)
         self._call("nlm_fd_autotune_tiles", C.byref(t), C.byref(u),
@@ -245,6 +247,12 @@ class GpuFD:
 
     def set_tile(self, tile: int):
         self._call("nlm_fd_set_tile", int(tile))
+
+    def get_tile(self):
+        """(nodes of a workgroup's tile, wavefronts sharing a slice)."""
+        t, k = C.c_int(), C.c_int()
+        self._call("nlm_fd_get_tile", C.byref(t), C.byref(k))
+        return t.value, k.value
 
     def timed_steps(self, nsteps: int):
         tot = C.c_double()

@@ -362,9 +362,13 @@ void FDModel<T>::initHObjects() {
           "nlm_fd_autotune_tiles");
     const int t = tile == 128 ? 0 : tile == 512 ? 2 : 1;
     const int k = chosen == 2 ? 0 : chosen == 8 ? 2 : 1;
-    std::cout << "FDModel: autotuner chose tiles of " << tile << " nodes, "
-              << chosen << " slots per pass (" << us[3 * t + k]
-              << " us per step)\n";
+    int kept = 0;
+    check(nlm_fd_get_tile(d_ctx, &kept, nullptr), "nlm_fd_get_tile");
+    std::cout << "FDModel: autotuner chose tiles of " << kept << " nodes";
+    if (kept == tile)
+      std::cout << ", " << chosen << " slots per pass (" << us[3 * t + k]
+                << " us per step)";
+    std::cout << "\n";
   }
 }
 

@@ -305,3 +305,45 @@ def test_fused_verlet_steps(precision, shape):
         assert np.array_equal(a, b)
     if dim == 2:
         assert outs[0][3].sum() > 0
+
+
+@pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
+                                       NLM_PREC_FP32_FORCE],
+                         ids=["exact", "fp64", "fp32"])
+@pytest.mark.parametrize("kind", ["plate", "state"])
+def test_autotuner_keeps_a_faster_setup(precision, kind):
+    """On a model that starts on tiles of 64 nodes the autotuner leaves a setup
+    that is no slower than the one it found, and the setup's tile can be set
+    again."""
+    from nlmech_amd.engine import GpuFD, NlmError
+    progress(f"[gpu] autotuner on a small model, {kind} mode {precision}")
+    if kind == "plate":
+        p = pr.plate2d(100, 100, 1e-3, 3, 1e-7, 1, pull=0.5)
+    else:
+        p = pr.cube3d(16, 1e-3, 3, 1e-7, 1, jitter=0.02, sigma_v=1e-3)
+
+    def us(g):  # best of five: other work on the box only adds
+        return min(g.timed_steps(101)[1] for _ in range(5)) * 1e3
+
+    with GpuFD(p, precision=precision) as g:
+        g.init()
+        own = g.get_tile()
+        assert own[0] == 64 and own[1] > 1
+        before = us(g)
+        tile, chunk, tab = g.autotune_tiles()
+        assert tile in (128, 256, 512) and chunk in (2, 4, 8)
+        tuned, after = g.get_tile(), us(g)
+        g.set_tile(tile)
+        table = us(g)
+        g.set_tile(64)
+        assert g.get_tile() == own
+        progress(f"[gpu]   {own} {before:.2f} us, tuned {tuned} {after:.2f}, "
+                 f"{tile} {table:.2f}")
+        assert tuned[0] in (64, tile)
+        # (the tuner times 6 steps, 4 of the state-based passes)
+        assert after <= 1.15 * before
+    with GpuFD(pr.plate2d(300, 280, 1e-3, 3, 1e-7, 1),
+               precision=precision) as g:
+        assert g.get_tile()[0] != 64
+        with pytest.raises(NlmError):
+            g.set_tile(64)
