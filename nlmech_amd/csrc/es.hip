@@ -1104,12 +1104,16 @@ __global__ __launch_bounds__(256) void k_es_fields(
   put(stress6, S);
 }
 
-// A node field (internal order) in reference order.
+// A node field (internal order) in reference order: nodes lo .. lo + m - 1 of
+// that order.
 __global__ __launch_bounds__(256) void k_out_scalar(
     int64_t n, const double* __restrict__ src,
-    const int32_t* __restrict__ perm, double* __restrict__ dst) {
+    const int32_t* __restrict__ perm, int64_t lo, int64_t m,
+    double* __restrict__ dst) {
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) dst[perm[i]] = src[i];
+  if (i >= n) return;
+  const int64_t j = int64_t(perm[i]) - lo;
+  if (j >= 0 && j < m) dst[j] = src[i];
 }
 
 }  // namespace
@@ -1185,20 +1189,25 @@ extern "C" int nlm_fd_get_node_fields(nlm_ctx* c, double* theta, double* mw) {
   const double* const src[2] = {s.es_theta.as<double>(),
                                 s.es_mw.as<double>()};
   double* const dst[2] = {theta, mw};
-  int rc;
-  if ((rc = reserve(c, s.out, 2 * sizeof(double) * size_t(s.n)))) return rc;
+  // each field in a half of the staging, as many nodes at a time as it holds
+  out_staging(c, 2 * sizeof(double) * size_t(s.n));
+  const int64_t held =
+      std::min(s.n, int64_t(s.out.bytes / (2 * sizeof(double))));
   const unsigned g = unsigned((s.n + 255) / 256);
-  for (int k = 0; k < 2; k++)
-    if (dst[k])
-      hipLaunchKernelGGL(k_out_scalar, dim3(g), dim3(256), 0, c->stream, s.n,
-                         src[k], s.perm_dev.as<int32_t>(),
-                         s.out.as<double>() + k * s.n);
-  NLM_HIP(c, hipGetLastError());
-  for (int k = 0; k < 2; k++)
-    if (dst[k])
-      NLM_HIP(c, hipMemcpyAsync(dst[k], s.out.as<double>() + k * s.n,
-                                sizeof(double) * size_t(s.n),
-                                hipMemcpyDeviceToHost, c->stream));
+  for (int64_t lo = 0; lo < s.n; lo += held) {
+    const int64_t m = std::min(held, s.n - lo);
+    for (int k = 0; k < 2; k++)
+      if (dst[k])
+        hipLaunchKernelGGL(k_out_scalar, dim3(g), dim3(256), 0, c->stream, s.n,
+                           src[k], s.perm_dev.as<int32_t>(), lo, m,
+                           s.out.as<double>() + k * held);
+    NLM_HIP(c, hipGetLastError());
+    for (int k = 0; k < 2; k++)
+      if (dst[k])
+        NLM_HIP(c, hipMemcpyAsync(dst[k] + lo, s.out.as<double>() + k * held,
+                                  sizeof(double) * size_t(m),
+                                  hipMemcpyDeviceToHost, c->stream));
+  }
   NLM_HIP(c, hipStreamSynchronize(c->stream));
   return NLM_OK;
 }

@@ -812,16 +812,19 @@ __global__ __launch_bounds__(256) void k_postproc(
 }
 
 // A node vector (internal order) as the boundary takes it: 3 components per
-// node in reference order, z = 0 in 2D.
+// node in reference order, z = 0 in 2D; nodes lo .. lo + m - 1 of that order.
 template <int DIM>
 __global__ __launch_bounds__(256) void k_out_vec(
     int64_t n, const typename VT<DIM>::T* __restrict__ src,
-    const int32_t* __restrict__ perm, double* __restrict__ dst) {
+    const int32_t* __restrict__ perm, int64_t lo, int64_t m,
+    double* __restrict__ dst) {
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
+  const int64_t j = int64_t(perm[i]) - lo;
+  if (j < 0 || j >= m) return;
   double v[3];
   load3<DIM>(src[i], v);
-  double* const o = dst + 3 * int64_t(perm[i]);
+  double* const o = dst + 3 * j;
   o[0] = v[0];
   o[1] = v[1];
   o[2] = v[2];
@@ -1737,6 +1740,8 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     m.low_dd_f = float(lows * lows);
     m.vex_dd_tol_f = float(6.1e-5 * lows * lows);
   }
+  // (the least the calls that return node fields work with)
+  if ((rc = reserve(c, s.out, kOutMin))) return rc;
   s.unroll = 4;
   if (es_mat) {
     // ElasticState constants (ElasticState.cpp:47-158, volumeCorrection.cpp)
@@ -1996,34 +2001,52 @@ int to_dev_vec(nlm_ctx* c, const double* src, DevBuf& dst) {
   return NLM_OK;
 }
 // Node vectors in reference order to the host: reordered on the device (a
-// host loop over the permutation took 2 to 4 ms a vector of 1e6 nodes), one
-// copy each, one wait.
+// host loop over the permutation took 2 to 4 ms a vector of 1e6 nodes) into
+// the context's staging, all at once or as many nodes at a time as it holds;
+// one wait.
 int from_dev_vecs(nlm_ctx* c, int count, const DevBuf* const* src,
                   double* const* dst) {
   FdState& s = c->fd;
   const size_t vec = sizeof(double) * 3 * size_t(s.n);
-  int rc, used = 0;
+  size_t used = 0;
   for (int k = 0; k < count; k++) used += dst[k] != nullptr;
-  if ((rc = reserve(c, s.out, vec * size_t(std::max(used, 1))))) return rc;
+  out_staging(c, vec * used);
   const int32_t* perm = s.perm_dev.as<int32_t>();
-  double* o = s.out.as<double>();
-  for (int k = 0; k < count; k++) {
-    if (!dst[k]) continue;
+  double* const base = s.out.as<double>();
+  const int64_t held = int64_t(s.out.bytes / (3 * sizeof(double)));
+  auto reorder = [&](const DevBuf& v, int64_t lo, int64_t m, double* o) {
     if (s.dim == 2)
       hipLaunchKernelGGL(k_out_vec<2>, dim3(node_blocks(s)), dim3(256), 0,
-                         c->stream, s.n, src[k]->as<double2>(), perm, o);
+                         c->stream, s.n, v.as<double2>(), perm, lo, m, o);
     else
       hipLaunchKernelGGL(k_out_vec<3>, dim3(node_blocks(s)), dim3(256), 0,
-                         c->stream, s.n, src[k]->as<double4>(), perm, o);
-    o += 3 * s.n;
-  }
-  NLM_HIP(c, hipGetLastError());
-  o = s.out.as<double>();
-  for (int k = 0; k < count; k++) {
-    if (!dst[k]) continue;
-    NLM_HIP(c, hipMemcpyAsync(dst[k], o, vec, hipMemcpyDeviceToHost,
-                              c->stream));
-    o += 3 * s.n;
+                         c->stream, s.n, v.as<double4>(), perm, lo, m, o);
+  };
+  if (held >= int64_t(used) * s.n) {
+    double* o = base;
+    for (int k = 0; k < count; k++)
+      if (dst[k]) {
+        reorder(*src[k], 0, s.n, o);
+        o += 3 * s.n;
+      }
+    NLM_HIP(c, hipGetLastError());
+    o = base;
+    for (int k = 0; k < count; k++)
+      if (dst[k]) {
+        NLM_HIP(c, hipMemcpyAsync(dst[k], o, vec, hipMemcpyDeviceToHost,
+                                  c->stream));
+        o += 3 * s.n;
+      }
+  } else {
+    for (int k = 0; k < count; k++)
+      for (int64_t lo = 0; dst[k] && lo < s.n; lo += held) {
+        const int64_t m = std::min(held, s.n - lo);
+        reorder(*src[k], lo, m, base);
+        NLM_HIP(c, hipGetLastError());
+        NLM_HIP(c, hipMemcpyAsync(dst[k] + 3 * lo, base,
+                                  sizeof(double) * 3 * size_t(m),
+                                  hipMemcpyDeviceToHost, c->stream));
+      }
   }
   NLM_HIP(c, hipStreamSynchronize(c->stream));
   return NLM_OK;
@@ -2239,12 +2262,13 @@ extern "C" int nlm_fd_postproc(nlm_ctx* c, float* Z, float* phi,
   if (s.material != NLM_MATERIAL_RNP_BOND)
     return fail(c, NLM_ERR_INVALID,
                 "nlm_fd_postproc: bond-based material only");
-  // fields in reference order in the context's staging, the outputs copied
-  // from there
-  const size_t n = size_t(s.n);
-  if ((rc = reserve(c, s.out, (sizeof(double) + 2 * sizeof(float)) * n)))
-    return rc;
-  double* const de = s.out.as<double>();
+  // fields in reference order in the context's staging (beyond its bound: in
+  // a buffer of the call), the outputs copied from there
+  const size_t n = size_t(s.n), need = (sizeof(double) + 2 * sizeof(float)) * n;
+  DevBuf own;
+  if (need <= kOutMax) out_staging(c, need);
+  if (s.out.bytes < need && (rc = alloc(c, own, need))) return rc;
+  double* const de = own.p ? own.as<double>() : s.out.as<double>();
   float* const dz = reinterpret_cast<float*>(de + n);
   float* const dp = dz + n;
   const int32_t* const perm = s.perm_dev.as<int32_t>();

@@ -228,7 +228,8 @@ struct FdState {
   int graph_chunk = 0;
   int graph_cur = -1;  // value of cur when the graph was captured
   DevBuf out;    // device staging of the calls that return node fields, in
-                 // reference order; grows to the largest call
+                 // reference order; kOutMin at setup, grows to the largest
+                 // call, kOutMax at most
   DevBuf bctab;  // BcTable
   BcTable bc_host{};
   std::vector<uint8_t> fix_host;
@@ -371,6 +372,23 @@ inline int alloc(nlm_ctx* c, DevBuf& b, size_t bytes) {
 // A workspace of at least `bytes` (kept when it is large enough).
 inline int reserve(nlm_ctx* c, DevBuf& b, size_t bytes) {
   return b.p && b.bytes >= bytes ? NLM_OK : alloc(c, b, bytes);
+}
+
+// Grows the staging of the node-field calls towards `bytes`, to kOutMax at
+// most; without the memory for it the staging stays as it is.
+constexpr size_t kOutMin = size_t(1) << 20, kOutMax = size_t(1) << 27;
+inline void out_staging(nlm_ctx* c, size_t bytes) {
+  DevBuf& b = c->fd.out;
+  if (bytes > kOutMax) bytes = kOutMax;
+  if (b.bytes >= bytes) return;
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  b.release();
+  b.p = p;
+  b.bytes = bytes;
 }
 
 // Drops the previous model's tangent, preconditioner, colors, aggregates and
