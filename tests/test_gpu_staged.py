@@ -205,6 +205,10 @@ def test_separated_bodies_3d(oracle, precision, gap):
 # changes (slices of 64 nodes: 256, 800, 2500, 3000), through the whole step:
 # the FP64 modes agree with the oracle, and a tile set by hand (with its own
 # split) gives the same bits, because split rows are added in list order.
+# FP32-force: the tiles pass between k_fd_st's split rows and the whole-row
+# kernels, each within that mode's bar of the oracle, 1e-6 of the displacement
+# and (its displacements being off by that much at the critical stretch) 1e-3
+# of the broken bonds.
 @pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
                                        NLM_PREC_FP32_FORCE],
                          ids=["exact", "fp64", "fp32"])
@@ -227,11 +231,15 @@ def test_split_rows(oracle, precision, shape):
             g.init()
             g.step(12)
             outs.append(g.get_state() + (g.get_bonds(),))
-    u, _, _, bonds = outs[0]
+    ref_bonds = o.get_bonds()
+    assert ref_bonds.sum() > 0
     if precision == NLM_PREC_FP32_FORCE:
-        assert np.linalg.norm(u - ur) <= 1e-6 * np.linalg.norm(ur)
+        for out in outs:
+            assert np.linalg.norm(out[0] - ur) <= 1e-6 * np.linalg.norm(ur)
+            assert (out[3] != ref_bonds).sum() <= 1e-3 * ref_bonds.sum()
         return
-    assert np.array_equal(bonds, o.get_bonds()) and bonds.sum() > 0
+    u, _, _, bonds = outs[0]
+    assert np.array_equal(bonds, ref_bonds)
     assert np.linalg.norm(u - ur) <= 1e-13 * np.linalg.norm(ur)
     for other in outs[1:]:
         for a, b in zip(outs[0], other):
@@ -251,11 +259,13 @@ def test_split_rows_3d(oracle, precision, shape):
     x, vol = pr.grid3d(*shape, h, jitter=0.02, seed=4)
     p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
                    dt=1e-7, nsteps=1, material=pr.rnp_material(dim=3),
-                   v0=np.random.default_rng(3).normal(size=x.shape))
+                   v0=4.0 * np.random.default_rng(3).normal(size=x.shape))
     o = oracle.OracleFD(p)
     o.init()
     o.step(4)
     u_ref = o.get_state()[0]
+    broken = o.get_bonds().sum()
+    assert broken > 0  # (at 1 m/s no bond breaks in 4 steps)
     with GpuFD(p, precision=precision) as g:
         g.init()
         g.step(4)
@@ -263,8 +273,8 @@ def test_split_rows_3d(oracle, precision, shape):
     f32 = precision == NLM_PREC_FP32_FORCE
     assert (np.linalg.norm(u - u_ref) <=
             (1e-6 if f32 else 1e-13) * np.linalg.norm(u_ref))
-    if not f32:
-        assert np.array_equal(bonds, o.get_bonds())
+    diff = (bonds != o.get_bonds()).sum()
+    assert diff <= (1e-3 * broken if f32 else 0)
 
 
 @pytest.mark.parametrize("precision", [NLM_PREC_FP64_EXACT, NLM_PREC_FP64,
