@@ -878,7 +878,12 @@ int es_autotune(nlm_ctx* c, int* chosen, double* best_us, double* us3) {
   NLM_HIP(c, hipEventCreate(&e0));
   NLM_HIP(c, hipEventCreate(&e1));
   const int reps = 4;
+  rc = tune_warm_up(c, e0, e1, [&] {
+    for (int r = 0; r < reps; r++)
+      launch_any(c, KIND_CD, false, s.time, s.time + s.dt, 4);
+  });
   for (int k : {1, 0, 2}) {
+    if (rc) break;
     const int U = cands[k];
     // (k_es_force_st has one width: its one time for every width)
     if (U != 4 && st_pass(c, s, true)) {
@@ -906,6 +911,7 @@ int es_autotune(nlm_ctx* c, int* chosen, double* best_us, double* us3) {
   // restore pass 1's outputs of the current state
   NLM_HIP(c, hipMemcpyAsync(s.es_theta.p, th_save.p, s.es_theta.bytes,
                             hipMemcpyDeviceToDevice, c->stream));
+  if (rc) return rc;
   NLM_HIP(c, hipGetLastError());
   NLM_HIP(c, hipStreamSynchronize(c->stream));
   s.unroll = pick;

@@ -2433,6 +2433,11 @@ int time_chunks(nlm_ctx* c, double us[3]) {
   const int reps = 6;
   const bool st = staged_step(s);
   us[0] = us[2] = 0.;
+  if ((rc = tune_warm_up(c, e0, e1, [&] {
+         for (int r = 0; r < reps; r++)
+           launch_mode<DIM, KIND_CD, false>(c, a, s.time, s.time + s.dt, 4);
+       })))
+    return rc;
   for (int k : {1, 0, 2}) {
     const int U = cands[k];
     if (s.precision == NLM_PREC_FP64_EXACT && U != 4) continue;
