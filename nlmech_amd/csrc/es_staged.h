@@ -472,10 +472,14 @@ __global__ __launch_bounds__(512) void k_es_force_st(
           dd = d == 0 ? X * X : dd + X * X;
         }
         const RootRcp oy = root_rcp(yy);
-        const double lx = root_rcp(dd).r;
+        double lx = root_rcp(dd).r;
         double c = lx > lowb ? quot(e.m.check_up - lx, e.m.h, e.m.rcp_h) : 1.;
-        if (__builtin_amdgcn_ballot_w64(fabs(lx - lowb) <= vtol) != 0ull)
-          if (fabs(lx - lowb) <= vtol && k0 + q < len) c = corr_exact();
+        // (inside the band: the root of 0, a NaN, too)
+        if (__builtin_amdgcn_ballot_w64(!(fabs(lx - lowb) > vtol)) != 0ull)
+          if (!(fabs(lx - lowb) > vtol) && k0 + q < len) {
+            c = corr_exact();
+            lx = dd == 0. ? 0. : lx;
+          }
         const double thj = n.v[DIM == 2 ? 7 : 8];
         const double es_i = quot(thi * lx, 3., kThird);
         const double es_j = quot(thj * lx, 3., kThird);

@@ -168,3 +168,29 @@ def test_force(oracle, mode, shape):
     bar = {NLM_PREC_FP64_EXACT: 1e-13, NLM_PREC_FP64: 1e-11,
            NLM_PREC_FP32_FORCE: 2e-6}[mode]
     assert np.linalg.norm(f - ref) <= bar * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_coincident_nodes(oracle, dim):
+    """Exact mode, no breaking: two nodes at one place that move apart.  The
+    bond's reference length 0 is exact, its force that of the oracle."""
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] staged state-based coincident nodes {dim}D")
+    h = 1e-3
+    if dim == 2:
+        p = pr.with_(plate(9, 8), material=pr.es_material(dim=2, sc=-1.0))
+    else:
+        p = pr.cube3d(7, h, 3, 1e-7, 1, ny=6, nz=5, jitter=0.02, sc=-1.0)
+    p.x[31] = p.x[30]
+    u = np.zeros((p.n, 3))
+    u[:, :dim] = np.random.default_rng(6).normal(scale=1e-6, size=(p.n, dim))
+    o = oracle.OracleES(p)
+    o.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+    o.compute_forces()
+    ref = o.get_state()[2]
+    assert np.all(np.isfinite(ref))
+    with GpuFD(p, precision=NLM_PREC_FP64_EXACT) as g:
+        g.set_state(u=u, v=np.zeros_like(u), f=np.zeros_like(u))
+        g.compute_forces()
+        f = g.get_state()[2]
+    assert np.linalg.norm(f - ref) <= 1e-13 * np.linalg.norm(ref)
