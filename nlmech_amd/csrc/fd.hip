@@ -1259,8 +1259,10 @@ size_t halo_rec_bytes(int dim, int precision, bool nofail) {
 //     7.3 / 7.8, 256 x 1 9.5 / 10.4; 200 x 190 (594): 64 x 4 11.8 / 14.0,
 //     256 x 1 13.1 / 15.4; 333 x 217 (1130), FP64: 64 x 4 13.0, 256 x 1 11.5;
 //   2D FP32-force, 157: 64 x 8 5.4, 256 x 1 7.8; 594: 64 x 4 7.2, 256 x 1
-//     10.4; 400 x 397 (2482): 128 x 2 13.5, 256 x 1 14.5; 619 x 451 (4362):
-//     128 x 2 23.1, 256 x 1 20.4;
+//     10.4; 128 x 2 against 256 x 1 at horizons of 3 h / 4 h: 889 slices 7.2 /
+//     9.1 against 7.8 / 10.5; 2557 9.7 / 13.5 against 10.4 / 14.8; 2608 12.3 /
+//     18.5 against 10.4 / 14.9 (the device holds five workgroups a CU, 2560
+//     slices); 619 x 451 (4362): 23.1 against 20.4 at 4 h;
 //   3D FP64 / exact, 20 x 18 x 22 (124): 64 x 8 11.6 / 14.0, 256 x 1 24 / 32;
 //     41 x 37 x 45 (1067): 64 x 8 33 / 42, 128 x 1 49 / 67; 72 x 64 x 56
 //     (4032): 64 x 4 83 / 107, 256 x 1 65 / 91, 128 x 1 97 / 138, 128 x 4
@@ -1276,7 +1278,7 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
   if (nslices <= 256) return {64, 8};
   if (nslices <= 800) return {64, 4};
   if (dim == 2) {
-    if (f32 && nslices <= 3000) return {128, 2};
+    if (f32 && nslices <= 2560) return {128, 2};
     return {256, 1};
   }
   if (f32) return {nslices <= 2500 ? 128 : 256, 2};

@@ -202,7 +202,7 @@ def test_separated_bodies_3d(oracle, precision, gap):
 
 
 # Trajectories over the sizes at which the rule for tiles and split rows
-# changes (slices of 64 nodes: 256, 800, 2500, 3000), through the whole step:
+# changes (slices of 64 nodes: 256, 800, 2500, 2560), through the whole step:
 # the FP64 modes agree with the oracle, and a tile set by hand (with its own
 # split) gives the same bits, because split rows are added in list order.
 # FP32-force: the tiles pass between k_fd_st's split rows and the whole-row
@@ -357,3 +357,23 @@ def test_autotuner_keeps_a_faster_setup(precision, kind):
         assert g.get_tile()[0] != 64
         with pytest.raises(NlmError):
             g.set_tile(64)
+
+
+def step_us(p, precision):
+    """Microseconds per step, best of eight: other work on the box only adds."""
+    from nlmech_amd.engine import GpuFD
+    with GpuFD(p, precision=precision) as g:
+        g.init()
+        return min(g.timed_steps(101)[1] for _ in range(8)) * 1e3
+
+
+@pytest.mark.parametrize("ratio", [3, 4])
+def test_time_across_the_last_split(ratio):
+    """2D FP32-force at 2557 and 2608 slices, the last split rows and the first
+    whole rows: 2 % more nodes, no jump in time (split rows at 2608: a second
+    round of workgroups, 1.27 and 1.37 times)."""
+    progress(f"[gpu] time across the last split, horizon {ratio} h")
+    us = [step_us(pr.plate2d(s, s - 3, 1e-3, ratio, 1e-7, 1),
+                  NLM_PREC_FP32_FORCE) for s in (406, 410)]
+    progress(f"[gpu]   {us[0]:.2f} {us[1]:.2f} us")
+    assert us[1] <= 1.18 * us[0]
