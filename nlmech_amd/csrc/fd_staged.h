@@ -39,7 +39,9 @@ namespace nlm {
 
 // Halo record of the FP64 modes: position, displacement and the volume (FP64
 // mode: times c4, and J when constant).  10- and 14-dword strides spread
-// record starts over 32 of the 64 LDS banks.
+// record starts over 32 of the 64 LDS banks; with flags 12 and 18 dwords over
+// 16 and 32 (3D without padding, 16 dwords, over 4: 56 x 57 x 60 nodes with a
+// no-fail region, FP64 146 instead of 69 us a step, exact 157 instead of 140).
 template <int DIM, bool NOFAIL>
 struct alignas(8) StRec64 {
   double x[DIM];
@@ -51,7 +53,7 @@ struct alignas(8) StRec64<DIM, true> {
   double x[DIM];
   double u[DIM];
   double c;
-  uint32_t flags, pad;
+  uint32_t flags, pad[DIM == 3 ? 3 : 1];
 };
 
 // FP32-force mode, 2D: the scaled displacement in FP64, the scaled
@@ -428,9 +430,13 @@ inline size_t st_round_bytes(int dim, int precision, int tile, int parts) {
 
 // Bytes of a halo record.
 inline size_t st_rec_bytes(int dim, int precision, bool nofail) {
-  return (precision == kModeFp32 ? sizeof(StRec32<3, false>)
-                                 : size_t(2 * dim + 1) * 8) +
-         (nofail && !(dim == 2 && precision == kModeFp32) ? 8 : 0);
+  const bool f32 = precision == kModeFp32;
+  if (dim == 2)
+    return f32 ? sizeof(StRec32<2, false>)
+               : nofail ? sizeof(StRec64<2, true>) : sizeof(StRec64<2, false>);
+  if (f32)
+    return nofail ? sizeof(StRec32<3, true>) : sizeof(StRec32<3, false>);
+  return nofail ? sizeof(StRec64<3, true>) : sizeof(StRec64<3, false>);
 }
 
 // Launch of the staged kernel for the configured tile (fd_st2.hip,

@@ -377,3 +377,18 @@ def test_time_across_the_last_split(ratio):
                   NLM_PREC_FP32_FORCE) for s in (406, 410)]
     progress(f"[gpu]   {us[0]:.2f} {us[1]:.2f} us")
     assert us[1] <= 1.18 * us[0]
+
+
+def test_time_of_no_fail_records():
+    """3D FP64: the records with no-fail flags cost about what they carry (a
+    stride of 16 dwords: 2.3 times the step without the region)."""
+    progress("[gpu] time of no-fail records")
+    h = 1e-3
+    x, vol = pr.grid3d(56, 57, 60, h, jitter=0.0, seed=4)
+    p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3 * h, h=h,
+                   dt=1e-8, nsteps=1, material=pr.rnp_material(dim=3))
+    interior = np.ones(p.n, np.uint8)
+    interior[:p.n // 10] = 0
+    us = [step_us(q, NLM_PREC_FP64) for q in (p, pr.with_(p, interior=interior))]
+    progress(f"[gpu]   {us[0]:.1f} {us[1]:.1f} us")
+    assert us[1] <= 1.4 * us[0]
