@@ -1325,8 +1325,10 @@ int stage_parts(int dim, int precision, int64_t nslices, int tile) {
   if (tile == r.tile) return r.parts;
   if (precision != NLM_PREC_FP32_FORCE) {
     if (tile >= 256) return 1;
-    // (3D: 256-node tiles that do not fit fall to 128 x 4)
-    return std::max(r.parts == 1 && dim == 3 ? 4 : 1,
+    // (3D: 256-node tiles that do not fit fall to 128 x 4, and those to 64 x 8:
+    // 56 x 57 x 60 nodes, horizon 4 h, FP64 / exact 153 / 213 us, 64 x 4 223 /
+    // 294, direct gathers 213 / 345)
+    return std::max(r.parts == 1 && dim == 3 ? 512 / tile : 1,
                     std::min(r.parts, 512 / tile));
   }
   return std::max(1, std::min(r.parts, 512 / tile));

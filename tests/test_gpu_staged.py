@@ -392,3 +392,19 @@ def test_time_of_no_fail_records():
     us = [step_us(q, NLM_PREC_FP64) for q in (p, pr.with_(p, interior=interior))]
     progress(f"[gpu]   {us[0]:.1f} {us[1]:.1f} us")
     assert us[1] <= 1.4 * us[0]
+
+
+def test_time_of_wide_horizons():
+    """3D FP64, horizon 4 h, whose halos fit tiles of 64 nodes: a large block
+    costs no more a node than a small one (rows shared by four wavefronts and
+    not eight: 1.33 times)."""
+    progress("[gpu] time of wide horizons in 3D")
+    h = 1e-3
+    us = []
+    for shape in ((40, 36, 44), (56, 57, 60)):
+        x, vol = pr.grid3d(*shape, h, jitter=0.0, seed=4)
+        p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=4 * h, h=h,
+                       dt=1e-8, nsteps=1, material=pr.rnp_material(dim=3))
+        us.append(step_us(p, NLM_PREC_FP64) / p.n * 1e3)
+    progress(f"[gpu]   {us[0]:.3f} {us[1]:.3f} ns a node")
+    assert us[1] <= 1.15 * us[0]
