@@ -842,6 +842,11 @@ size_t es_halo_lds_bytes(int precision, int64_t halo_max) {
   return size_t(halo_max + 1) * es_record_bytes(precision);
 }
 
+size_t es_force_lds(int precision, int64_t halo_max, int tile, int parts,
+                    size_t lds_max) {
+  return es_st_lds(3, precision, halo_max, tile, parts, true, lds_max).bytes;
+}
+
 void es_launch_force(nlm_ctx* c, bool base_f, double t) {
   launch_any(c, KIND_FORCE, base_f, t, t, 4);
 }

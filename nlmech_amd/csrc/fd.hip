@@ -1299,6 +1299,14 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
 //     46.7, 128 x 4 72.5 / 47.9 / 30.9, before 96.4 / 56.3 / 46.0; 80 x 80 x
 //     80 (8000): 256 x 1 317 / 241 / 166, 128 x 4 465 / 261 / 154, 256 x 2
 //     499 / 338 / 140, before 523 / 269 / 166.
+// 3D FP64 above 2500 slices: 256 x 1, but 128 x 4 where a CU's LDS holds one
+// workgroup of the force pass at 256 x 1 (four wavefronts; halos of blocks that
+// the Morton order cuts unevenly) and two at 128 x 4.  256 x 1 / 128 x 4 /
+// before: 65 x 65 x 65 (4292) 201 / 158 / 261, 70 x 70 x 70 239 / 191 / 202, 90
+// x 90 x 90 562 / 408 / 643; one at either, 74 x 75 x 76 279 / 309 / 369; two
+// at 256 x 1, 64 x 64 x 64 138 / 147 / 149, 60 x 60 x 60 at a horizon of 2 h 52
+// / 59 / 56.
+constexpr StageRule kEs64Split{128, 4};
 StageRule es_stage_rule(int dim, int precision, int64_t nslices) {
   const bool f32 = precision == NLM_PREC_FP32_FORCE;
   if (nslices <= 400) return {64, 8};
@@ -1307,11 +1315,14 @@ StageRule es_stage_rule(int dim, int precision, int64_t nslices) {
     return f32 ? StageRule{128, 2} : StageRule{256, 1};
   }
   if (f32) return nslices <= 2500 ? StageRule{128, 4} : StageRule{256, 2};
-  if (precision == NLM_PREC_FP64 && nslices <= 2500) return {128, 4};
+  if (precision == NLM_PREC_FP64 && nslices <= 2500) return kEs64Split;
   return {256, 1};
 }
-// Parts at a tile set by hand: at most 512 threads a workgroup.
+// Parts at a tile set by hand: at most 512 threads a workgroup; 3D FP64: whole
+// rows from 256 nodes on (80 x 80 x 80: 256 x 2 338 us, 256 x 1 241).
 int es_stage_parts(int dim, int precision, int64_t nslices, int tile) {
+  if (dim == 3 && precision == NLM_PREC_FP64)
+    return tile >= 256 ? 1 : 512 / tile;
   const StageRule r = es_stage_rule(dim, precision, nslices);
   return std::max(1, std::min(r.parts, 512 / tile));
 }
@@ -1425,13 +1436,31 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   else rule = es_stage_rule(dim, p->precision, (n + 63) / 64);
   int tile = rule.tile;
   build_layout(dim, n, p->x, mesh_h, h_row, h_col, tile / 64, L);
-  bool fits = (L.halo_max + 1) * int64_t(bond3 ? rec : kHaloRecBudget) <=
-              64 * 1024;
-  while (bond3 && !fits && tile > 64) {
-    tile /= 2;
+  auto halos = [&](int bn) {
+    tile = bn;
     L.nblocks = (L.nslices * 64 + tile - 1) / tile;
     build_halos(n, L.nslices, L.sl_ptr.data(), L.colS.data(), tile / 64,
                 L.halo_ptr, L.halo, L.colL, L.halo_max);
+  };
+  if (es_mat && dim == 3 && p->precision == NLM_PREC_FP64 && tile == 256) {
+    int lds_max = 0;
+    NLM_HIP(c, hipDeviceGetAttribute(&lds_max,
+                                     hipDeviceAttributeMaxSharedMemoryPerBlock,
+                                     c->device));
+    auto need = [&](const StageRule& r) {
+      return es_force_lds(p->precision, L.halo_max, r.tile, r.parts,
+                          size_t(lds_max));
+    };
+    if (2 * need(rule) > size_t(lds_max)) {
+      halos(kEs64Split.tile);
+      if (2 * need(kEs64Split) <= size_t(lds_max)) rule = kEs64Split;
+      else halos(rule.tile);
+    }
+  }
+  bool fits = (L.halo_max + 1) * int64_t(bond3 ? rec : kHaloRecBudget) <=
+              64 * 1024;
+  while (bond3 && !fits && tile > 64) {
+    halos(tile / 2);
     fits = (L.halo_max + 1) * int64_t(rec) <= 64 * 1024;
   }
   s.perm_host = L.perm;

@@ -249,6 +249,9 @@ void fd_launch_force(nlm_ctx* c, bool base_f, double t);
 int es_prepare(nlm_ctx* c);
 // LDS bytes of a staged state-based launch for a halo of halo_max nodes
 size_t es_halo_lds_bytes(int precision, int64_t halo_max);
+// The same of the 3D force pass k_es_force_st
+size_t es_force_lds(int precision, int64_t halo_max, int tile, int parts,
+                    size_t lds_max);
 void es_launch_force(nlm_ctx* c, bool base_f, double t);
 void es_launch_fused(nlm_ctx* c, double tf, double tn);
 // fused pass pair reading the step times from tdev (graph capture)

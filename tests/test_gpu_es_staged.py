@@ -194,3 +194,23 @@ def test_coincident_nodes(oracle, dim):
         g.compute_forces()
         f = g.get_state()[2]
     assert np.linalg.norm(f - ref) <= 1e-13 * np.linalg.norm(ref)
+
+
+def test_time_of_uneven_halos():
+    """3D FP64: a block that the Morton order cuts unevenly (70^3) costs no
+    more a node than one it cuts evenly, 64^3 (on tiles of 256 nodes, one a
+    CU: 1.33 times), and takes the same steps at every tile."""
+    from nlmech_amd.engine import GpuFD
+    progress("[gpu] time of uneven halos")
+    us, state = [], []
+    for n in (64, 70):
+        p = pr.cube3d(n, 1e-3, 3, 1e-7, 1, jitter=0.0, sigma_v=1e-3)
+        with GpuFD(p, precision=NLM_PREC_FP64) as g:
+            g.init()
+            us.append(min(g.timed_steps(21)[1] for _ in range(8)) * 1e6 / p.n)
+    for tile in (None, 128, 256):
+        state.append(run(p, NLM_PREC_FP64, 3, tile))
+    progress(f"[gpu]   {us[0]:.3f} {us[1]:.3f} ns a node")
+    assert us[1] <= 1.2 * us[0]
+    for other in state[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(state[0], other))
