@@ -1298,7 +1298,9 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
 //     15.9, before 92 / 51 / 43; 47 x 39 x 33 (945): 256 x 1 65.3 / 53.2 /
 //     46.7, 128 x 4 72.5 / 47.9 / 30.9, before 96.4 / 56.3 / 46.0; 80 x 80 x
 //     80 (8000): 256 x 1 317 / 241 / 166, 128 x 4 465 / 261 / 154, 256 x 2
-//     499 / 338 / 140, before 523 / 269 / 166.
+//     499 / 338 / 140, before 523 / 269 / 166; short rows (row: bonds a node),
+//     60 x 60 x 60 at a horizon of 2 h (25), FP32-force: 256 x 1 39.7, 256 x 2
+//     41.9, before 39.9.
 // 3D FP64 above 2500 slices: 256 x 1, but 128 x 4 where a CU's LDS holds one
 // workgroup of the force pass at 256 x 1 (four wavefronts; halos of blocks that
 // the Morton order cuts unevenly) and two at 128 x 4.  256 x 1 / 128 x 4 /
@@ -1307,23 +1309,26 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
 // at 256 x 1, 64 x 64 x 64 138 / 147 / 149, 60 x 60 x 60 at a horizon of 2 h 52
 // / 59 / 56.
 constexpr StageRule kEs64Split{128, 4};
-StageRule es_stage_rule(int dim, int precision, int64_t nslices) {
+StageRule es_stage_rule(int dim, int precision, int64_t nslices,
+                        int64_t row) {
   const bool f32 = precision == NLM_PREC_FP32_FORCE;
   if (nslices <= 400) return {64, 8};
   if (dim == 2) {
     if (nslices <= 2500) return {64, 4};
     return f32 ? StageRule{128, 2} : StageRule{256, 1};
   }
-  if (f32) return nslices <= 2500 ? StageRule{128, 4} : StageRule{256, 2};
+  if (f32 && nslices <= 2500) return {128, 4};
+  if (f32) return {256, row < 32 ? 1 : 2};
   if (precision == NLM_PREC_FP64 && nslices <= 2500) return kEs64Split;
   return {256, 1};
 }
 // Parts at a tile set by hand: at most 512 threads a workgroup; 3D FP64: whole
 // rows from 256 nodes on (80 x 80 x 80: 256 x 2 338 us, 256 x 1 241).
-int es_stage_parts(int dim, int precision, int64_t nslices, int tile) {
+int es_stage_parts(int dim, int precision, int64_t nslices, int64_t row,
+                   int tile) {
   if (dim == 3 && precision == NLM_PREC_FP64)
     return tile >= 256 ? 1 : 512 / tile;
-  const StageRule r = es_stage_rule(dim, precision, nslices);
+  const StageRule r = es_stage_rule(dim, precision, nslices, row);
   return std::max(1, std::min(r.parts, 512 / tile));
 }
 
@@ -1433,7 +1438,7 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
   const size_t rec = halo_rec_bytes(dim, p->precision, has_nofail);
   StageRule rule{256, 1};
   if (!es_mat) rule = stage_rule(dim, p->precision, (n + 63) / 64);
-  else rule = es_stage_rule(dim, p->precision, (n + 63) / 64);
+  else rule = es_stage_rule(dim, p->precision, (n + 63) / 64, nnz / n);
   int tile = rule.tile;
   build_layout(dim, n, p->x, mesh_h, h_row, h_col, tile / 64, L);
   auto halos = [&](int bn) {
@@ -2620,7 +2625,7 @@ int retile(nlm_ctx* c, int bn) {
     return rc;
   s.halo_max = hmax;
   s.tile = bn;
-  s.parts = es ? es_stage_parts(s.dim, s.precision, ns, bn)
+  s.parts = es ? es_stage_parts(s.dim, s.precision, ns, s.nnz / n, bn)
                : stage_parts(s.dim, s.precision, ns, bn);
   if (es) es_set_quantum(s.es, org_range);
   return NLM_OK;

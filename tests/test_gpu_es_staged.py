@@ -214,3 +214,14 @@ def test_time_of_uneven_halos():
     assert us[1] <= 1.2 * us[0]
     for other in state[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(state[0], other))
+
+
+def test_short_rows_are_not_split():
+    """3D FP32-force above 2500 slices: rows of 25 bonds keep one wavefront (two
+    cost more than they gain), rows of 81 have two."""
+    from nlmech_amd.engine import GpuFD
+    progress("[gpu] short rows are not split")
+    for ratio, parts in ((2, 1), (3, 2)):
+        p = pr.cube3d(56, 1e-3, ratio, 1e-7, 1, jitter=0.0)
+        with GpuFD(p, precision=NLM_PREC_FP32_FORCE) as g:
+            assert g.get_tile() == (256, parts)
