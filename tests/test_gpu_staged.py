@@ -408,3 +408,31 @@ def test_time_of_wide_horizons():
         us.append(step_us(p, NLM_PREC_FP64) / p.n * 1e3)
     progress(f"[gpu]   {us[0]:.3f} {us[1]:.3f} ns a node")
     assert us[1] <= 1.15 * us[0]
+
+
+@pytest.mark.parametrize("kind", ["bond", "state"])
+def test_time_of_setup(kind):
+    """A model whose tile follows from its halos (3D FP64: 256 nodes do not
+    fit, 128 do) is set up about as fast as one of one tile (the halos of both
+    tiles sorted by one thread: 1.9 times)."""
+    import time
+
+    from nlmech_amd.engine import GpuFD
+    progress(f"[gpu] time of setup {kind}")
+    x, vol = pr.grid3d(60, 60, 60, 1e-3, jitter=0.0, seed=4)
+    mat = pr.rnp_material if kind == "bond" else pr.es_material
+    p = pr.Problem(name="block", dim=3, x=x, vol=vol, horizon=3e-3, h=1e-3,
+                   dt=1e-8, nsteps=1, material=mat(dim=3))
+    ms, tiles = [], []
+    for precision in (NLM_PREC_FP32_FORCE, NLM_PREC_FP64):
+        best = 1e9
+        for _ in range(4):
+            t = time.perf_counter()
+            with GpuFD(p, precision=precision) as g:
+                best = min(best, time.perf_counter() - t)
+                tile = g.get_tile()[0]
+        ms.append(1e3 * best)
+        tiles.append(tile)
+    progress(f"[gpu]   {ms[0]:.0f} {ms[1]:.0f} ms")
+    assert tiles == [256, 128]
+    assert ms[1] <= 1.5 * ms[0]
