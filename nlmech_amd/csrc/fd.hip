@@ -1229,17 +1229,19 @@ std::vector<uint16_t> staged_entries(const std::vector<uint16_t>& colL,
                                      int64_t nslices, const uint16_t* rowlen,
                                      int64_t n) {
   std::vector<uint16_t> out(colL.size(), 0);
-  for (int64_t sl = 0; sl < nslices; sl++) {
-    const int64_t e0 = sl_ptr[sl];
-    const int64_t width = (sl_ptr[sl + 1] - e0) / 64;
-    for (int64_t k = 0; k < width; k++)
-      for (int lane = 0; lane < 64; lane++) {
-        const int64_t e = e0 + 64 * k + lane, a = sl * 64 + lane;
-        if (a < n && k < int64_t(rowlen[a]))
-          out[size_t(e)] =
-              uint16_t((uint32_t(colL[size_t(e)]) + 1u) * uint32_t(rec));
-      }
-  }
+  parallel_chunks(nslices, [&](int64_t s0, int64_t s1) {
+    for (int64_t sl = s0; sl < s1; sl++) {
+      const int64_t e0 = sl_ptr[sl];
+      const int64_t width = (sl_ptr[sl + 1] - e0) / 64;
+      for (int64_t k = 0; k < width; k++)
+        for (int lane = 0; lane < 64; lane++) {
+          const int64_t e = e0 + 64 * k + lane, a = sl * 64 + lane;
+          if (a < n && k < int64_t(rowlen[a]))
+            out[size_t(e)] =
+                uint16_t((uint32_t(colL[size_t(e)]) + 1u) * uint32_t(rec));
+        }
+    }
+  }, 512);
   return out;
 }
 
@@ -1709,27 +1711,33 @@ extern "C" int nlm_fd_setup(nlm_ctx* c, const nlm_fd_problem* p) {
     std::vector<unsigned long long> vw(size_t(nent / 64 + 8), 0ull);
     if (!es_mat) {
       const double tol = 3e-5 * m.low_band;
-      for (int64_t sl = 0; sl < L.nslices; sl++) {
-        const int64_t e0 = L.sl_ptr[sl];
-        const int64_t width = (L.sl_ptr[sl + 1] - e0) / 64;
-        for (int64_t k = 0; k < width; k++) {
-          unsigned long long word = 0ull;
-          for (int lane = 0; lane < 64; lane++) {
-            const int64_t a = sl * 64 + lane;
-            if (a >= n || k >= int64_t(L.rowlen[a])) continue;
-            const int64_t g = L.colS[e0 + 64 * k + lane];
-            double d2 = 0.;
-            for (int d = 0; d < dim; d++) {
-              const double e = hx[g * stride + d] - hx[a * stride + d];
-              d2 += e * e;
-              bond_max = std::max(bond_max, std::fabs(e));
+      std::mutex mu;
+      parallel_chunks(L.nslices, [&](int64_t s0, int64_t s1) {
+        double longest = 0.;
+        for (int64_t sl = s0; sl < s1; sl++) {
+          const int64_t e0 = L.sl_ptr[sl];
+          const int64_t width = (L.sl_ptr[sl + 1] - e0) / 64;
+          for (int64_t k = 0; k < width; k++) {
+            unsigned long long word = 0ull;
+            for (int lane = 0; lane < 64; lane++) {
+              const int64_t a = sl * 64 + lane;
+              if (a >= n || k >= int64_t(L.rowlen[a])) continue;
+              const int64_t g = L.colS[e0 + 64 * k + lane];
+              double d2 = 0.;
+              for (int d = 0; d < dim; d++) {
+                const double e = hx[g * stride + d] - hx[a * stride + d];
+                d2 += e * e;
+                longest = std::max(longest, std::fabs(e));
+              }
+              if (d2 == 0. || std::fabs(std::sqrt(d2) - m.low_band) <= tol)
+                word |= 1ull << lane;
             }
-            if (d2 == 0. || std::fabs(std::sqrt(d2) - m.low_band) <= tol)
-              word |= 1ull << lane;
+            vw[size_t(e0 / 64 + k)] = word;
           }
-          vw[size_t(e0 / 64 + k)] = word;
         }
-      }
+        std::lock_guard<std::mutex> lock(mu);
+        bond_max = std::max(bond_max, longest);
+      }, 512);
     }
     if ((rc = up(s.vexw, vw.data(), sizeof(unsigned long long) * vw.size())))
       return rc;

@@ -21,7 +21,6 @@
 #include <cmath>
 #include <cstdint>
 #include <numeric>
-#include <thread>
 #include <vector>
 
 #include "layout.h"
@@ -46,23 +45,6 @@ uint64_t spread3(uint64_t v) {  // 21 bits -> every 3rd bit
   v = (v | (v << 4)) & 0x10c30c30c30c30c3ull;
   v = (v | (v << 2)) & 0x1249249249249249ull;
   return v;
-}
-
-// Runs body(lo, hi) over [0, count) split into contiguous chunks, one per
-// host thread (at most 16); fewer than `least` items stay on the caller's.
-template <class F>
-void parallel_chunks(int64_t count, F body, int64_t least = 4096) {
-  int64_t nt = int64_t(std::thread::hardware_concurrency());
-  nt = std::max<int64_t>(1, std::min<int64_t>(nt, 16));
-  if (count < least) nt = 1;
-  const int64_t chunk = (count + nt - 1) / nt;
-  std::vector<std::thread> th;
-  for (int64_t t = 0; t < nt; t++) {
-    const int64_t lo = t * chunk, hi = std::min(count, lo + chunk);
-    if (lo >= hi) break;
-    th.emplace_back([=, &body] { body(lo, hi); });
-  }
-  for (auto& x : th) x.join();
 }
 
 // The distinct node ids of a block and their positions (open addressing, at
