@@ -61,6 +61,43 @@ extern "C" int nlm_ctx_create(nlm_ctx** out, int device) {
   return NLM_OK;
 }
 
+namespace nlm {
+
+// Up to kOutMin bytes through pinned memory, one device copy for all: a copy to
+// pageable memory costs about 15 us (three vectors of 810 nodes, get_state:
+// 70 us with a copy each, 32 us with one).
+int outputs_to_host(nlm_ctx* c, const void* base, int count, void* const* dst,
+                    const size_t* bytes) {
+  size_t total = 0;
+  for (int k = 0; k < count; k++) total += bytes[k];
+  void*& host = c->fd.out_host;
+  if (total <= kOutMin && !host &&
+      hipHostMalloc(&host, kOutMin, hipHostMallocDefault) != hipSuccess) {
+    host = nullptr;
+    (void)hipGetLastError();
+  }
+  const bool pinned = total > 0 && total <= kOutMin && host;
+  if (pinned) {
+    NLM_HIP(c, hipMemcpyAsync(host, base, total, hipMemcpyDeviceToHost,
+                              c->stream));
+    NLM_HIP(c, hipStreamSynchronize(c->stream));
+  }
+  const char* const dev = static_cast<const char*>(base);
+  size_t off = 0;
+  for (int k = 0; k < count; off += bytes[k++]) {
+    if (!dst[k] || !bytes[k]) continue;
+    if (pinned)
+      std::memcpy(dst[k], static_cast<const char*>(host) + off, bytes[k]);
+    else
+      NLM_HIP(c, hipMemcpyAsync(dst[k], dev + off, bytes[k],
+                                hipMemcpyDeviceToHost, c->stream));
+  }
+  if (!pinned) NLM_HIP(c, hipStreamSynchronize(c->stream));
+  return NLM_OK;
+}
+
+}  // namespace nlm
+
 extern "C" void nlm_ctx_destroy(nlm_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
@@ -73,6 +110,7 @@ extern "C" void nlm_ctx_destroy(nlm_ctx* c) {
   if (c->qs.e0) (void)hipEventDestroy(c->qs.e0);
   if (c->qs.e1) (void)hipEventDestroy(c->qs.e1);
   if (c->qs.hctl) (void)hipHostFree(c->qs.hctl);
+  if (c->fd.out_host) (void)hipHostFree(c->fd.out_host);
   hipStream_t st = c->stream;
   delete c;  // frees every device buffer
   if (st) (void)hipStreamDestroy(st);

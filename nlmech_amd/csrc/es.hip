@@ -1213,6 +1213,12 @@ extern "C" int nlm_fd_get_node_fields(nlm_ctx* c, double* theta, double* mw) {
                            src[k], s.perm_dev.as<int32_t>(), lo, m,
                            s.out.as<double>() + k * held);
     NLM_HIP(c, hipGetLastError());
+    if (held == s.n) {
+      void* const to[2] = {theta, mw};
+      const size_t bytes[2] = {sizeof(double) * size_t(s.n),
+                               sizeof(double) * size_t(s.n)};
+      return outputs_to_host(c, s.out.p, 2, to, bytes);
+    }
     for (int k = 0; k < 2; k++)
       if (dst[k])
         NLM_HIP(c, hipMemcpyAsync(dst[k] + lo, s.out.as<double>() + k * held,

@@ -2076,13 +2076,10 @@ int from_dev_vecs(nlm_ctx* c, int count, const DevBuf* const* src,
         o += 3 * s.n;
       }
     NLM_HIP(c, hipGetLastError());
-    o = base;
-    for (int k = 0; k < count; k++)
-      if (dst[k]) {
-        NLM_HIP(c, hipMemcpyAsync(dst[k], o, vec, hipMemcpyDeviceToHost,
-                                  c->stream));
-        o += 3 * s.n;
-      }
+    std::vector<void*> to(dst, dst + count);
+    std::vector<size_t> bytes(to.size());
+    for (int k = 0; k < count; k++) bytes[k] = dst[k] ? vec : 0;
+    return outputs_to_host(c, base, count, to.data(), bytes.data());
   } else {
     for (int k = 0; k < count; k++)
       for (int64_t lo = 0; dst[k] && lo < s.n; lo += held) {
@@ -2326,17 +2323,10 @@ extern "C" int nlm_fd_postproc(nlm_ctx* c, float* Z, float* phi,
     hipLaunchKernelGGL(k_postproc<3>, dim3(g), dim3(256), 0, c->stream,
                        make_args<3>(c), dz, dp, de, perm);
   NLM_HIP(c, hipGetLastError());
-  if (Z)
-    NLM_HIP(c, hipMemcpyAsync(Z, dz, sizeof(float) * n, hipMemcpyDeviceToHost,
-                              c->stream));
-  if (phi)
-    NLM_HIP(c, hipMemcpyAsync(phi, dp, sizeof(float) * n,
-                              hipMemcpyDeviceToHost, c->stream));
-  if (energy)
-    NLM_HIP(c, hipMemcpyAsync(energy, de, sizeof(double) * n,
-                              hipMemcpyDeviceToHost, c->stream));
-  NLM_HIP(c, hipStreamSynchronize(c->stream));
-  return NLM_OK;
+  void* const to[3] = {energy, Z, phi};
+  const size_t bytes[3] = {sizeof(double) * n, sizeof(float) * n,
+                           sizeof(float) * n};
+  return outputs_to_host(c, de, 3, to, bytes);
 }
 
 extern "C" int nlm_fd_postproc_noalloc(nlm_ctx* c, float* Z, float* phi,

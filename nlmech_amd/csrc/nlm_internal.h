@@ -230,6 +230,7 @@ struct FdState {
   DevBuf out;    // device staging of the calls that return node fields, in
                  // reference order; kOutMin at setup, grows to the largest
                  // call, kOutMax at most
+  void* out_host = nullptr;  // pinned, kOutMin bytes (outputs_to_host)
   DevBuf bctab;  // BcTable
   BcTable bc_host{};
   std::vector<uint8_t> fix_host;
@@ -390,6 +391,11 @@ inline void out_staging(nlm_ctx* c, size_t bytes) {
   b.p = p;
   b.bytes = bytes;
 }
+
+// Copies `count` outputs that lie behind each other at `base` on the device,
+// bytes[k] each, to dst[k] (null: not wanted) and waits (ctx.cpp).
+int outputs_to_host(nlm_ctx* c, const void* base, int count, void* const* dst,
+                    const size_t* bytes);
 
 // Drops the previous model's tangent, preconditioner, colors, aggregates and
 // captured batch of the quasi-static solver, and the graph network's reverse

@@ -79,3 +79,26 @@ def test_dilatation_alone():
         t2 = np.full(p.n, 7.0)
         rc = g.lib.nlm_fd_get_node_fields(g.ctx, capi.ptr(t2, C.c_double), None)
         assert rc == 0 and np.array_equal(th, t2) and np.all(mw > 0)
+
+
+def test_time_of_small_outputs():
+    """Three vectors of 810 nodes cost little more than one (a copy each to
+    pageable memory: more than twice)."""
+    import time
+
+    from nlmech_amd.engine import GpuFD
+    progress("[gpu] time of small outputs")
+    p = pr.plate2d(30, 27, 1e-3, 3, 1e-7, 1)
+    us = []
+    with GpuFD(p) as g:
+        out = [np.zeros((p.n, 3)) for _ in range(3)]
+        ptrs = [o.ctypes.data_as(C.POINTER(C.c_double)) for o in out]
+        for args in ([ptrs[0], None, None], ptrs):
+            best = 1e9
+            for _ in range(200):
+                t = time.perf_counter()
+                g._call("nlm_fd_get_state", *args)
+                best = min(best, time.perf_counter() - t)
+            us.append(1e6 * best)
+    progress(f"[gpu]   {us[0]:.0f} {us[1]:.0f} us")
+    assert us[1] <= 1.8 * us[0]
