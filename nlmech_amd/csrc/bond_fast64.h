@@ -5,25 +5,27 @@
 // and square root with their range scaling, exp) are written here for the
 // range that a bond's quantities have:
 //
-//  sqrt and quotients of the exact mode come out correctly rounded, so they
-//  are the bits of the IEEE operations: Goldschmidt's iteration from the
-//  hardware's reciprocal square root, then Markstein's final step q' = q +
-//  (a - b q) y with the residual taken by a fused multiply-add (P. Markstein,
-//  "Software division and square root using Goldschmidt's algorithms", RNC6,
-//  2004).  One iteration gives the length, its reciprocal and the square's
-//  reciprocal together, so the quotients S = dx.du / |dx|^2 and dx / |dx|
+//  sqrt and quotients of the exact mode are the bits of the IEEE operations
+//  (measured, not proven: of 6.3e9 random operands of each, none differs):
+//  Goldschmidt's iteration from the hardware's reciprocal square root, then
+//  Markstein's final step q' = q + (a - b q) y with the residual taken by a
+//  fused multiply-add (P. Markstein, "Software division and square root using
+//  Goldschmidt's algorithms", RNC6, 2004).  One iteration gives the length,
+//  its reciprocal and the square's reciprocal together, so the quotients
+//  S = dx.du / |dx|^2 and dx / |dx|
 //  take three operations each.  No range scaling: the lengths of a mesh lie
 //  far inside the exponent range (checked at setup, kStagedLenMin/Max).
 //
 //  exp of the softening factor: the exponent x = -beta r S^2 of a bond that
 //  does not break lies in [-0.5 f^2 (1 + 2e-5), 0], f the critical-stretch
 //  factor; with f <= 1 one polynomial covers it with no range reduction
-//  (0.8 ulp against high-precision arithmetic; the general form 0.7 ulp).
+//  (0.88 ulp against high-precision arithmetic; the general form 0.89 ulp; the
+//  library's exp 0.5).
 //  The coefficients interpolate (exp(x) - 1)/x at Chebyshev points.
 //
 // Every decision keeps the rule of bond_rnp.h: a bond inside a guard band is
-// decided by the exact evaluation after the chunk.  The comparisons are
-// written so that a NaN counts as inside the band.
+// decided by the exact evaluation after the chunk.  The break test's
+// comparisons here are written so that a NaN counts as inside the band.
 #pragma once
 
 #include "bond_rnp.h"
@@ -141,7 +143,8 @@ __device__ __forceinline__ double influence_rn(const RnpDev& m, double r) {
 }
 
 // Exact mode, common path: the operations of bond_exact in its order, bit
-// for bit (72 instead of about 170 vector instructions a bond in 2D).
+// for bit except exp, which the deferred evaluations still call (81 instead of
+// about 170 vector instructions a slot in 2D).
 // F is 0 for broken bonds, bonds left to the exact evaluation (ex) and the
 // zero-volume record of padded slots.  band: breakable bonds at or past the
 // break test's lower bound.
@@ -176,8 +179,8 @@ __device__ __forceinline__ void bond_exact_fast(
   for (int d = 0; d < DIM; d++) F[d] = s * quot(dx[d], o.r, o.yr);
 }
 
-// FP64 mode, common path (about 42 instead of 71 vector instructions a bond
-// in 2D).  cvj = vol_j c4 (J when constant).  The volume-correction factor
+// FP64 mode, common path (49 instead of 71 vector instructions a slot in
+// 2D).  cvj = vol_j c4 (J when constant).  The volume-correction factor
 // enters as fac / r = min((check_up/h) / r - 1/h, 1/r).
 template <int DIM, int INF, bool NOFAIL, bool SHORT, bool ACC>
 __device__ __forceinline__ void bond_fp64_staged(

@@ -1272,6 +1272,9 @@ size_t halo_rec_bytes(int dim, int precision, bool nofail) {
 //   3D FP32-force, 124: 64 x 8 8.4, 256 x 1 20.5; 1067: 128 x 2 20.0, 64 x 8
 //     22.6, 256 x 1 24.8; 4032: 256 x 2 43.7, 128 x 2 44.9, 256 x 1 51.5.
 // Direct gathers before (3D): 1067, FP64 61; 4032, FP32-force 95.
+// (72 x 64 x 56 has halos of 1120 nodes; blocks that the Morton order cuts
+// unevenly exceed the 64 KiB of 16-bit offsets at 256 FP64 records and take
+// 128 x 4: 65 x 65 x 65 FP64 / exact 93 / 124, direct gathers 129 / 204.)
 struct StageRule {
   int tile, parts;
 };
@@ -1295,12 +1298,15 @@ StageRule stage_rule(int dim, int precision, int64_t nslices) {
 //     11.3 / 10.4, before 28.1 / 19.1 / 16.3; 301 x 257 (1209): 64 x 4 23.3 /
 //     20.1 / 15.2, 256 x 1 28.6 / 23.9 / 19.8, before 40.0 / 26.9 / 23.0;
 //     600 x 500 (4688): 256 x 1 58.2 / 47.9 / 35.5, 64 x 4 65.3 / 54.8 /
-//     38.8, before 84.8 / 57.6 / 46.5;
+//     38.8, before 84.8 / 57.6 / 46.5; FP32-force at 128 x 2, 410 x 407 (2608)
+//     22.3, 620 x 617 (5978) 41.5, before 30.0 / 56.2;
 //   3D exact / FP64 / FP32-force, 20 x 18 x 22 (124): 64 x 8 25.6 / 20.3 /
 //     15.9, before 92 / 51 / 43; 47 x 39 x 33 (945): 256 x 1 65.3 / 53.2 /
 //     46.7, 128 x 4 72.5 / 47.9 / 30.9, before 96.4 / 56.3 / 46.0; 80 x 80 x
 //     80 (8000): 256 x 1 317 / 241 / 166, 128 x 4 465 / 261 / 154, 256 x 2
-//     499 / 338 / 140, before 523 / 269 / 166; short rows (row: bonds a node),
+//     499 / 338 / 140, before 523 / 269 / 166; FP32-force around the line, 128
+//     x 4 / 256 x 2: 48 x 48 x 48 (1728) 50.6 / 47.6, 54 x 54 x 54 (2461) 61.6 /
+//     68.9, 60 x 60 x 60 (3375) 81.1 / 82.2, 64 x 64 x 64 90.2 / 84.3; short rows (row: bonds a node),
 //     60 x 60 x 60 at a horizon of 2 h (25), FP32-force: 256 x 1 39.7, 256 x 2
 //     41.9, before 39.9.
 // 3D FP64 above 2500 slices: 256 x 1, but 128 x 4 where a CU's LDS holds one

@@ -1,7 +1,7 @@
 // fd_staged.h -- the LDS-staged bond-based step kernel of the FP64 modes
 // and of every mode in 3D (k_fd_st).
 //
-// A workgroup owns a tile of the layout's internal order (128, 256 or 512
+// A workgroup owns a tile of the layout's internal order (64 to 512
 // nodes): it stages the tile's halo -- every node its rows reference -- in
 // LDS once (one record a node) and reads neighbors through 16-bit LDS byte
 // offsets.  Record 0 is a zero-volume record far from every node; padded
