@@ -376,7 +376,8 @@ def test_time_across_the_last_split(ratio):
     us = [step_us(pr.plate2d(s, s - 3, 1e-3, ratio, 1e-7, 1),
                   NLM_PREC_FP32_FORCE) for s in (406, 410)]
     progress(f"[gpu]   {us[0]:.2f} {us[1]:.2f} us")
-    assert us[1] <= 1.18 * us[0]
+    # (1.08 and 1.12 measured, the runs of one box within 3 %)
+    assert us[1] <= (1.18 if ratio == 3 else 1.25) * us[0]
 
 
 def test_time_of_no_fail_records():
@@ -435,4 +436,5 @@ def test_time_of_setup(kind):
         tiles.append(tile)
     progress(f"[gpu]   {ms[0]:.0f} {ms[1]:.0f} ms")
     assert tiles == [256, 128]
-    assert ms[1] <= 1.5 * ms[0]
+    # (1.03 to 1.16 measured; host threads)
+    assert ms[1] <= 1.7 * ms[0]
