@@ -332,7 +332,7 @@ def test_autotuner_keeps_a_faster_setup(precision, kind):
     else:
         p = pr.cube3d(16, 1e-3, 3, 1e-7, 1, jitter=0.02, sigma_v=1e-3)
 
-    def us(g):  # best of five: other work on the box only adds
+    def us(g):  # best of five: other work on the machine only adds
         return min(g.timed_steps(101)[1] for _ in range(5)) * 1e3
 
     with GpuFD(p, precision=precision) as g:
@@ -360,7 +360,7 @@ def test_autotuner_keeps_a_faster_setup(precision, kind):
 
 
 def step_us(p, precision):
-    """Microseconds per step, best of eight: other work on the box only adds."""
+    """Microseconds per step, best of eight: other work on the machine only adds."""
     from nlmech_amd.engine import GpuFD
     with GpuFD(p, precision=precision) as g:
         g.init()
@@ -376,7 +376,7 @@ def test_time_across_the_last_split(ratio):
     us = [step_us(pr.plate2d(s, s - 3, 1e-3, ratio, 1e-7, 1),
                   NLM_PREC_FP32_FORCE) for s in (406, 410)]
     progress(f"[gpu]   {us[0]:.2f} {us[1]:.2f} us")
-    # (1.08 and 1.12 measured, the runs of one box within 3 %)
+    # (1.08 and 1.12 measured, repeated runs within 3 %)
     assert us[1] <= (1.18 if ratio == 3 else 1.25) * us[0]
 
 
